@@ -329,7 +329,7 @@ ptg_status ptg_walk_subtree(const ptg_walk_tree *wt, const int32_t *start_slot, 
 /* ptg_walk without a workspace, for callers that cannot allocate (code under HIP graph capture,
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  The same
  * kernels and results as ptg_walk; the walk control block and the per-wave spill stacks live in a
- * static device array of the library (80 MiB + 4 KiB per GPU, held until the process ends: 4096
+ * static device array of the library (80 MiB + 8 KiB per GPU, held until the process ends: 4096
  * spill entries per wave for the 5120 waves of a 256-CU grid; measured walks need at most 1344).
  * Nothing is allocated and nothing synchronises.  err (device int32, required) receives the
  * walk's flags instead of ptg_walk_check: 0 fine, bit 0 a traversal stack exceeded the spill

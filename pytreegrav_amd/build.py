@@ -33,6 +33,7 @@ COMMON = [
 UNITS = {
     "build.hip": ["-ffp-contract=off"],
     "walk.hip": [],
+    "walk64.hip": [],
     "direct.hip": [],
     "learned.hip": [],
     "colden.hip": [],

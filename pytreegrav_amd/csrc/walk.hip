@@ -15,36 +15,18 @@
 #include <algorithm>
 #include <mutex>
 
-#include "ptg_common.hpp"
+#include "walk_shared.hpp"
 
-#define WALK_WAVES 4
-#define SCAP 768       // LDS traversal stack entries per wave (>= 512, the most children one step pushes)
-#define SPILL 256      // entries refilled from global memory at a time (<= SCAP - 512)
-#define GCAP 16384     // global spill entries per wave
 // a list is evaluated in multiples of LF entries once it holds LF (a power of 2: 64, or 32 for the
 // six-wave variant); a list holds LF - 1 + one step's 64 entries (ICAP)
-#define NXCD 8
-#define CTR_STRIDE 32  // int32 words between per-XCD counters (128 B)
-
-template <typename T> struct alignas(4 * sizeof(T)) V4 {
-    T x, y, z, w;
-};
 
 template <typename T, bool QUAD, int LF> struct WaveLds {
     static constexpr int ICAP = LF + 64;
     int stack[SCAP];
     V4<T> nodes[ICAP];  // accepted nodes: x y z m
-    T nh[sizeof(T) == 8 ? ICAP : 1];  // node softening (FP64 exact path only)
     T nq[QUAD ? 6 * ICAP : 1];
     V4<T> parts[ICAP];  // particles: x y z m
     T ph[ICAP];
-};
-
-struct WalkCtl {
-    int32_t ctr[NXCD * CTR_STRIDE];   // per-XCD group counters
-    int32_t err;
-    int32_t hwm;  // deepest global spill stack (entries) any wave reached in the last walk
-    int32_t pad[30];
 };
 
 template <typename T> struct WalkArgs {
@@ -81,134 +63,9 @@ template <typename T> struct WalkArgs {
     WalkCtl *ctl;
     int *spill;
     int gcap;  // global spill entries per wave (GCAP, or what the static scratch of ptg_walk_noalloc gives)
-    const int32_t *start = nullptr;  // subtree walks: device slot of the element every walk starts at
 };
-
-// ---- softening kernels (kernel.py:4-75), generic precision ----
-template <typename T> __device__ __forceinline__ T force_kernel(T r, T h)
-{
-    if (r > h) return T(1) / (r * r * r);
-    T hinv = T(1) / h;
-    T q = r * hinv;
-    if (q <= T(0.5)) return (T(10.666666666666666666) + q * q * (T(-38.4) + T(32.0) * q)) * hinv * hinv * hinv;
-    return (T(21.333333333333) - T(48.0) * q + T(38.4) * q * q - T(10.666666666667) * q * q * q -
-            T(0.066666666667) / (q * q * q)) *
-           hinv * hinv * hinv;
-}
-
-template <typename T> __device__ __forceinline__ T tidal_kernel(T r, T h)
-{
-    if (r > h) {
-        T r2 = r * r;
-        return T(3) / (r2 * r2 * r);
-    }
-    T hinv = T(1) / h;
-    T hinv2 = hinv * hinv;
-    T hinv5 = hinv2 * hinv2 * hinv;
-    T q = r * hinv;
-    if (q <= T(0.5)) return (T(76.8) - T(96.0) * q) * hinv5;
-    T qinv = T(1) / q;
-    T qinv3 = qinv * qinv * qinv;
-    return (T(48.0) * qinv - T(76.8) + T(32.0) * q - T(0.2) * qinv3 * qinv * qinv) * hinv5;
-}
-
-template <typename T> __device__ __forceinline__ T potential_kernel(T r, T h)
-{
-    if (h == T(0)) return T(-1) / r;
-    T hinv = T(1) / h;
-    T q = r * hinv;
-    if (q <= T(0.5)) return (T(-2.8) + q * q * (T(5.33333333333333333) + q * q * (T(6.4) * q - T(9.6)))) * hinv;
-    if (q <= T(1))
-        return (T(-3.2) + T(0.066666666666666666666) / q +
-                q * q * (T(10.666666666666666666666) + q * (T(-16.0) + q * (T(9.6) - T(2.1333333333333333333333) * q)))) *
-               hinv;
-    return T(-1) / r;
-}
 
 __device__ __forceinline__ float fast_rsqrt(float x) { return __builtin_amdgcn_rsqf(x); }
-__device__ __forceinline__ double fast_rsqrt(double x) { return 1.0 / sqrt(x); }
-
-template <int FIELDS> struct NW {
-    static constexpr int POT = (FIELDS & PTG_POT) ? 1 : 0;
-    static constexpr int ACC = (FIELDS & PTG_ACC) ? 1 : 0;
-    static constexpr int TID = (FIELDS & PTG_TIDAL) ? 1 : 0;
-    static constexpr int W = POT + 3 * ACC + 9 * TID;
-};
-
-// per-target accumulators: phi, g(3), T(6 independent)
-template <typename T> struct Acc {
-    T phi, gx, gy, gz, txx, tyy, tzz, txy, txz, tyz;
-};
-
-// One source element on one target, with the reference's branches (grouped_treewalk.py:75-153):
-// r2 > 0 self skip, softened iff r < max(h_s, h_t), quadrupole terms for nodes only.
-template <typename T, int FIELDS, bool QUADTERM>
-__device__ __forceinline__ void interact_exact(Acc<T> &a, T sx, T sy, T sz, T M, T hs, const T *q, T tx, T ty, T tz,
-                                               T th)
-{
-    constexpr bool P = NW<FIELDS>::POT, G = NW<FIELDS>::ACC, D = NW<FIELDS>::TID;
-    T dx = sx - tx, dy = sy - ty, dz = sz - tz;
-    T r2 = dx * dx + dy * dy + dz * dz;
-    if (!(r2 > T(0))) return;
-    T r = sqrt(r2);
-    T ht = hs > th ? hs : th;
-    bool softened = r < ht;
-    T phi = 0, K = 0, Q = 0;
-    if (P) phi = softened ? M * potential_kernel(r, ht) : -M / r;
-    if (G || D) K = softened ? M * force_kernel(r, ht) : M / (r * r2);
-    if (D) Q = softened ? M * tidal_kernel(r, ht) : T(3) * K / r2;
-    T gx = 0, gy = 0, gz = 0;
-    if (G) {
-        gx = K * dx;
-        gy = K * dy;
-        gz = K * dz;
-    }
-    T txx = 0, tyy = 0, tzz = 0, txy = 0, txz = 0, tyz = 0;
-    if (D) {
-        txx = Q * dx * dx - K;
-        tyy = Q * dy * dy - K;
-        tzz = Q * dz * dz - K;
-        txy = Q * dx * dy;
-        txz = Q * dx * dz;
-        tyz = Q * dy * dz;
-    }
-    if (QUADTERM) {
-        T qxx = q[0], qxy = q[1], qxz = q[2], qyy = q[3], qyz = q[4], qzz = q[5];
-        T r5inv = T(1) / (r2 * r2 * r);
-        T r7inv = r5inv / r2;
-        T qdx = qxx * dx + qxy * dy + qxz * dz;
-        T qdy = qxy * dx + qyy * dy + qyz * dz;
-        T qdz = qxz * dx + qyz * dy + qzz * dz;
-        T A = dx * qdx + dy * qdy + dz * qdz;
-        if (P) phi += T(-0.5) * A * r5inv;
-        if (G) {
-            T quad_fac = A * r7inv;
-            gx += T(2.5) * quad_fac * dx - qdx * r5inv;
-            gy += T(2.5) * quad_fac * dy - qdy * r5inv;
-            gz += T(2.5) * quad_fac * dz - qdz * r5inv;
-        }
-        if (D) {
-            T diag = T(-2.5) * A * r7inv;
-            T fac = T(17.5) * A * r7inv / r2;
-            txx += qxx * r5inv - T(10.0) * dx * qdx * r7inv + diag + fac * dx * dx;
-            tyy += qyy * r5inv - T(10.0) * dy * qdy * r7inv + diag + fac * dy * dy;
-            tzz += qzz * r5inv - T(10.0) * dz * qdz * r7inv + diag + fac * dz * dz;
-            txy += qxy * r5inv - T(5.0) * (dx * qdy + dy * qdx) * r7inv + fac * dx * dy;
-            txz += qxz * r5inv - T(5.0) * (dx * qdz + dz * qdx) * r7inv + fac * dx * dz;
-            tyz += qyz * r5inv - T(5.0) * (dy * qdz + dz * qdy) * r7inv + fac * dy * dz;
-        }
-    }
-    a.phi += phi;
-    a.gx += gx;
-    a.gy += gy;
-    a.gz += gz;
-    a.txx += txx;
-    a.tyy += tyy;
-    a.tzz += tzz;
-    a.txy += txy;
-    a.txz += txz;
-    a.tyz += tyz;
-}
 
 // Accepted node on one target, fast path: the acceptance test guarantees r > h_t, h_s and r > 0.
 template <typename T, int FIELDS, bool QUAD>
@@ -451,56 +308,7 @@ __device__ __forceinline__ void exp_eval(Acc<T> &a, const GroupExp<T> &E, T ux, 
     }
 }
 
-// gap between x and the interval [lo, hi] (0 inside): bmin - x and x - bmax are exact differences,
-// so this equals the two-sided branch form bit for bit
-__device__ __forceinline__ float box_gap(float x, float lo, float hi) { return fmaxf(fmaxf(lo - x, x - hi), 0.f); }
-__device__ __forceinline__ double box_gap(double x, double lo, double hi) { return fmax(fmax(lo - x, x - hi), 0.0); }
-
-// Stack spill: when sp entries plus the tot children about to be pushed exceed SCAP, the bottom
-// ks entries (the excess rounded up to 64, at most sp; tot <= 512 <= SCAP so ks >= the excess)
-// go to the wave's global spill stack and the rest move down.  Any order of visits gives the same
-// accepted sets, so the global stack is refilled from its top when the LDS stack runs empty.
-static_assert(SCAP >= 512 && SPILL >= 64 && SPILL <= SCAP - 512, "stack geometry");
-__device__ __forceinline__ int spill_count(int sp, int tot)
-{
-    const int ex = sp + tot - SCAP;
-    return std::min(sp, (ex + 63) & ~63);
-}
-__device__ __forceinline__ void spill_bottom(int *stack, int *dst, int sp, int ks, int lane)
-{
-    for (int q = lane; q < ks; q += 64) dst[q] = stack[q];
-    __builtin_amdgcn_wave_barrier();
-    // read [ks + q, ks + q + 64) before writing [q, q + 64); later reads lie above earlier writes
-    for (int q = 0; q < sp - ks; q += 64) {
-        const int v = (q + lane < sp - ks) ? stack[ks + q + lane] : 0;
-        __builtin_amdgcn_wave_barrier();
-        if (q + lane < sp - ks) stack[q + lane] = v;
-        __builtin_amdgcn_wave_barrier();
-    }
-}
-
-// lanes below this one whose bit is set in m
-__device__ __forceinline__ int lanes_below(uint64_t m)
-{
-    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
-
-// exclusive prefix sum across the wave of v in [0, 15] (children counts), one ballot per bit;
-// tot receives the wave total
-__device__ __forceinline__ int small_excl_scan(int v, int &tot)
-{
-    int below = 0, t = 0;
-#pragma unroll
-    for (int b = 0; b < 4; b++) {
-        const uint64_t m = ptg_ballot((v >> b) & 1);
-        below += lanes_below(m) << b;
-        t += (int)__popcll(m) << b;
-    }
-    tot = t;
-    return below;
-}
-
-template <typename T, int TPL, int FIELDS, bool QUAD, bool EXACT, int LF>
+template <typename T, int TPL, int FIELDS, bool QUAD, int LF>
 __device__ __forceinline__ void flush_nodes(const WaveLds<T, QUAD, LF> &L, int cnt, Acc<T> (&acc)[TPL],
                                             const T (&tx)[TPL], const T (&ty)[TPL], const T (&tz)[TPL],
                                             const T (&th)[TPL])
@@ -514,15 +322,12 @@ __device__ __forceinline__ void flush_nodes(const WaveLds<T, QUAD, LF> &L, int c
         }
 #pragma unroll
         for (int j = 0; j < TPL; j++) {
-            if constexpr (EXACT)
-                interact_exact<T, FIELDS, QUAD>(acc[j], s.x, s.y, s.z, s.w, L.nh[k], q, tx[j], ty[j], tz[j], th[j]);
-            else
-                interact_node_fast<T, FIELDS, QUAD>(acc[j], s, q, tx[j], ty[j], tz[j]);
+            interact_node_fast<T, FIELDS, QUAD>(acc[j], s, q, tx[j], ty[j], tz[j]);
         }
     }
 }
 
-template <typename T, int TPL, int FIELDS, bool QUAD, bool EXACT, int LF>
+template <typename T, int TPL, int FIELDS, bool QUAD, int LF>
 __device__ __forceinline__ void flush_parts(const WaveLds<T, QUAD, LF> &L, int cnt, Acc<T> (&acc)[TPL],
                                             const T (&tx)[TPL], const T (&ty)[TPL], const T (&tz)[TPL],
                                             const T (&th)[TPL])
@@ -532,10 +337,7 @@ __device__ __forceinline__ void flush_parts(const WaveLds<T, QUAD, LF> &L, int c
         T hs = L.ph[k];
 #pragma unroll
         for (int j = 0; j < TPL; j++) {
-            if constexpr (EXACT)
-                interact_exact<T, FIELDS, false>(acc[j], s.x, s.y, s.z, s.w, hs, nullptr, tx[j], ty[j], tz[j], th[j]);
-            else
-                interact_part_fast<T, FIELDS>(acc[j], s, hs, tx[j], ty[j], tz[j], th[j]);
+            interact_part_fast<T, FIELDS>(acc[j], s, hs, tx[j], ty[j], tz[j], th[j]);
         }
     }
 }
@@ -557,13 +359,12 @@ template <typename T, int TPL, int VAR> struct WalkOcc {
     static constexpr int blocks_per_cu = fast && VAR == 2 ? 6 : 5;
 };
 
-template <typename T, int TPL, int FIELDS, bool QUAD, bool EXACT, bool EXP, int VAR>
+template <typename T, int TPL, int FIELDS, bool QUAD, bool EXP, int VAR>
 __global__ __launch_bounds__(64 * WALK_WAVES) __attribute__((amdgpu_waves_per_eu(WalkOcc<T, TPL, VAR>::waves)))
 void k_walk(WalkArgs<T> A)
 {
     constexpr int LF = WalkOcc<T, TPL, VAR>::lf;
-    static_assert(!EXP || (sizeof(T) == 4 && !QUAD && !EXACT && !NW<FIELDS>::TID),
-                  "the group expansion is an FP32 monopole potential/acceleration path");
+    static_assert(!EXP || (!QUAD && !NW<FIELDS>::TID), "the group expansion is a monopole potential/acceleration path");
     __shared__ WaveLds<T, QUAD, LF> lds[WALK_WAVES];
     const int wave = threadIdx.x >> 6, lane = ptg_lane();
     WaveLds<T, QUAD, LF> &L = lds[wave];
@@ -598,13 +399,9 @@ void k_walk(WalkArgs<T> A)
                     else hi = mid;
                 }
                 root = (int)lo;
-                if (sizeof(T) == 4) {
-                    ox = A.cubes[4 * lo];
-                    oy = A.cubes[4 * lo + 1];
-                    oz = A.cubes[4 * lo + 2];
-                } else {
-                    ox = oy = oz = 0.0;
-                }
+                ox = A.cubes[4 * lo];
+                oy = A.cubes[4 * lo + 1];
+                oz = A.cubes[4 * lo + 2];
             }
 
             // ---- targets: lane holds a0 + lane + 64 j ----
@@ -668,19 +465,9 @@ void k_walk(WalkArgs<T> A)
                 eps_x = A.eps_exp * (A.eps_scale ? (T)A.eps_scale[root] : T(1));
             }
 
-            // the root of system s occupies walk slot s; a subtree walk (the FP64 reference-branch
-            // walk only) starts at its element's slot instead (wave-uniform; an out-of-range slot is
-            // reported, and dropped when popped like any corrupt link, so it walks nothing)
-            int first = root;
-            if constexpr (EXACT) {
-                if (A.start) {
-                    first = __builtin_amdgcn_readfirstlane(*A.start);
-                    if ((first < 0 || first >= A.nslots) && lane == 0) atomicOr(&A.ctl->err, 4);
-                }
-            }
             int sp = 1, gsp = 0, nn = 0, np = 0;
             bool overflow = false;
-            if (lane == 0) L.stack[0] = first;
+            if (lane == 0) L.stack[0] = root;  // the root of system s occupies walk slot s
             __builtin_amdgcn_wave_barrier();
 
             for (;;) {
@@ -714,32 +501,23 @@ void k_walk(WalkArgs<T> A)
                 const T dxm = box_gap(X.x, bmin0, bmax0), dym = box_gap(X.y, bmin1, bmax1), dzm = box_gap(X.z, bmin2, bmax2);
                 const T r2m = dxm * dxm + dym * dym + dzm * dzm;
                 const T hh = X2.x > hmax ? X2.x : hmax;
-                bool acc_node, far_part = false;
-                if constexpr (EXACT) {
-                    // the reference's test as written: r_min > max(size/theta + delta, h + 0.6 size + delta)
-                    const T r_min = sqrt(r2m);
-                    const T c1 = X2.y / A.theta + X2.z;
-                    const T c2 = hh + X2.y * T(0.6) + X2.z;
-                    acc_node = ve && !ispart && r_min > (c1 > c2 ? c1 : c2);
-                } else {
-                    // the same test on squared distances (every threshold is >= 0), with 1/theta;
-                    // evaluated without branches (bitwise &) so the slot's aux record is one load
-                    // issued with the others, not a second round trip inside a branch
-                    const T c1 = X2.y * A.inv_theta + X2.z;
-                    const T c2 = hh + X2.y * T(0.6) + X2.z;
-                    const T c = c1 > c2 ? c1 : c2;
-                    acc_node = ve & !ispart & (r2m > c * c);
-                    // a particle farther from the group's box than every softening radius (and not
-                    // inside it) needs neither the softening nor the self test -> node list
-                    far_part = ve & ispart & (r2m > hh * hh);
-                    if (A.crit == 1) {
-                        // error-bounded: also require the quadrupole term the monopole drops,
-                        // 3.5 |Q| / r^4, to stay below eps (theta is then only a loose cap)
-                        acc_node = acc_node & (X2.w < A.eps * r2m * r2m);
-                    } else if (A.crit == 2) {
-                        // learned: r_min beyond the node's predicted opening radius
-                        acc_node = acc_node & (r2m > X2.w * X2.w);
-                    }
+                // the reference's test (treewalk.py:22-25) on squared distances (every threshold is >= 0),
+                // with 1/theta; evaluated without branches (bitwise &) so the slot's aux record is one
+                // load issued with the others, not a second round trip inside a branch
+                const T c1 = X2.y * A.inv_theta + X2.z;
+                const T c2 = hh + X2.y * T(0.6) + X2.z;
+                const T c = c1 > c2 ? c1 : c2;
+                bool acc_node = ve & !ispart & (r2m > c * c);
+                // a particle farther from the group's box than every softening radius (and not
+                // inside it) needs neither the softening nor the self test -> node list
+                const bool far_part = ve & ispart & (r2m > hh * hh);
+                if (A.crit == 1) {
+                    // error-bounded: also require the quadrupole term the monopole drops,
+                    // 3.5 |Q| / r^4, to stay below eps (theta is then only a loose cap)
+                    acc_node = acc_node & (X2.w < A.eps * r2m * r2m);
+                } else if (A.crit == 2) {
+                    // learned: r_min beyond the node's predicted opening radius
+                    acc_node = acc_node & (r2m > X2.w * X2.w);
                 }
                 bool acc_part = ve && ispart && !far_part;
                 acc_node = acc_node || far_part;
@@ -767,7 +545,6 @@ void k_walk(WalkArgs<T> A)
                 if (acc_node) {
                     const int at = nn + lanes_below(bn);
                     L.nodes[at] = X;
-                    if (EXACT) L.nh[at] = X2.x;
                     if (QUAD) {
                         const T *q = A.quad + 8 * (int64_t)e;
 #pragma unroll
@@ -808,11 +585,10 @@ void k_walk(WalkArgs<T> A)
 
                 if (nn >= LF) {
                     const int c = nn & ~(LF - 1);  // c >= LF > nn - c
-                    flush_nodes<T, TPL, FIELDS, QUAD, EXACT, LF>(L, c, acc, tx, ty, tz, th);
+                    flush_nodes<T, TPL, FIELDS, QUAD, LF>(L, c, acc, tx, ty, tz, th);
                     __builtin_amdgcn_wave_barrier();
                     if (lane < nn - c) {  // reads [c, nn) and writes [0, nn - c): disjoint
                         L.nodes[lane] = L.nodes[c + lane];
-                        if (EXACT) L.nh[lane] = L.nh[c + lane];
                         if (QUAD)
                             for (int q = 0; q < 6; q++) L.nq[6 * lane + q] = L.nq[6 * (c + lane) + q];
                     }
@@ -821,7 +597,7 @@ void k_walk(WalkArgs<T> A)
                 }
                 if (np >= LF) {
                     const int c = np & ~(LF - 1);
-                    flush_parts<T, TPL, FIELDS, QUAD, EXACT, LF>(L, c, acc, tx, ty, tz, th);
+                    flush_parts<T, TPL, FIELDS, QUAD, LF>(L, c, acc, tx, ty, tz, th);
                     __builtin_amdgcn_wave_barrier();
                     if (lane < np - c) {  // disjoint ranges, as above
                         L.parts[lane] = L.parts[c + lane];
@@ -835,8 +611,8 @@ void k_walk(WalkArgs<T> A)
                 if (lane == 0) atomicOr(&A.ctl->err, 1);
                 continue;
             }
-            flush_nodes<T, TPL, FIELDS, QUAD, EXACT, LF>(L, nn, acc, tx, ty, tz, th);
-            flush_parts<T, TPL, FIELDS, QUAD, EXACT, LF>(L, np, acc, tx, ty, tz, th);
+            flush_nodes<T, TPL, FIELDS, QUAD, LF>(L, nn, acc, tx, ty, tz, th);
+            flush_parts<T, TPL, FIELDS, QUAD, LF>(L, np, acc, tx, ty, tz, th);
             __builtin_amdgcn_wave_barrier();
             if constexpr (EXP) {
                 exp_wave_sum(E);
@@ -929,7 +705,7 @@ extern "C" size_t ptg_walk_workspace_bytes(int64_t nt, int group_size)
 // overlap on one device (different streams) race.  Host code never passes the array's name to a
 // kernel (that is a host-side stand-in): it uses the address hipGetSymbolAddress returns, looked up
 // once per device with that device current and kept per device.
-#define NOALLOC_BYTES ((80u << 20) + 4096u)  // 4096 spill entries per wave for 5120 resident waves
+#define NOALLOC_BYTES ((80u << 20) + 8192u)  // 4096 spill entries per wave for 5120 resident waves
 #define NOALLOC_MIN_GCAP 2048  // spill entries per wave the static scratch must leave
 #define NOALLOC_MAX_DEVICES 64
 static __device__ __align__(256) char scratch[NOALLOC_BYTES];
@@ -974,20 +750,20 @@ __global__ void k_walk_err_out(const WalkCtl *ctl, int32_t *err)
     if (threadIdx.x == 0) *err = ctl->err;
 }
 
-template <typename T, int TPL, int FIELDS, bool QUAD, bool EXACT, bool EXP, int VAR = 0>
+template <typename T, int TPL, int FIELDS, bool QUAD, bool EXP, int VAR = 0>
 static ptg_status launch_t(const WalkArgs<T> &a, int64_t max_blocks, hipStream_t s)
 {
     static int per_cu = 0;
     if (per_cu == 0) {
         int nb = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_walk<T, TPL, FIELDS, QUAD, EXACT, EXP, VAR>,
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_walk<T, TPL, FIELDS, QUAD, EXP, VAR>,
                                                          64 * WALK_WAVES, 0) != hipSuccess ||
             nb < 1)
             nb = 1;
         per_cu = std::min(nb, WalkOcc<T, TPL, VAR>::blocks_per_cu);
     }
     int64_t blocks = std::min<int64_t>(max_blocks, (int64_t)num_cus() * per_cu);
-    k_walk<T, TPL, FIELDS, QUAD, EXACT, EXP, VAR><<<(unsigned)blocks, 64 * WALK_WAVES, 0, s>>>(a);
+    k_walk<T, TPL, FIELDS, QUAD, EXP, VAR><<<(unsigned)blocks, 64 * WALK_WAVES, 0, s>>>(a);
     PTG_LAUNCH_CHECK();
     return PTG_OK;
 }
@@ -998,32 +774,30 @@ template <typename T, int TPL, int FIELDS, bool EXP>
 static ptg_status launch_var(const WalkArgs<T> &a, int variant, int64_t blocks, hipStream_t s)
 {
     if constexpr (sizeof(T) == 4 && TPL == 1) {
-        if (variant == 1) return launch_t<T, TPL, FIELDS, false, false, EXP, 1>(a, blocks, s);
-        if (variant == 2) return launch_t<T, TPL, FIELDS, false, false, EXP, 2>(a, blocks, s);
+        if (variant == 1) return launch_t<T, TPL, FIELDS, false, EXP, 1>(a, blocks, s);
+        if (variant == 2) return launch_t<T, TPL, FIELDS, false, EXP, 2>(a, blocks, s);
     }
-    return launch_t<T, TPL, FIELDS, false, false, EXP, 0>(a, blocks, s);
+    return launch_t<T, TPL, FIELDS, false, EXP, 0>(a, blocks, s);
 }
 
-template <typename T, int TPL, bool EXACT>
+template <typename T, int TPL>
 static ptg_status launch_fq(const WalkArgs<T> &a, int fields, bool quad, bool expand, int variant, int64_t blocks,
                             hipStream_t s)
 {
-    if constexpr (sizeof(T) == 4 && !EXACT) {
-        if (expand) {  // checked by the caller: monopole, potential and/or acceleration
-            if (fields == PTG_POT) return launch_var<T, TPL, PTG_POT, true>(a, variant, blocks, s);
-            if (fields == PTG_ACC) return launch_var<T, TPL, PTG_ACC, true>(a, variant, blocks, s);
-            return launch_var<T, TPL, PTG_POT | PTG_ACC, true>(a, variant, blocks, s);
-        }
-        if (!quad) {
-            if (fields == PTG_POT) return launch_var<T, TPL, PTG_POT, false>(a, variant, blocks, s);
-            if (fields == PTG_ACC) return launch_var<T, TPL, PTG_ACC, false>(a, variant, blocks, s);
-            if (fields == (PTG_POT | PTG_ACC)) return launch_var<T, TPL, PTG_POT | PTG_ACC, false>(a, variant, blocks, s);
-        }
+    if (expand) {  // checked by the caller: monopole, potential and/or acceleration
+        if (fields == PTG_POT) return launch_var<T, TPL, PTG_POT, true>(a, variant, blocks, s);
+        if (fields == PTG_ACC) return launch_var<T, TPL, PTG_ACC, true>(a, variant, blocks, s);
+        return launch_var<T, TPL, PTG_POT | PTG_ACC, true>(a, variant, blocks, s);
+    }
+    if (!quad) {
+        if (fields == PTG_POT) return launch_var<T, TPL, PTG_POT, false>(a, variant, blocks, s);
+        if (fields == PTG_ACC) return launch_var<T, TPL, PTG_ACC, false>(a, variant, blocks, s);
+        if (fields == (PTG_POT | PTG_ACC)) return launch_var<T, TPL, PTG_POT | PTG_ACC, false>(a, variant, blocks, s);
     }
 #define PTG_F(F)                                                              \
     case F:                                                                   \
-        return quad ? launch_t<T, TPL, F, true, EXACT, false>(a, blocks, s)   \
-                    : launch_t<T, TPL, F, false, EXACT, false>(a, blocks, s);
+        return quad ? launch_t<T, TPL, F, true, false>(a, blocks, s)          \
+                    : launch_t<T, TPL, F, false, false>(a, blocks, s);
     switch (fields) {
         PTG_F(1) PTG_F(2) PTG_F(3) PTG_F(4) PTG_F(5) PTG_F(6) PTG_F(7)
     }
@@ -1032,13 +806,13 @@ static ptg_status launch_fq(const WalkArgs<T> &a, int fields, bool quad, bool ex
     return PTG_ERR_ARG;
 }
 
-template <typename T, bool EXACT>
+template <typename T>
 static ptg_status launch_walk(const WalkArgs<T> &a, int fields, bool quad, bool expand, int variant, int64_t blocks,
                               hipStream_t s)
 {
-    if (a.gs <= 64) return launch_fq<T, 1, EXACT>(a, fields, quad, expand, variant, blocks, s);
-    if (a.gs <= 128) return launch_fq<T, 2, EXACT>(a, fields, quad, expand, variant, blocks, s);
-    return launch_fq<T, 4, EXACT>(a, fields, quad, expand, variant, blocks, s);
+    if (a.gs <= 64) return launch_fq<T, 1>(a, fields, quad, expand, variant, blocks, s);
+    if (a.gs <= 128) return launch_fq<T, 2>(a, fields, quad, expand, variant, blocks, s);
+    return launch_fq<T, 4>(a, fields, quad, expand, variant, blocks, s);
 }
 
 // ptg_walk and ptg_walk_noalloc: ws/ws_bytes is the caller's workspace, or nullptr with noalloc set
@@ -1164,19 +938,18 @@ static ptg_status walk_impl(const ptg_walk_tree *wt, const ptg_forest *forest, c
                           group_size, (float)theta, (float)(1.0 / theta), crit, (float)eps, (float)eps_exp,
                           expand ? criterion->expansion_rel : 0.0f, eps_scale, G, wt->origin[0], wt->origin[1],
                           wt->origin[2],
-                          fn, fo, fc, out, counters, ctl, spill, gcap, start_slot};
+                          fn, fo, fc, out, counters, ctl, spill, gcap};
         if (exact) {
             ptg_set_error("ptg_walk: the exact branch set is evaluated in FP64; use prec=PTG_F64");
             return PTG_ERR_ARG;
         }
-        st = launch_walk<float, false>(a, fields, quadrupole != 0, expand, variant, blocks, s);
+        st = launch_walk<float>(a, fields, quadrupole != 0, expand, variant, blocks, s);
     } else if (wt->prec == PTG_F64) {
-        WalkArgs<double> a{(const V4<double> *)wt->xyzm, (const V4<double> *)wt->aux, (const int2 *)wt->kids,
-                           (const double *)wt->quad, pos, soft, perm, targets_sorted != 0, wt->nslots, nt, ptg_cdiv(nt, group_size), group_offsets, group_count,
-                           group_size, theta, 1.0 / theta, crit, eps, 0.0, 0.0, nullptr, G,
-                           wt->origin[0], wt->origin[1], wt->origin[2],
-                           fn, fo, fc, out, counters, ctl, spill, gcap, start_slot};
-        st = launch_walk<double, true>(a, fields, quadrupole != 0, false, 0, blocks, s);
+        Walk64Args a{(const V4<double> *)wt->xyzm, (const V4<double> *)wt->aux, (const int2 *)wt->kids,
+                     (const double *)wt->quad, pos, soft, perm, targets_sorted != 0, wt->nslots, nt,
+                     ptg_cdiv(nt, group_size), group_offsets, group_count, group_size, theta, 1.0 / theta, G,
+                     wt->origin[0], wt->origin[1], wt->origin[2], fn, fo, out, counters, ctl, start_slot};
+        st = ptg_walk64_launch(a, fields, quadrupole != 0, num_cus(), gcap, (char *)ws, ws_bytes, s);
     } else {
         ptg_set_error("ptg_walk: prec must be PTG_F32 or PTG_F64");
         return PTG_ERR_ARG;
