@@ -413,6 +413,16 @@ ptg_status ptg_rms_rows(const double *x, int64_t rows, int stride, int col, int 
 ptg_status ptg_column_rays(const ptg_tree_arrays *tree, int64_t n, int64_t nnodes, const ptg_walk_tree *wt,
                            const double *targets, int64_t nt, const double *rays, int64_t nrays, int per_target,
                            const int64_t *order, double *out, int32_t *err, int64_t *counters, void *stream);
+/* The ray-traced columns of shared unit rays by bundles of 64 consecutive targets of `order` (nrays, nt),
+ * or of the targets as given (NULL): one wavefront walks the FP64 pack once for its bundle.  The same
+ * particles and chord terms as ptg_column_rays, summed in the bundle's order.  err as there. */
+ptg_status ptg_column_bundles(const ptg_walk_tree *wt, const double *targets, int64_t nt, const double *rays,
+                              int64_t nrays, const int64_t *order, double *out, int32_t *err, void *stream);
+/* order[i][..] = the targets in the 2D Morton order of their positions across unit ray i (no reference
+ * counterpart).  At most 65536 rays and 2^31 - 1 (target, ray) pairs; asynchronous. */
+size_t ptg_ray_orders_workspace_bytes(int64_t n, int64_t nrays);
+ptg_status ptg_ray_orders(const double *pos, int64_t n, const double *rays, int64_t nrays, int64_t *order, void *ws,
+                          size_t ws_bytes, void *stream);
 /* Angular-binned (rays=None): out (nt, 6), the mean column per equal-area sky bin, with groups of
  * group_size consecutive targets sharing one traversal opened at the node's distance to the group's
  * box (ColumnDensityBinned_grouped :1197-1276; group_size 1 is ColumnDensityWalk_binned :976-1028).

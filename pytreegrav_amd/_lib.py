@@ -124,6 +124,9 @@ SIGNATURES = {
     "ptg_walk_workspace_bytes": (_c.c_size_t, [_i64, _c.c_int]),
     "ptg_column_rays": (_c.c_int, [_c.POINTER(TreeArrays), _i64, _i64, _c.POINTER(WalkTree), _vp, _i64, _vp, _i64,
                                    _c.c_int, _vp, _vp, _vp, _vp, _vp]),
+    "ptg_column_bundles": (_c.c_int, [_c.POINTER(WalkTree), _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp]),
+    "ptg_ray_orders_workspace_bytes": (_c.c_size_t, [_i64, _i64]),
+    "ptg_ray_orders": (_c.c_int, [_vp, _i64, _vp, _i64, _vp, _vp, _c.c_size_t, _vp]),
     "ptg_column_binned": (_c.c_int, [_c.POINTER(TreeArrays), _i64, _i64, _c.POINTER(WalkTree), _vp, _i64, _i64, _dbl,
                                      _vp, _vp, _vp, _c.c_size_t, _vp, _vp]),
     "ptg_column_workspace_bytes": (_c.c_size_t, [_i64]),

@@ -1031,6 +1031,109 @@ extern "C" ptg_status ptg_morton_order(const double *pos, int64_t n, int64_t *or
     return PTG_OK;
 }
 
+// ---- target orders across rays (ptg_column_bundles) ----
+// an orthonormal pair perpendicular to the unit ray u
+__device__ __forceinline__ void ray_frame(const double *u, double (&e1)[3], double (&e2)[3])
+{
+    const double x = fabs(u[0]) < 0.9 ? 1.0 : 0.0, y = 1.0 - x;  // the axis crossed with u: x or y
+    e1[0] = -u[2] * y;
+    e1[1] = u[2] * x;
+    e1[2] = u[0] * y - u[1] * x;
+    const double r = rsqrt(e1[0] * e1[0] + e1[1] * e1[1] + e1[2] * e1[2]);
+    for (int k = 0; k < 3; k++) e1[k] *= r;
+    e2[0] = u[1] * e1[2] - u[2] * e1[1];
+    e2[1] = u[2] * e1[0] - u[0] * e1[2];
+    e2[2] = u[0] * e1[1] - u[1] * e1[0];
+}
+
+// key of (ray, target): the ray, then the 2D Morton order of the target across it, `bits` per axis of
+// the square around the targets' bounding sphere
+__global__ __launch_bounds__(256) void k_ray_keys(const double *pos, int64_t n, const double *rays, int64_t nr, int bits,
+                                                  const Geom *g, uint64_t *keys, uint32_t *vals)
+{
+    const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (id >= n * nr) return;
+    const int64_t r = id / n, i = id - r * n;
+    double e1[3], e2[3], a = 0, b = 0;
+    ray_frame(rays + 3 * r, e1, e2);
+    for (int k = 0; k < 3; k++) {
+        const double d = pos[3 * i + k] - g->center[k];
+        a += d * e1[k];
+        b += d * e2[k];
+    }
+    // the bounding cube's half diagonal is 0.866 of its side
+    const double top = (double)(1u << bits), scale = top * g->inv * (1.0 / 1.7320508);
+    const uint64_t qa = (uint64_t)fmin(fmax(a * scale + 0.5 * top, 0.0), top - 1.0);
+    const uint64_t qb = (uint64_t)fmin(fmax(b * scale + 0.5 * top, 0.0), top - 1.0);
+    uint64_t key = 0;
+    for (int k = 0; k < bits; k++) key |= ((qa >> k & 1) << (2 * k)) | ((qb >> k & 1) << (2 * k + 1));
+    keys[id] = ((uint64_t)r << (2 * bits)) | key;
+    vals[id] = (uint32_t)i;
+}
+
+struct RayWS {
+    double *part;
+    Geom *geom;
+    uint64_t *kA, *kB;
+    uint32_t *vA, *vB;
+    RsWS rs;
+};
+static bool carve_rays(PtgArena &A, int64_t cnt, RayWS &w)
+{
+    w.part = A.take<double>(6 * BB_BLOCKS);
+    w.geom = A.take<Geom>(1);
+    w.kA = A.take<uint64_t>(cnt);
+    w.kB = A.take<uint64_t>(cnt);
+    w.vA = A.take<uint32_t>(cnt);
+    w.vB = A.take<uint32_t>(cnt);
+    carve_rs(A, cnt, w.rs);
+    return A.ok();
+}
+
+extern "C" size_t ptg_ray_orders_workspace_bytes(int64_t n, int64_t nrays)
+{
+    PtgArena A(nullptr, 0);
+    RayWS w;
+    carve_rays(A, std::max<int64_t>(n * nrays, 1), w);
+    return A.used;
+}
+
+// One sort of all (ray, target) pairs: four 8-bit passes, where a 63-bit Morton sort per ray took 27
+// launches each (six rays of 1e5 targets: 1.2 ms for the orders, 0.16 ms now).
+extern "C" ptg_status ptg_ray_orders(const double *pos, int64_t n, const double *rays, int64_t nrays, int64_t *order,
+                                     void *ws, size_t ws_bytes, void *stream)
+{
+    hipStream_t s = (hipStream_t)stream;
+    if (n < 0 || nrays < 0 || nrays > (1 << 16) || n * nrays > 0x7fffffffLL ||
+        (n * nrays > 0 && (!pos || !rays || !order))) {
+        ptg_set_error("ptg_ray_orders: needs pos, rays and order, at most 65536 rays and 2^31 - 1 pairs");
+        return PTG_ERR_ARG;
+    }
+    const int64_t cnt = n * nrays;
+    if (cnt == 0) return PTG_OK;
+    PtgArena A(ws, ws_bytes);
+    RayWS w;
+    if (!ws || !carve_rays(A, cnt, w)) {
+        ptg_set_error("ptg_ray_orders: workspace too small (%zu < %zu)", ws_bytes,
+                      ptg_ray_orders_workspace_bytes(n, nrays));
+        return PTG_ERR_WORKSPACE;
+    }
+    int rbits = 0;
+    while ((1ll << rbits) < nrays) rbits++;
+    const int bits = (32 - rbits) / 2;
+    const int nb = (int)std::min<int64_t>(BB_BLOCKS, std::max<int64_t>(1, ptg_cdiv(n, 1024)));
+    k_bbox_partial<<<nb, 256, 0, s>>>(pos, n, w.part);
+    k_bbox_final<<<1, 256, 0, s>>>(w.part, nb, w.geom);
+    k_ray_keys<<<grid1(cnt), 256, 0, s>>>(pos, n, rays, nrays, bits, w.geom, w.kA, w.vA);
+    PTG_LAUNCH_CHECK();
+    bool in_first;
+    ptg_status st = radix_sort(w.kA, w.vA, w.kB, w.vB, cnt, 2 * bits + rbits, w.rs, &in_first, s);
+    if (st) return st;
+    k_u32_to_i64<<<grid1(cnt), 256, 0, s>>>(in_first ? w.vA : w.vB, cnt, order);
+    PTG_LAUNCH_CHECK();
+    return PTG_OK;
+}
+
 // forest offsets: 0 = offsets[0] < offsets[1] - 1 < ... with offsets[nsys] = n (every system holds at
 // least two particles)
 __global__ __launch_bounds__(256) void k_check_offsets(const int64_t *off, int64_t nsys, int64_t n, Counters *c)

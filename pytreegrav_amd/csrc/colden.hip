@@ -227,6 +227,214 @@ __global__ __launch_bounds__(64 * CR_WAVES) void k_column_rays_wave(const D4 *xy
     if (ctr) cd_count(ctr, 0, visits);
 }
 
+// ---- ray-traced walk of bundles: 64 targets that neighbour each other across one shared ray ----
+// One wavefront walks the tree once for its bundle, 64 elements per step (one per lane): an element is
+// opened or listed when it could meet any of the bundle's rays, tested in coordinates across the ray
+// against the bundle's rectangle, and, where the rectangle is wide against the element's reach, against
+// four quarter bundles' rectangles and then their targets one by one.  Listed particles are evaluated for
+// all 64 targets by the chord formulae of the per-target walk.  A superset of each target's own path is
+// walked, so every particle its ray crosses is met; the others add nothing.
+//
+// Bound: instruction issue (about 14 FP64 instructions per listed particle, 200 per step) and, in
+// launches of few bundles, the chain of loads per step.  Six axis rays of 1e5 targets in a Gaussian
+// cloud: 8.3 -> 0.85 ms against one element per step for all lanes (k_column_rays_wave, still the walk
+// of per-target rays, whose bundles are not parallel).
+#define CN_WAVES 4
+#define CN_SCAP 1024  // LDS stack; near its top a step takes fewer elements, so it needs no spill
+#define CN_LIST 32    // the list is evaluated in multiples of CN_LIST
+#define CN_ICAP (CN_LIST + 64)
+#define CN_WIDE 4.0   // a rectangle wider than CN_WIDE reaches is refined: 1.60 ms against 1.70 at 1, 11.8 if never
+
+struct CnLds {
+    int stack[CN_SCAP];
+    D4 part[CN_ICAP];     // x, y, z and the weight 3 m / (4 pi h^2)
+    double h[CN_ICAP], hinv[CN_ICAP];
+    double a[64], b[64];  // the targets across the ray
+};
+
+// 1/sqrt(x) by the hardware estimate and one cubic step (1-2 ulp), and sqrt(x) of x >= 0
+__device__ __forceinline__ double cn_rsqrt(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
+}
+__device__ __forceinline__ double cn_sqrt(double x) { return x > 0.0 ? x * cn_rsqrt(x) : 0.0; }
+
+__device__ __forceinline__ double cn_gap(double x, double lo, double hi) { return fmax(fmax(lo - x, x - hi), 0.0); }
+
+__device__ __forceinline__ void cn_flush(const CnLds &S, int c, double px, double py, double pz, double rx, double ry,
+                                         double rz, double &column)
+{
+    for (int k = 0; k < c; k++) {
+        const D4 P = S.part[k];
+        const double h = S.h[k];
+        const double dx = P.x - px, dy = P.y - py, dz = P.z - pz;
+        const double r2 = dx * dx + dy * dy + dz * dz;
+        const double z = rx * dx + ry * dy + rz * dz;
+        const double b2 = r2 - z * z, hh = h * h;
+        // b2 < 0 by rounding: skipped, as ColumnDensityWalk_singleray does
+        const bool inside = !(r2 > hh);
+        if (b2 >= 0 && b2 < hh && (inside || z > 0)) {
+            const double hinv = S.hinv[k];
+            const double half = cn_sqrt(1.0 - b2 * (hinv * hinv));
+            column += P.w * (inside ? z * hinv + half : 2.0 * half);
+        }
+    }
+}
+
+__global__ __launch_bounds__(64 * CN_WAVES) __attribute__((amdgpu_waves_per_eu(4))) void k_column_bundles(const D4 *xyzm, const D4 *aux, const int2 *kids,
+                                                                  int64_t nslots, const double *tp, int64_t nt,
+                                                                  const double *rays, int64_t nr, const int64_t *order,
+                                                                  double *out, int32_t *err)
+{
+    __shared__ CnLds lds[CN_WAVES];
+    const int wave = threadIdx.x >> 6, lane = ptg_lane();
+    CnLds &S = lds[wave];
+    const int64_t ntb = (nt + 63) / 64;
+    // contiguous runs of bundles per XCD (block b runs on XCD b mod 8; the grid is a multiple of 8): neighbours share their paths in its L2
+    const int64_t per = gridDim.x / 8, blk = (blockIdx.x % 8) * per + blockIdx.x / 8;
+    const int64_t task = blk * CN_WAVES + wave;
+    if (task >= ntb * nr) return;  // whole wavefronts only: task is uniform
+    const int64_t i = task / ntb, jr = (task % ntb) * 64 + lane;
+    const bool live = jr < nt;
+    const int64_t jl = live ? jr : nt - 1;  // idle lanes repeat the last target
+    const int64_t j = order ? order[i * nt + jl] : jl;
+    const double rx = rays[3 * i], ry = rays[3 * i + 1], rz = rays[3 * i + 2];
+    const double px = tp[3 * j], py = tp[3 * j + 1], pz = tp[3 * j + 2];
+    // frame of the bundle: origin at its first finite target, e1 and e2 across the ray, e3 along it.  A ray that
+    // is not of unit length meets every element (its columns are the formulae's, not a geometry's).
+    const double len2 = rx * rx + ry * ry + rz * rz;
+    const double slack0 = fabs(len2 - 1.0) < 1e-9 ? 0.0 : INFINITY;
+    const bool fin = isfinite(px) && isfinite(py) && isfinite(pz);  // others see no column and bound nothing
+    const uint64_t mf = ptg_ballot(fin);
+    const int ol = mf ? (int)__ffsll((unsigned long long)mf) - 1 : 0;
+    const double ox = __shfl(px, ol, 64), oy = __shfl(py, ol, 64), oz = __shfl(pz, ol, 64);
+    const double ax = fabs(rx) < 0.9 ? 1.0 : 0.0, ay = 1.0 - ax;
+    double e1x = -rz * ay, e1y = rz * ax, e1z = rx * ay - ry * ax;
+    const double en = 1.0 / sqrt(e1x * e1x + e1y * e1y + e1z * e1z);
+    e1x *= en;
+    e1y *= en;
+    e1z *= en;
+    const double e2x = ry * e1z - rz * e1y, e2y = rz * e1x - rx * e1z, e2z = rx * e1y - ry * e1x;
+    const double qx = fin ? px - ox : 0.0, qy = fin ? py - oy : 0.0, qz = fin ? pz - oz : 0.0;
+    const double ta = e1x * qx + e1y * qy + e1z * qz, tb = e2x * qx + e2y * qy + e2z * qz;
+    const double tc = rx * qx + ry * qy + rz * qz;
+    S.a[lane] = ta;
+    S.b[lane] = tb;
+    // rectangles of the quarters (lanes 16 s .. 16 s + 15) and of the bundle, and its nearest start
+    double alo = ta, ahi = ta, blo = tb, bhi = tb;
+#pragma unroll
+    for (int d = 1; d < 16; d <<= 1) {
+        alo = fmin(alo, __shfl_xor(alo, d, 64));
+        ahi = fmax(ahi, __shfl_xor(ahi, d, 64));
+        blo = fmin(blo, __shfl_xor(blo, d, 64));
+        bhi = fmax(bhi, __shfl_xor(bhi, d, 64));
+    }
+    const double qalo = alo, qahi = ahi, qblo = blo, qbhi = bhi;
+#pragma unroll
+    for (int d = 16; d < 64; d <<= 1) {
+        alo = fmin(alo, __shfl_xor(alo, d, 64));
+        ahi = fmax(ahi, __shfl_xor(ahi, d, 64));
+        blo = fmin(blo, __shfl_xor(blo, d, 64));
+        bhi = fmax(bhi, __shfl_xor(bhi, d, 64));
+    }
+    const double clo = ptg_wave_min(tc);
+    const double side = fmax(ahi - alo, bhi - blo);
+    const double tmax = fmax(fmax(fabs(alo), fabs(ahi)), fmax(fabs(blo), fabs(bhi)));
+    const double fac_density = 3.0 / (4.0 * 3.14159265358979323846);
+    double column = 0.0;
+    int sp = 1, np = 0;
+    if (lane == 0) S.stack[0] = 0;  // the root's walk slot
+    __builtin_amdgcn_wave_barrier();
+    while (sp > 0) {
+        // 64 elements, or as many as the stack has room for the children of
+        const int k = std::min(std::min(sp, 64), (CN_SCAP - sp) / 7);
+        if (k < 1) {  // deeper than the stack: the caller reruns the stackless walk
+            if (lane == 0) atomicOr(err, 2);
+            break;
+        }
+        const int base = sp - k;
+        int e = lane < k ? S.stack[base + lane] : 0;
+        const bool ve = lane < k && e >= 0 && e < nslots;
+        if (lane < k && !ve) atomicOr(err, 1);  // a corrupt link is reported, never followed
+        if (!ve) e = 0;
+        __builtin_amdgcn_wave_barrier();
+        sp = base;
+        const D4 X = xyzm[e], X2 = aux[e];
+        const int2 K = kids[e];
+        const bool ispart = K.y == 0;
+        const double dx = X.x - ox, dy = X.y - oy, dz = X.z - oz;
+        const double ea = e1x * dx + e1y * dy + e1z * dz, eb = e2x * dx + e2y * dy + e2z * dz;
+        const double ec = rx * dx + ry * dy + rz * dz;
+        // the coordinates above and the targets' carry a few 2^-53 of the distances: 1e-14 covers them
+        double reach = ispart ? X2.x : X2.x + X2.y * 0.8660254037844386 + X2.z;
+        reach += 1e-14 * (fabs(dx) + fabs(dy) + fabs(dz) + tmax) + slack0;
+        const double rr = reach * reach;
+        const double ga = cn_gap(ea, alo, ahi), gb = cn_gap(eb, blo, bhi);
+        bool hit = ve & (ga * ga + gb * gb <= rr) & (ec + reach > clo) & (!ispart | (X2.x > 0.0));
+        if (ptg_ballot(hit & (side > CN_WIDE * reach))) {
+            bool any = !(side > CN_WIDE * reach);
+            for (int q = 0; q < 4; q++) {
+                const double l0 = __shfl(qalo, 16 * q, 64), l1 = __shfl(qahi, 16 * q, 64);
+                const double m0 = __shfl(qblo, 16 * q, 64), m1 = __shfl(qbhi, 16 * q, 64);
+                const double a2 = cn_gap(ea, l0, l1), b2 = cn_gap(eb, m0, m1);
+                bool near = hit & !any & (a2 * a2 + b2 * b2 <= rr);
+                if (ptg_ballot(near & (fmax(l1 - l0, m1 - m0) > CN_WIDE * reach))) {
+                    bool one = !(fmax(l1 - l0, m1 - m0) > CN_WIDE * reach);
+                    for (int t = 16 * q; t < 16 * q + 16; t++) {
+                        const double da = ea - S.a[t], db = eb - S.b[t];
+                        one |= da * da + db * db <= rr;
+                    }
+                    near &= one;
+                }
+                any |= near;
+            }
+            hit &= any;
+        }
+        const bool list = hit & ispart;
+        const uint64_t bl = ptg_ballot(list);
+        if (list) {
+            const int at = np + (int)__popcll(bl & ptg_lanemask_lt());
+            const double hinv = 1.0 / X2.x;
+            S.part[at] = D4{X.x, X.y, X.z, fac_density * X.w * hinv * hinv};
+            S.h[at] = X2.x;
+            S.hinv[at] = hinv;
+        }
+        np += (int)__popcll(bl);
+        const int cnt = hit & !ispart ? std::min(std::max(K.y, 0), 8) : 0;
+        int below = 0, tot = 0;  // exclusive sum of counts below 16, one ballot per bit
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            const uint64_t m = ptg_ballot((cnt >> b) & 1);
+            below += (int)__popcll(m & ptg_lanemask_lt()) << b;
+            tot += (int)__popcll(m) << b;
+        }
+        {
+            int *dst = &S.stack[sp + below];
+#pragma unroll
+            for (int c = 0; c < 8; c++)
+                if (c < cnt) dst[c] = K.x + c;
+        }
+        sp += tot;
+        __builtin_amdgcn_wave_barrier();
+        if (np >= CN_LIST) {
+            const int c = np & ~(CN_LIST - 1);
+            cn_flush(S, c, px, py, pz, rx, ry, rz, column);
+            __builtin_amdgcn_wave_barrier();
+            if (lane < np - c) {  // reads [c, np) and writes [0, np - c): disjoint
+                S.part[lane] = S.part[c + lane];
+                S.h[lane] = S.h[c + lane];
+                S.hinv[lane] = S.hinv[c + lane];
+            }
+            __builtin_amdgcn_wave_barrier();
+            np -= c;
+        }
+    }
+    cn_flush(S, np, px, py, pz, rx, ry, rz, column);
+    if (live) out[j * nr + i] = column;
+}
+
 // angular_bin_scalar (treewalk.py:38-45)
 __device__ __forceinline__ int cd_bin(double d0, double d1, double d2)
 {
@@ -664,6 +872,30 @@ extern "C" ptg_status ptg_column_rays(const ptg_tree_arrays *tree, int64_t n, in
     k_column_rays<<<(unsigned)ptg_cdiv(work, CD_THREADS), CD_THREADS, 0, s>>>(*tree, n, n + nnodes, targets, nt, rays,
                                                                               nrays, per_target != 0, out, err,
                                                                               (unsigned long long *)counters);
+    PTG_LAUNCH_CHECK();
+    return PTG_OK;
+}
+
+extern "C" ptg_status ptg_column_bundles(const ptg_walk_tree *wt, const double *targets, int64_t nt, const double *rays,
+                                         int64_t nrays, const int64_t *order, double *out, int32_t *err, void *stream)
+{
+    hipStream_t s = (hipStream_t)stream;
+    if (!wt || wt->prec != PTG_F64 || !wt->xyzm || !wt->aux || !wt->kids || wt->nslots < 1 || nt < 0 || nrays < 1 ||
+        !rays || !out || !err || (nt > 0 && !targets)) {
+        ptg_set_error("ptg_column_bundles: needs the FP64 walk pack, targets, nrays >= 1, rays, out and err");
+        return PTG_ERR_ARG;
+    }
+    k_column_err_init<<<1, 1, 0, s>>>(err);
+    PTG_LAUNCH_CHECK();
+    if (nt == 0) return PTG_OK;
+    const int64_t blocks = ptg_cdiv(ptg_cdiv(nt, 64) * nrays, CN_WAVES);
+    if (blocks > 0x7ffffff8LL) {
+        ptg_set_error("ptg_column_bundles: too many (target, ray) pairs for one launch");
+        return PTG_ERR_ARG;
+    }
+    k_column_bundles<<<(unsigned)((blocks + 7) / 8 * 8), 64 * CN_WAVES, 0, s>>>(
+        (const D4 *)wt->xyzm, (const D4 *)wt->aux, (const int2 *)wt->kids, wt->nslots, targets, nt, rays, nrays, order,
+        out, err);
     PTG_LAUNCH_CHECK();
     return PTG_OK;
 }

@@ -674,17 +674,17 @@ def _check_counters(counters, k):
 
 def _ray_orders(tp, rays):
     """(nr, nt) int64: for each ray u, the targets sorted by the 2D Morton order of their coordinates
-    in a plane perpendicular to u (ptg_morton_order with the third coordinate zero)."""
-    orders = []
-    for u in rays.cpu().numpy():
-        u = u / np.linalg.norm(u)
-        a = np.array([1.0, 0.0, 0.0]) if abs(u[0]) < 0.9 else np.array([0.0, 1.0, 0.0])
-        e1 = np.cross(u, a)
-        e1 /= np.linalg.norm(e1)
-        e2 = np.cross(u, e1)
-        basis = torch.tensor(np.stack([e1, e2, np.zeros(3)], 1), dtype=torch.float64, device=tp.device)
-        orders.append(morton_order(tp @ basis))
-    return torch.stack(orders).contiguous()
+    in a plane perpendicular to u (ptg_ray_orders)."""
+    L = _lib.load()
+    nt, nr = tp.shape[0], rays.shape[0]
+    orders = torch.empty((nr, nt), dtype=torch.int64, device=device())
+    step = min(nr, max(1, (1 << 25) // nt), 1 << 16)  # rays per sort: its buffers hold 32 bytes a pair
+    ws = workspace(L.ptg_ray_orders_workspace_bytes(nt, step))
+    for i in range(0, nr, step):
+        k = min(step, nr - i)
+        check(L.ptg_ray_orders(ptr(tp), nt, ptr(rays[i:]), k, ptr(orders[i:]), ptr(ws), ws.numel(), stream()),
+              "ptg_ray_orders")
+    return orders
 
 
 def random_rotations(rays, nt, first_seed=0):
@@ -699,9 +699,10 @@ def random_rotations(rays, nt, first_seed=0):
 
 
 def column_rays(tree, targets, rays, per_target=False, counters=None):
-    """Ray-traced column density (ptg_column_rays): (nt, nr) float64 device tensor for targets (nt, 3)
-    and unit rays (nr, 3), or per-target rays (nt, nr, 3) when per_target.  counters: optional device
-    int64 tensor; [0] accumulates the elements visited."""
+    """Ray-traced column density: (nt, nr) float64 device tensor for targets (nt, 3) and unit rays (nr, 3)
+    (ptg_column_bundles), or per-target rays (nt, nr, 3) when per_target (ptg_column_rays).  counters:
+    optional device int64 tensor; [0] accumulates the elements visited by every target's own walk (which
+    ptg_column_rays then makes, for shared rays too)."""
     L = _lib.load()
     tp = to_dev(targets, (-1, 3))
     nt = tp.shape[0]
@@ -716,11 +717,15 @@ def column_rays(tree, targets, rays, per_target=False, counters=None):
     # shared rays: per ray, the targets in 2D Morton order of their position across the ray, so the
     # 64 targets of a wavefront walk nearly the same path
     order = _ray_orders(tp, r) if not per_target and nt > 64 else None
-    # the wavefront walk over the FP64 pack; a tree deeper than its stack reruns the stackless walk
+    # the wavefront walks over the FP64 pack; a tree deeper than their stacks reruns the stackless walk
     for wt in (_lib.ctypes.byref(tree.pack(PTG_F64, False)["wt"]), None):
-        check(L.ptg_column_rays(_lib.ctypes.byref(tree.arrays), tree.n, tree.nnodes, wt, ptr(tp), nt, ptr(r), nr,
-                                int(bool(per_target)), ptr(order) if wt is not None else None, ptr(out), ptr(err),
-                                ptr(counters), stream()), "ptg_column_rays")
+        if wt is not None and not per_target and counters is None:
+            check(L.ptg_column_bundles(wt, ptr(tp), nt, ptr(r), nr, ptr(order), ptr(out), ptr(err), stream()),
+                  "ptg_column_bundles")
+        else:
+            check(L.ptg_column_rays(_lib.ctypes.byref(tree.arrays), tree.n, tree.nnodes, wt, ptr(tp), nt, ptr(r),
+                                    nr, int(bool(per_target)), ptr(order) if wt is not None else None, ptr(out),
+                                    ptr(err), ptr(counters), stream()), "ptg_column_rays")
         e = int(err.item())
         if e & 1:
             raise RuntimeError("ptg_column_rays: corrupt tree links")
