@@ -427,9 +427,8 @@ ptg_status ptg_ray_orders(const double *pos, int64_t n, const double *rays, int6
  * group_size consecutive targets sharing one traversal opened at the node's distance to the group's
  * box (ColumnDensityBinned_grouped :1197-1276; group_size 1 is ColumnDensityWalk_binned :976-1028).
  * group_size <= 64 walks the FP64 walk pack wt of the same tree (ptg_pack_walk, PTG_F64) with
- * ptg_column_workspace_bytes(group_size) of workspace (groups whose traversal passes 32768 visits are
- * finished by a second pass that deals their subtrees out to 64 wavefronts); larger groups use the
- * tree's links (wt, ws may be NULL).
+ * ptg_column_workspace_bytes(group_size) of workspace (traversals past a budget of visits are finished
+ * in parts by later passes, as the FP64 walk's); larger groups use the tree's links (wt, ws may be NULL).
  * err: 1 corrupt links, 2 a traversal stack overflow.  counters (nullable, device int64[2],
  * accumulated): [0] element-target pairs evaluated, [1] elements visited by the group traversals. */
 size_t ptg_column_workspace_bytes(int64_t group_size);

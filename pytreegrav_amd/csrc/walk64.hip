@@ -19,14 +19,15 @@
 //
 // Bound: instruction issue, about 60 % of it the traversal (250 instructions per 64-element step).
 // Whole calls, against one wave per group evaluating every entry for 8 of its 64 lanes with IEEE
-// square roots and divisions: 1e6-particle Plummer sphere 333 -> 6.1 ms (the walk 3.2 ms of it where
-// it took 332), uniform cube of 1e5 6.0 -> 0.87 ms, tidal tensors with quadrupoles of 6e4 23.3 -> 1.6 ms.
+// square roots and divisions: 1e6-particle Plummer sphere 333 -> 4.8 ms, uniform cube of 1e5 6.0 -> 0.83
+// ms, tidal tensors with quadrupoles of 6e4 23.3 -> 1.3 ms.  Angle-binned columns of 2e5 particles
+// against their own walk (two waves per SIMD, six selected adds and a division a pair): 4.9 -> 2.25 ms.
 
 #include "walk_shared.hpp"
 
 #define LIST 32           // a list is evaluated in multiples of LIST entries once it holds LIST
 #define ICAP (LIST + 64)  // LIST - 1 entries + one step's 64
-#define BUDGET 4096       // visits after which a task is deferred (not in the last round), at least
+#define BUDGET 3072       // visits after which a task is deferred (not in the last round), at least
 #define SHARES0 64        // tasks a deferred group is cut into, at most (of DIV0 stack entries or more)
 #define DIV0 16
 #define SHARES 128        // tasks a deferred task is cut into, at most (of DIV stack entries or more)
@@ -46,20 +47,28 @@ struct Walk64Pool {
     int gcap;
     int *entries;  // saved stacks
     int ecap;
-    // task tables: the deferred groups, then the tasks of rounds 1, 2, ..; table k starts at base[k]
-    // and holds cap[k] (cap[0] = 0: nothing is deferred)
-    Walk64Task *tasks;
-    int base[WALK_ROUNDS], cap[WALK_ROUNDS];
+    Walk64Task *tasks;  // the deferred groups, then the tasks of rounds 1, 2, ..
+    double *partial;    // one row of gs * WI sums per entry of tasks
     int budget, shares0, shares;
-    double *partial;    // one row of gs * WI sums per task and deferred group, in the order of tasks
+    // this launch: its round (level of the sums), its table (cap entries of tasks from base on) and the
+    // next one's (next_cap 0: nothing is deferred).  Scalars: arrays indexed by the round would put the
+    // arguments into scratch memory.
+    int round, base, cap, next_base, next_cap;
 };
 
-template <bool QUAD> struct Lds64 {
+// FIELDS of the angle-binned column density (treewalk.py:976-1028, :1197-1276): six sums per target, kept
+// in LDS, since which of them a pair adds to differs from lane to lane (one LDS add instead of six
+// selected ones)
+#define BINS 8
+#define SKY_BIN (4.0 * 3.14159265358979323846 / 6.0)  // solid angle of a bin
+
+template <int FIELDS, bool QUAD> struct Lds64 {
     int stack[SCAP];
     V4<double> nodes[ICAP];  // elements no target can be inside the softening of: x y z m
     double nq[QUAD ? 6 * ICAP : 1];
     V4<double> parts[ICAP];  // particles: x y z m
     double ph[ICAP];
+    double bins[FIELDS == BINS ? 6 * 64 : 1];  // [bin][lane]
 };
 
 // 1/sqrt(x) and 1/x: the hardware estimate (2^-24) with one cubic step, 1-2 ulp
@@ -182,6 +191,49 @@ __device__ __forceinline__ void pair_part(Acc<double> &a, const V4<double> &s, d
     add_pair<FIELDS>(a, phi, K, Q, dx, dy, dz);
 }
 
+// angle-binned columns of one lane: LDS sums bins[64 * bin] (units of mass / distance^2) and the part
+// that goes to every bin alike
+struct Sky {
+    double *bins;
+    double iso;
+
+    __device__ __forceinline__ void add(double dx, double dy, double dz, double v)
+    {
+        // angular_bin_scalar (treewalk.py:38-45)
+        const double ax = fabs(dx), ay = fabs(dy), az = fabs(dz);
+        const bool x = ax > ay && ax > az, y = ay > az;
+        const double d = x ? dx : y ? dy : dz;
+        const int bin = (x ? 0 : y ? 2 : 4) + (d > 0 ? 0 : 1);
+        __hip_atomic_fetch_add(bins + 64 * bin, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    }
+    // an element farther than its radius: a point mass
+    __device__ __forceinline__ void node(const V4<double> &s, double tx, double ty, double tz)
+    {
+        const double dx = s.x - tx, dy = s.y - ty, dz = s.z - tz;
+        add(dx, dy, dz, s.w * rcp64(fmin(dx * dx + dy * dy + dz * dz, R2_MAX)));
+    }
+    // a particle: a point mass outside its radius h, a blend of the isotropic and directed limits inside
+    __device__ __forceinline__ void part(const V4<double> &s, double h, double tx, double ty, double tz)
+    {
+        const double dx = s.x - tx, dy = s.y - ty, dz = s.z - tz;
+        const double r2 = fmin(dx * dx + dy * dy + dz * dz, R2_MAX), hh = h * h;
+        const bool out = r2 > hh;
+        double v = s.w * rcp64(out ? r2 : 1.0);
+        if (ptg_ballot(!out)) {
+            if (!out) {
+                v = 0.0;
+                if (h > 0) {
+                    const double hinv = rcp64(h), col0 = s.w * (3.0 / (4.0 * 3.14159265358979323846) * SKY_BIN) * hinv * hinv;
+                    const double fac = r2 > 0 ? r2 * rsqrt64(r2) * hinv : 0.0;
+                    iso += (1.0 - fac) * col0;
+                    v = 2.0 * col0 * fac;
+                }
+            }
+        }
+        add(dx, dy, dz, v);
+    }
+};
+
 // components of one target's sums, in the order they are stored in a partial row
 template <int FIELDS, typename F> __device__ __forceinline__ void each_sum(Acc<double> &a, F f)
 {
@@ -201,13 +253,14 @@ template <int FIELDS, typename F> __device__ __forceinline__ void each_sum(Acc<d
     }
 }
 template <int FIELDS> struct Sums {
-    static constexpr int WI = NW<FIELDS>::POT + 3 * NW<FIELDS>::ACC + 6 * NW<FIELDS>::TID;
+    static constexpr int WI = FIELDS == BINS ? 6 : NW<FIELDS>::POT + 3 * NW<FIELDS>::ACC + 6 * NW<FIELDS>::TID;
+    static constexpr int WO = FIELDS == BINS ? 6 : NW<FIELDS>::W;  // output row
 };
 
 // the output row o[] entries that sum c of a target fills (two for an off-diagonal tidal component)
 template <int FIELDS> __device__ __forceinline__ void store_sum(double *o, int c, double v)
 {
-    constexpr int PA = NW<FIELDS>::POT + 3 * NW<FIELDS>::ACC;
+    constexpr int PA = FIELDS == BINS ? 6 : NW<FIELDS>::POT + 3 * NW<FIELDS>::ACC;
     if (!NW<FIELDS>::TID || c < PA) {
         o[c] = v;
         return;
@@ -244,23 +297,24 @@ __device__ __forceinline__ int take(int32_t *counter, int n, int cap)
 
 // waves per SIMD the registers are capped for: four where the LDS lets four blocks onto a CU
 template <int TPL, int FIELDS, bool QUAD> struct Occ64 {
-    static constexpr int waves = TPL == 1 && !QUAD && !NW<FIELDS>::TID ? 4 : 1;
+    static constexpr int waves = FIELDS == BINS ? 3 : TPL == 1 && !QUAD && !NW<FIELDS>::TID ? 4 : 1;
 };
 
 template <int TPL, int FIELDS, bool QUAD>
 __global__ __launch_bounds__(64 * WALK_WAVES) __attribute__((amdgpu_waves_per_eu(Occ64<TPL, FIELDS, QUAD>::waves)))
-void k_walk64(const Walk64Args A, const Walk64Pool B, int round)
+void k_walk64(const Walk64Args A, const Walk64Pool B)
 {
+    const int round = B.round;
     constexpr int WI = Sums<FIELDS>::WI;
-    __shared__ Lds64<QUAD> lds[WALK_WAVES];
+    __shared__ Lds64<FIELDS, QUAD> lds[WALK_WAVES];
     const int wave = threadIdx.x >> 6, lane = ptg_lane();
-    Lds64<QUAD> &L = lds[wave];
+    Lds64<FIELDS, QUAD> &L = lds[wave];
     int *spill = B.spill + ((int64_t)blockIdx.x * WALK_WAVES + wave) * (int64_t)B.gcap;
     const int xcd = blockIdx.x % NXCD;
     int64_t n_int = 0, n_vis = 0, n_part = 0;
     int ghw = 0;
     const int64_t ngroups = A.goff ? (int64_t)__builtin_amdgcn_readfirstlane(*A.gcount) : A.ngroups;
-    const int ntask = round ? std::min(__builtin_amdgcn_readfirstlane(A.ctl->ntask[round]), B.cap[round]) : 0;
+    const int ntask = round ? std::min(__builtin_amdgcn_readfirstlane(A.ctl->ntask[round]), B.cap) : 0;
     if (round && ntask == 0) return;
     // targets per slice, a power of two
     int P = 64;
@@ -282,7 +336,7 @@ void k_walk64(const Walk64Args A, const Walk64Pool B, int round)
             int64_t g = work;
             int t_off = 0, t_stride = 0, t_count = 0;
             if (round) {
-                const Walk64Task *T = &B.tasks[B.base[round] + work];
+                const Walk64Task *T = &B.tasks[B.base + work];
                 g = __builtin_amdgcn_readfirstlane(T->group);
                 t_off = __builtin_amdgcn_readfirstlane(T->off);
                 t_stride = __builtin_amdgcn_readfirstlane(T->stride);
@@ -314,13 +368,13 @@ void k_walk64(const Walk64Args A, const Walk64Pool B, int round)
             for (int j = 0; j < TPL; j++) {
                 const int o = tl + 64 * j;
                 tval[j] = o < mt;
-                tidx[j] = tval[j] ? A.perm[a0 + o] : 0;
+                tidx[j] = !tval[j] ? 0 : A.perm ? A.perm[a0 + o] : a0 + o;
                 if (tval[j]) {
                     const int64_t src = A.sorted ? a0 + o : tidx[j];
                     tx[j] = A.pos[3 * src] - ox;
                     ty[j] = A.pos[3 * src + 1] - oy;
                     tz[j] = A.pos[3 * src + 2] - oz;
-                    th[j] = A.soft[src];
+                    th[j] = A.soft ? A.soft[src] : -INFINITY;
                     bmin0 = std::min(bmin0, tx[j]);
                     bmin1 = std::min(bmin1, ty[j]);
                     bmin2 = std::min(bmin2, tz[j]);
@@ -342,6 +396,9 @@ void k_walk64(const Walk64Args A, const Walk64Pool B, int round)
             Acc<double> acc[TPL];
 #pragma unroll
             for (int j = 0; j < TPL; j++) acc[j] = Acc<double>{0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+            Sky sky{&L.bins[FIELDS == BINS ? lane : 0], 0.0};
+            if (FIELDS == BINS)
+                for (int q = 0; q < 6; q++) L.bins[64 * q + lane] = 0.0;
 
             int sp = 1, gsp = 0, nn = 0, np = 0, visits = 0;
             bool overflow = false;
@@ -361,13 +418,13 @@ void k_walk64(const Walk64Args A, const Walk64Pool B, int round)
             }
             __builtin_amdgcn_wave_barrier();
             // The more groups share the device, the longer one may run alone, and the fewer should pay for
-            // being cut: 4096 visits against 8192 take 0.83 / 0.95 ms (walk and build, 1e5 particles), 8192
-            // against 16384 2.88 / 3.30 (3e5), 12288 against 8192 6.8 / 8.0 (6e5, clumpy).  Counted per
-            // system, so that a system's cuts are those it has alone.
+            // being cut: budgets of 3072 against 8192 take 0.83 / 0.95 ms (walk and build, uniform 1e5), 3
+            // against 2 times 4096 6.8 / 8.0 (clumpy 6e5).  Counted per system, so that a system's cuts
+            // are those it has alone.
             const int64_t sg = (A.nsys > 0 ? A.soff[root + 1] - A.soff[root] : A.nt) / A.gs;
             int budget = B.budget * (round || sg <= 16384 ? 1 : sg <= 65536 ? 2 : sg <= 262144 ? 3 : 16);
-            if (round == WALK_ROUNDS - 1 || B.cap[0] == 0) budget = 0x7fffffff;
-            int child0 = -1, nchild = 0, slot = round ? B.base[round] + (int)work : -1;
+            if (B.next_cap == 0) budget = 0x7fffffff;
+            int child0 = -1, nchild = 0, slot = round ? B.base + (int)work : -1;
 
             for (;;) {
                 if (sp == 0) {
@@ -381,16 +438,17 @@ void k_walk64(const Walk64Args A, const Walk64Pool B, int round)
                 if (visits >= budget) {
                     // save the stack as interleaved shares of the next round; out of room: go on here
                     const int cnt = gsp + sp;
-                    nchild = std::max(1, round ? std::min(B.shares, cnt / DIV) : std::min(B.shares0, cnt / DIV0));
-                    const int cap = B.cap[round + 1];
+                    const int most = round ? B.shares : B.shares0, part = round ? cnt / DIV : cnt / DIV0;
+                    nchild = part > most ? most : part < 1 ? 1 : part;
+                    const int cap = B.next_cap;
                     int off = -1, at = cap;
                     if (lane == 0 && cnt <= nchild * SCAP) {
-                        if (round == 0) slot = take(&A.ctl->ntask[0], 1, B.cap[0]);
-                        if (round || slot < B.cap[0]) {
+                        if (round == 0) slot = take(&A.ctl->ntask[0], 1, B.cap);  // table 0 starts at 0
+                        if (round || slot < B.cap) {
                             at = take(&A.ctl->ntask[round + 1], nchild, cap);
                             if (at <= cap - nchild) off = take(&A.ctl->npool, cnt, B.ecap);
                             if (off > B.ecap - cnt) off = -1;
-                            if (off >= 0) child0 = B.base[round + 1] + at;
+                            if (off >= 0) child0 = B.next_base + at;
                             // a record without shares, should there be no room
                             B.tasks[slot].group = (int32_t)g;
                             B.tasks[slot].child0 = child0;
@@ -403,7 +461,7 @@ void k_walk64(const Walk64Args A, const Walk64Pool B, int round)
                     child0 = __builtin_amdgcn_readfirstlane(child0);
                     // the entries taken below cap are filled in any case: the next round reads all of them
                     for (int q = lane; q < nchild && at + q < cap; q += 64) {
-                        Walk64Task &T = B.tasks[B.base[round + 1] + at + q];
+                        Walk64Task &T = B.tasks[B.next_base + at + q];
                         T.group = (int32_t)g;
                         T.nchild = 0;
                         T.off = off + q;
@@ -499,8 +557,10 @@ void k_walk64(const Walk64Args A, const Walk64Pool B, int round)
                     for (int q = sl; q < c; q += slices) {
                         const V4<double> s = L.nodes[q];
 #pragma unroll
-                        for (int j = 0; j < TPL; j++)
-                            pair_node<FIELDS, QUAD>(acc[j], s, &L.nq[QUAD ? 6 * q : 0], tx[j], ty[j], tz[j]);
+                        for (int j = 0; j < TPL; j++) {
+                            if constexpr (FIELDS == BINS) sky.node(s, tx[j], ty[j], tz[j]);
+                            else pair_node<FIELDS, QUAD>(acc[j], s, &L.nq[QUAD ? 6 * q : 0], tx[j], ty[j], tz[j]);
+                        }
                     }
                     __builtin_amdgcn_wave_barrier();
                     if (lane < nn - c) {  // reads [c, nn) and writes [0, nn - c): disjoint
@@ -516,7 +576,10 @@ void k_walk64(const Walk64Args A, const Walk64Pool B, int round)
                     for (int q = sl; q < c; q += slices) {
                         const V4<double> s = L.parts[q];
 #pragma unroll
-                        for (int j = 0; j < TPL; j++) pair_part<FIELDS>(acc[j], s, L.ph[q], tx[j], ty[j], tz[j], th[j]);
+                        for (int j = 0; j < TPL; j++) {
+                            if constexpr (FIELDS == BINS) sky.part(s, L.ph[q], tx[j], ty[j], tz[j]);
+                            else pair_part<FIELDS>(acc[j], s, L.ph[q], tx[j], ty[j], tz[j], th[j]);
+                        }
                     }
                     __builtin_amdgcn_wave_barrier();
                     if (lane < np - c) {  // disjoint ranges, as above
@@ -535,16 +598,30 @@ void k_walk64(const Walk64Args A, const Walk64Pool B, int round)
             for (int q = sl; q < nn; q += slices) {
                 const V4<double> s = L.nodes[q];
 #pragma unroll
-                for (int j = 0; j < TPL; j++)
-                    pair_node<FIELDS, QUAD>(acc[j], s, &L.nq[QUAD ? 6 * q : 0], tx[j], ty[j], tz[j]);
+                for (int j = 0; j < TPL; j++) {
+                    if constexpr (FIELDS == BINS) sky.node(s, tx[j], ty[j], tz[j]);
+                    else pair_node<FIELDS, QUAD>(acc[j], s, &L.nq[QUAD ? 6 * q : 0], tx[j], ty[j], tz[j]);
+                }
             }
             for (int q = sl; q < np; q += slices) {
                 const V4<double> s = L.parts[q];
 #pragma unroll
-                for (int j = 0; j < TPL; j++) pair_part<FIELDS>(acc[j], s, L.ph[q], tx[j], ty[j], tz[j], th[j]);
+                for (int j = 0; j < TPL; j++) {
+                    if constexpr (FIELDS == BINS) sky.part(s, L.ph[q], tx[j], ty[j], tz[j]);
+                    else pair_part<FIELDS>(acc[j], s, L.ph[q], tx[j], ty[j], tz[j], th[j]);
+                }
             }
             __builtin_amdgcn_wave_barrier();
-            for (int d = P; d < 64; d <<= 1) {
+            [[maybe_unused]] double bin[FIELDS == BINS ? 6 : 1];
+            if constexpr (FIELDS == BINS) {
+#pragma unroll
+                for (int q = 0; q < 6; q++) bin[q] = L.bins[64 * q + lane] + sky.iso;
+                for (int d = P; d < 64; d <<= 1) {
+#pragma unroll
+                    for (int q = 0; q < 6; q++) bin[q] += __shfl_xor(bin[q], d, 64);
+                }
+            }
+            for (int d = P; FIELDS != BINS && d < 64; d <<= 1) {
 #pragma unroll
                 for (int j = 0; j < TPL; j++) each_sum<FIELDS>(acc[j], [&](double &v) { v += __shfl_xor(v, d, 64); });
             }
@@ -556,11 +633,19 @@ void k_walk64(const Walk64Args A, const Walk64Pool B, int round)
                 if (!tval[j] || sl != 0) continue;
                 int c = 0;
                 if (whole) {
-                    double *o = A.out + tidx[j] * NW<FIELDS>::W;
+                    double *o = A.out + tidx[j] * Sums<FIELDS>::WO;
                     each_sum<FIELDS>(acc[j], [&](double &v) { store_sum<FIELDS>(o, c++, A.G * v); });
+                    if constexpr (FIELDS == BINS) {
+#pragma unroll
+                        for (int q = 0; q < 6; q++) o[q] = A.G * bin[q];
+                    }
                 } else {
                     double *o = B.partial + ((int64_t)slot * A.gs + tl + 64 * j) * WI;
                     each_sum<FIELDS>(acc[j], [&](double &v) { o[c++] = v; });
+                    if constexpr (FIELDS == BINS) {
+#pragma unroll
+                        for (int q = 0; q < 6; q++) o[q] = bin[q];
+                    }
                 }
             }
         }
@@ -569,34 +654,34 @@ void k_walk64(const Walk64Args A, const Walk64Pool B, int round)
     if (lane == 0 && A.counters) {
         atomicAdd((unsigned long long *)&A.counters[0], (unsigned long long)n_int);
         atomicAdd((unsigned long long *)&A.counters[1], (unsigned long long)n_vis);
-        atomicAdd((unsigned long long *)&A.counters[2], (unsigned long long)n_part);
+        if (FIELDS != BINS) atomicAdd((unsigned long long *)&A.counters[2], (unsigned long long)n_part);
     }
 }
 
-// Adds to the row of each deferred task of round `level` the rows of its shares, in order; level 0:
+// Adds to the row of each deferred task of round B.round the rows of its shares, in order; round 0:
 // the deferred groups, whose totals are the results.  One wave per deferred task, deepest level first.
 template <int FIELDS>
-__global__ __launch_bounds__(256) void k_walk64_sum(const Walk64Args A, const Walk64Pool B, int level)
+__global__ __launch_bounds__(256) void k_walk64_sum(const Walk64Args A, const Walk64Pool B)
 {
     constexpr int WI = Sums<FIELDS>::WI;
-    const int nt = std::min(__builtin_amdgcn_readfirstlane(A.ctl->ntask[level]), B.cap[level]);
+    const int nt = std::min(__builtin_amdgcn_readfirstlane(A.ctl->ntask[B.round]), B.cap);
     const int64_t rs = (int64_t)A.gs * WI;
     for (int t = blockIdx.x * 4 + (threadIdx.x >> 6); t < nt; t += gridDim.x * 4) {
-        const Walk64Task T = B.tasks[B.base[level] + t];
+        const Walk64Task T = B.tasks[B.base + t];
         if (T.nchild == 0) continue;
         const Group64 grp = group_of(A, T.group);
         const int nv = grp.mt * WI;
-        double *row = B.partial + (B.base[level] + t) * rs;
+        double *row = B.partial + (int64_t)(B.base + t) * rs;
         const double *kids = B.partial + T.child0 * rs;
         for (int v = ptg_lane(); v < nv; v += 64) {
             double s = row[v];
 #pragma unroll 8
             for (int k = 0; k < T.nchild; k++) s += kids[k * rs + v];
-            if (level) {
+            if (B.round) {
                 row[v] = s;
             } else {
-                const int64_t o = A.perm[grp.a0 + v / WI];
-                store_sum<FIELDS>(A.out + o * NW<FIELDS>::W, v % WI, A.G * s);
+                const int64_t t = grp.a0 + v / WI, o = A.perm ? A.perm[t] : t;
+                store_sum<FIELDS>(A.out + o * Sums<FIELDS>::WO, v % WI, A.G * s);
             }
         }
     }
@@ -628,7 +713,11 @@ static ptg_status launch(const Walk64Args &a, int cus, int gcap, char *ws, size_
     };
     b.gcap = gcap;
     b.spill = (int *)carve((size_t)cus * per_cu * WALK_WAVES * gcap * sizeof(int));
-    const size_t left = ws_bytes > at ? ws_bytes - at : 0;
+    if (at > ws_bytes) {
+        ptg_set_error("FP64 walk: workspace too small (%zu < %zu)", ws_bytes, at);
+        return PTG_ERR_WORKSPACE;
+    }
+    const size_t left = ws_bytes - at;
     const size_t pool = std::min<size_t>(left / 8 * 3, 48u << 20);
     const size_t row = (size_t)a.gs * Sums<FIELDS>::WI * sizeof(double);
     // an ordinary group's traversal stays well inside the budget: it grows as 1 / theta^2 and with the group
@@ -637,28 +726,36 @@ static ptg_status launch(const Walk64Args &a, int cus, int gcap, char *ws, size_
     b.shares0 = (int)std::min<size_t>(SHARES0, std::max<size_t>(16, SHARE_BYTES / row));
     b.shares = (int)std::min<size_t>(SHARES, std::max<size_t>(16, SHARE_BYTES / row));
     const size_t nrows = left > pool + 1024 ? (left - pool - 1024) / (row + sizeof(Walk64Task)) : 0;
-    const int most = (int)std::min<size_t>(MAX_TASKS, nrows * 3 / 5);
+    const int most = (int)std::min<size_t>(MAX_TASKS, nrows / 2);
+    int base[WALK_ROUNDS + 1] = {}, cap[WALK_ROUNDS + 1] = {}, n = 0;
     if (most >= SHARES) {
         b.ecap = (int)(pool / sizeof(int));
         b.entries = (int *)carve(pool);
-        int n = 0;
-        for (int k = 0; k < WALK_ROUNDS; k++) {  // nrows * 0.6 * (1/8 + 1 + 1/4 + 1/4) rows at most
-            b.base[k] = n;
-            n += b.cap[k] = k == 0 ? most / 8 : k == 1 ? most : most / 4;
+        for (int k = 0; k < WALK_ROUNDS; k++) {  // nrows / 2 * (1/8 + 1 + 3 * 1/4) rows at most
+            base[k] = n;
+            n += cap[k] = k == 0 ? most / 8 : k == 1 ? most : most / 4;
         }
         b.tasks = (Walk64Task *)carve(n * sizeof(Walk64Task));
         b.partial = (double *)carve(n * row);
     }
     const int64_t blocks = (int64_t)cus * per_cu;
     // a task of round r is what r budgets left of one traversal, which visits a slot once
-    const int rounds = b.cap[0] ? (int)std::min<int64_t>(WALK_ROUNDS, 1 + a.nslots / b.budget) : 1;
+    const int rounds = n ? (int)std::min<int64_t>(WALK_ROUNDS, 1 + a.nslots / b.budget) : 1;
     for (int round = 0; round < rounds; round++) {
         const int64_t nb = round || a.goff ? blocks : std::min(blocks, ptg_cdiv(a.ngroups, WALK_WAVES));
-        k_walk64<TPL, FIELDS, QUAD><<<(unsigned)nb, 64 * WALK_WAVES, 0, s>>>(a, b, round);
+        b.round = round;
+        b.base = base[round];
+        b.cap = cap[round];
+        b.next_base = base[round + 1];
+        b.next_cap = cap[round + 1];
+        k_walk64<TPL, FIELDS, QUAD><<<(unsigned)nb, 64 * WALK_WAVES, 0, s>>>(a, b);
         PTG_LAUNCH_CHECK();
     }
-    for (int level = rounds - 2; level >= 0; level--) {
-        k_walk64_sum<FIELDS><<<256, 256, 0, s>>>(a, b, level);
+    for (int round = rounds - 2; round >= 0; round--) {
+        b.round = round;
+        b.base = base[round];
+        b.cap = cap[round];
+        k_walk64_sum<FIELDS><<<256, 256, 0, s>>>(a, b);
         PTG_LAUNCH_CHECK();
     }
     return PTG_OK;
@@ -686,4 +783,9 @@ ptg_status ptg_walk64_launch(const Walk64Args &a, int fields, bool quad, int cus
     if (a.gs <= 64) return launch_fields<1>(a, fields, quad, cus, gcap, ws, ws_bytes, s);
     if (a.gs <= 128) return launch_fields<2>(a, fields, quad, cus, gcap, ws, ws_bytes, s);
     return launch_fields<4>(a, fields, quad, cus, gcap, ws, ws_bytes, s);
+}
+
+ptg_status ptg_walk64_bins(const Walk64Args &a, int cus, int gcap, char *ws, size_t ws_bytes, hipStream_t s)
+{
+    return launch<1, BINS, false>(a, cus, gcap, ws, ws_bytes, s);
 }

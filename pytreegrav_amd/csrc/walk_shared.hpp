@@ -17,7 +17,7 @@ template <typename T> struct alignas(4 * sizeof(T)) V4 {
     T x, y, z, w;
 };
 
-#define WALK_ROUNDS 4  // FP64 walk: the group pass and the passes over the subtrees it deferred
+#define WALK_ROUNDS 5  // FP64 walk: the group pass and the passes over the subtrees it deferred
 
 struct WalkCtl {
     int32_t ctr[NXCD * CTR_STRIDE];   // per-XCD group counters
@@ -26,7 +26,7 @@ struct WalkCtl {
     int32_t pad[30];
     // FP64 walk: entries of the task tables (deferred groups, then the tasks of rounds 1, 2, ..), stack
     // entries saved, per-XCD counters of the tasks taken
-    int32_t ntask[WALK_ROUNDS], npool, pad2[27];
+    int32_t ntask[WALK_ROUNDS], npool, pad2[31 - WALK_ROUNDS];
     int32_t tctr[(WALK_ROUNDS - 1) * NXCD * CTR_STRIDE];
 };
 
@@ -98,8 +98,8 @@ struct Walk64Args {
     const int2 *kids;
     const double *quad;  // 8 per slot
     const double *pos;
-    const double *soft;
-    const int64_t *perm;
+    const double *soft;   // NULL: none
+    const int64_t *perm;  // NULL: the targets in the order given
     int sorted;  // pos/soft are indexed by the sorted target position (perm maps the outputs only)
     int64_t nslots;
     int64_t nt;
@@ -120,5 +120,8 @@ struct Walk64Args {
 
 // launches the walk on a workspace whose control block ws starts with (cleared by the caller); gcap =
 // spill entries per wave; cus = the device's compute units
+// angle-binned column density (colden.hip): groups of gs <= 64 sorted targets, six sums each (soft and
+// perm NULL: no softening, rows in target order), scaled by G
+ptg_status ptg_walk64_bins(const Walk64Args &a, int cus, int gcap, char *ws, size_t ws_bytes, hipStream_t s);
 ptg_status ptg_walk64_launch(const Walk64Args &a, int fields, bool quad, int cus, int gcap, char *ws, size_t ws_bytes,
                              hipStream_t s);
