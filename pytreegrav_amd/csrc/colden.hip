@@ -535,7 +535,7 @@ static int cb_cus()
 extern "C" size_t ptg_column_workspace_bytes(int64_t group_size)
 {
     (void)group_size;
-    return ptg_align256(sizeof(WalkCtl)) + (size_t)cb_cus() * 3 * WALK_WAVES * CB_GCAP * sizeof(int) + CB_POOL;
+    return walk_control_bytes() + (size_t)cb_cus() * 3 * WALK_WAVES * CB_GCAP * sizeof(int) + CB_POOL;
 }
 
 // the walk's flags as ptg_column_binned reports them
@@ -543,11 +543,6 @@ __global__ void k_column_err_out(const WalkCtl *ctl, int32_t *err)
 {
     if (ctl->err) *err |= 2;  // a traversal stack overflow
 }
-__global__ void k_column_ctl_init(WalkCtl *ctl)
-{
-    for (int i = threadIdx.x; i < (int)(sizeof(WalkCtl) / 4); i += blockDim.x) ((int32_t *)ctl)[i] = 0;
-}
-
 __global__ void k_column_err_init(int32_t *err) { *err = 0; }
 static ptg_status column_common(const ptg_tree_arrays *tree, int64_t n, int64_t nnodes, const double *targets,
                                 int64_t nt, const char *who)
@@ -726,8 +721,8 @@ extern "C" ptg_status ptg_column_binned(const ptg_tree_arrays *tree, int64_t n, 
             return PTG_ERR_ARG;
         }
         WalkCtl *ctl = (WalkCtl *)ws;
-        k_column_ctl_init<<<1, 256, 0, s>>>(ctl);
-        PTG_LAUNCH_CHECK();
+        st = walk_clear(ctl, s);
+        if (st) return st;
         const Walk64Args a{(const V4<double> *)wt->xyzm, (const V4<double> *)wt->aux, (const int2 *)wt->kids, nullptr,
                            targets, nullptr, nullptr, 1, wt->nslots, nt, ptg_cdiv(nt, group_size), nullptr, nullptr,
                            (int)group_size, theta, 1.0 / theta, 6.0 / (4.0 * 3.14159265358979323846), 0.0, 0.0, 0.0, 0,

@@ -17,6 +17,11 @@
 
 #include "walk_shared.hpp"
 
+#define BUDGET 4096  // visits after which a traversal is cut (walk_shared.hpp), at least
+
+// groups a system has at least where its traversals are cut
+__host__ __device__ constexpr int cut_groups(int fields) { return fields & PTG_TIDAL ? 2048 : 1024; }
+
 // a list is evaluated in multiples of LF entries once it holds LF (a power of 2: 64, or 32 for the
 // six-wave variant); a list holds LF - 1 + one step's 64 entries (ICAP)
 
@@ -61,8 +66,6 @@ template <typename T> struct WalkArgs {
     double *out;
     int64_t *counters;
     WalkCtl *ctl;
-    int *spill;
-    int gcap;  // global spill entries per wave (GCAP, or what the static scratch of ptg_walk_noalloc gives)
 };
 
 __device__ __forceinline__ float fast_rsqrt(float x) { return __builtin_amdgcn_rsqf(x); }
@@ -359,36 +362,51 @@ template <typename T, int TPL, int VAR> struct WalkOcc {
     static constexpr int blocks_per_cu = fast && VAR == 2 ? 6 : 5;
 };
 
-template <typename T, int TPL, int FIELDS, bool QUAD, bool EXP, int VAR>
+// PASS: the groups' walks that are never cut, those that may be, the tasks of those that were
+enum { WHOLE, CUT, TASK };
+
+template <typename T, int TPL, int FIELDS, bool QUAD, bool EXP, int VAR, int PASS>
 __global__ __launch_bounds__(64 * WALK_WAVES) __attribute__((amdgpu_waves_per_eu(WalkOcc<T, TPL, VAR>::waves)))
-void k_walk(WalkArgs<T> A)
+void k_walk(const WalkArgs<T> A, const WalkPool B)
 {
     constexpr int LF = WalkOcc<T, TPL, VAR>::lf;
+    constexpr bool TASKS = PASS == TASK;
     static_assert(!EXP || (!QUAD && !NW<FIELDS>::TID), "the group expansion is a monopole potential/acceleration path");
     __shared__ WaveLds<T, QUAD, LF> lds[WALK_WAVES];
     const int wave = threadIdx.x >> 6, lane = ptg_lane();
     WaveLds<T, QUAD, LF> &L = lds[wave];
-    const int64_t gwave = (int64_t)blockIdx.x * WALK_WAVES + wave;
-    int *spill = A.spill + gwave * (int64_t)A.gcap;
+    int *spill = B.spill + ((int64_t)blockIdx.x * WALK_WAVES + wave) * (int64_t)B.gcap;
     const int xcd = blockIdx.x % NXCD;
-    int64_t n_int = 0, n_vis = 0, n_part = 0, n_exp = 0;
     int ghw = 0;  // this wave's deepest spill
     const int64_t ngroups = A.goff ? (int64_t)__builtin_amdgcn_readfirstlane(*A.gcount) : A.ngroups;
 
-    for (int attempt = 0; attempt < NXCD; attempt++) {
+    int closed = 0;
+    if (TASKS && agent_load(&A.ctl->open) == 0) return;  // nothing was deferred, or all of it is done
+
+    for (int attempt = 0; attempt < (TASKS ? 1 : NXCD); attempt++) {
         const int x = (xcd + attempt) % NXCD;
         const int64_t g_lo = ngroups * x / NXCD, g_hi = ngroups * (x + 1) / NXCD;
         for (;;) {
-            int gi = 0;
-            if (lane == 0) gi = atomicAdd(&A.ctl->ctr[x * CTR_STRIDE], 1);
-            gi = __builtin_amdgcn_readfirstlane(gi);
-            const int64_t g = g_lo + gi;
-            if (g >= g_hi) break;
-            const int64_t a0 = A.goff ? (int64_t)A.goff[g] : g * A.gs;
-            const int64_t e0 = A.goff ? (int64_t)A.goff[g + 1] : A.nt;
-            const int64_t b0 = e0 < a0 + A.gs ? e0 : a0 + A.gs;
-            const int mt = (int)(b0 - a0);
-            if (A.goff && e0 > b0 && lane == 0) atomicOr(&A.ctl->err, 2);  // a supplied group larger than group_size
+            int self = -1, t_off = 0, t_stride = 0, t_count = 0;
+            int64_t g;
+            if (TASKS) {
+                self = walk_ticket(A.ctl, B, lane, closed);
+                if (self < 0) break;
+                const WalkTask *W = &B.tasks[self];
+                g = __builtin_amdgcn_readfirstlane(agent_load(&W->group));
+                t_off = __builtin_amdgcn_readfirstlane(agent_load(&W->off));
+                t_stride = __builtin_amdgcn_readfirstlane(agent_load(&W->stride));
+                t_count = __builtin_amdgcn_readfirstlane(agent_load(&W->count));
+            } else {
+                int gi = 0;
+                if (lane == 0) gi = atomicAdd(&A.ctl->ctr[x * CTR_STRIDE], 1);
+                g = g_lo + __builtin_amdgcn_readfirstlane(gi);
+                if (g >= g_hi) break;
+            }
+            const WalkSpan grp = walk_span(A.goff, A.gs, A.nt, g);
+            const int64_t a0 = grp.a0;
+            const int mt = grp.mt;
+            if (grp.over && lane == 0) atomicOr(&A.ctl->err, 2);  // a supplied group larger than group_size
             int root = 0;
             double ox = A.ox, oy = A.oy, oz = A.oz;
             if (A.nsys > 0) {
@@ -406,17 +424,17 @@ void k_walk(WalkArgs<T> A)
 
             // ---- targets: lane holds a0 + lane + 64 j ----
             T tx[TPL], ty[TPL], tz[TPL], th[TPL];
-            int64_t tidx[TPL];
             bool tval[TPL];
+            int64_t tidx[TPL];  // rows of out, where the registers for them are there
             T bmin0 = INFINITY, bmin1 = INFINITY, bmin2 = INFINITY;
             T bmax0 = -INFINITY, bmax1 = -INFINITY, bmax2 = -INFINITY, hmax = -INFINITY;
 #pragma unroll
             for (int j = 0; j < TPL; j++) {
                 const int o = lane + 64 * j;
                 tval[j] = o < mt;
-                tidx[j] = tval[j] ? A.perm[a0 + o] : 0;
+                if (PASS == WHOLE) tidx[j] = tval[j] ? A.perm[a0 + o] : 0;
                 if (tval[j]) {
-                    const int64_t src = A.sorted ? a0 + o : tidx[j];
+                    const int64_t src = A.sorted ? a0 + o : PASS == WHOLE ? tidx[j] : A.perm[a0 + o];
                     tx[j] = (T)(A.pos[3 * src] - ox);
                     ty[j] = (T)(A.pos[3 * src + 1] - oy);
                     tz[j] = (T)(A.pos[3 * src + 2] - oz);
@@ -466,150 +484,198 @@ void k_walk(WalkArgs<T> A)
             }
 
             int sp = 1, gsp = 0, nn = 0, np = 0;
-            bool overflow = false;
-            if (lane == 0) L.stack[0] = root;  // the root of system s occupies walk slot s
+            bool overflow = false, cut = false;
+            if (TASKS) {
+                sp = t_count;  // <= SCAP: deeper stacks are not deferred
+                for (int q = lane; q < sp; q += 64) L.stack[q] = agent_load(&B.entries[t_off + (int64_t)q * t_stride]);
+            } else if (lane == 0) {
+                L.stack[0] = root;  // the root of system s occupies walk slot s
+            }
             __builtin_amdgcn_wave_barrier();
+            // Visits after which the traversal is cut.  Few groups: none, each opens much of the tree and its
+            // sums run over up to all particles in FP32, so that another order of the terms moves the
+            // fields (1e-4 of their RMS for 200 targets among 3e6 clumpy particles, tidal tensors 1e-3;
+            // with the groups asked for 8e-6, 8e-6).  Middling: the longest traversal sets the time (66000
+            // targets among 3e6 clumpy particles 22.4 -> 1.8 ms).  Many: the device is full without, and
+            // the tables would fill (1e6 clumpy targets of 1e6 particles: 14.5 ms, 9.8 as here, 14.6 with
+            // BUDGET; 2.2e6: 36 ms, 42 with BUDGET).  By the targets of the group's own system, so that a
+            // system's cuts are those it has alone.
+            int budget = 0x7fffffff;
+            if (PASS == TASK) {
+                budget = B.budget;
+            } else if (PASS == CUT) {
+                const int64_t sg = (A.nsys > 0 ? A.soff[root + 1] - A.soff[root] : A.nt) / A.gs;
+                const float many = fmaxf(1.0f, (float)sg * (1.0f / 5120));
+                if (sg >= cut_groups(FIELDS)) budget = (int)fminf((float)B.budget * many * sqrtf(many), 2e9f);
+            }
+            int nchild = 0, off = 0, child0 = 0;
+            // counts of this traversal: elements visited, listed, listed as particles; folded (per lane)
+            int n_vis = 0, n_list = 0, n_part = 0, n_exp = 0;
 
-            for (;;) {
-                // pop up to 64 stack entries, one per lane, refilling the LDS stack from the spill
-                // region when it is empty
-                if (sp == 0) {
-                    if (gsp > 0) {
-                        const int k = std::min(gsp, SPILL);
-                        for (int q = lane; q < k; q += 64) L.stack[q] = spill[gsp - k + q];
-                        __builtin_amdgcn_wave_barrier();
-                        gsp -= k;
-                        sp = k;
-                    } else {
-                        break;
-                    }
-                }
-                const int k = std::min(sp, 64);
-                const int base = sp - k;
-                int e = lane < k ? L.stack[base + lane] : 0;
-                const bool ve = lane < k && e >= 0 && e < A.nslots;  // a corrupt link is dropped, not followed
-                if (!ve) e = 0;
-                __builtin_amdgcn_wave_barrier();
-                sp = base;
-                n_vis += k;
-                const V4<T> X = A.xyzm[e];
-                const V4<T> X2 = A.aux[e];
-                const int2 K = A.kids[e];
-                const bool ispart = K.y == 0;
-                // distance to the box per axis: max(bmin - x, x - bmax, 0), the same value as the
-                // two-sided test (one max3 per axis)
-                const T dxm = box_gap(X.x, bmin0, bmax0), dym = box_gap(X.y, bmin1, bmax1), dzm = box_gap(X.z, bmin2, bmax2);
-                const T r2m = dxm * dxm + dym * dym + dzm * dzm;
-                const T hh = X2.x > hmax ? X2.x : hmax;
-                // the reference's test (treewalk.py:22-25) on squared distances (every threshold is >= 0),
-                // with 1/theta; evaluated without branches (bitwise &) so the slot's aux record is one
-                // load issued with the others, not a second round trip inside a branch
-                const T c1 = X2.y * A.inv_theta + X2.z;
-                const T c2 = hh + X2.y * T(0.6) + X2.z;
-                const T c = c1 > c2 ? c1 : c2;
-                bool acc_node = ve & !ispart & (r2m > c * c);
-                // a particle farther from the group's box than every softening radius (and not
-                // inside it) needs neither the softening nor the self test -> node list
-                const bool far_part = ve & ispart & (r2m > hh * hh);
-                if (A.crit == 1) {
-                    // error-bounded: also require the quadrupole term the monopole drops,
-                    // 3.5 |Q| / r^4, to stay below eps (theta is then only a loose cap)
-                    acc_node = acc_node & (X2.w < A.eps * r2m * r2m);
-                } else if (A.crit == 2) {
-                    // learned: r_min beyond the node's predicted opening radius
-                    acc_node = acc_node & (r2m > X2.w * X2.w);
-                }
-                bool acc_part = ve && ispart && !far_part;
-                acc_node = acc_node || far_part;
-                bool open = ve && !ispart && !acc_node;
-                if constexpr (EXP) {
-                    if (acc_node) {
-                        // accepted elements are outside every softening radius and r_min > 0,
-                        // so D >= r_min > 0; fold if the truncation bound is within the tolerance
-                        const T Dx = X.x - cx, Dy = X.y - cy, Dz = X.z - cz;
-                        T rinv;
-                        if (fold_test(X.w, Dx, Dy, Dz, rg, eps_x, A.exp_rel, rinv)) {
-                            exp_add(E, X.w, Dx, Dy, Dz, rinv);
-                            acc_node = false;
-                            n_exp++;
+            for (;;) {  // once more only where a deferred traversal finds no room
+                for (;;) {
+                    // pop up to 64 stack entries, one per lane, refilling the LDS stack from the spill
+                    // region when it is empty
+                    if (sp == 0) {
+                        if (gsp > 0) {
+                            const int k = std::min(gsp, SPILL);
+                            for (int q = lane; q < k; q += 64) L.stack[q] = spill[gsp - k + q];
+                            __builtin_amdgcn_wave_barrier();
+                            gsp -= k;
+                            sp = k;
+                        } else {
+                            break;
                         }
                     }
-                }
-
-                const uint64_t bp = ptg_ballot(acc_part), bn = ptg_ballot(acc_node);
-                if (acc_part) {
-                    const int at = np + lanes_below(bp);
-                    L.parts[at] = X;
-                    L.ph[at] = X2.x;
-                }
-                if (acc_node) {
-                    const int at = nn + lanes_below(bn);
-                    L.nodes[at] = X;
-                    if (QUAD) {
-                        const T *q = A.quad + 8 * (int64_t)e;
-#pragma unroll
-                        for (int c = 0; c < 6; c++) L.nq[6 * at + c] = q[c];
-                    }
-                }
-                const int addp = (int)__popcll(bp), addn = (int)__popcll(bn);
-                np += addp;
-                nn += addn;
-                n_int += (int64_t)(addp + addn) * mt;
-                n_part += (int64_t)addp * mt;
-
-                // push the children of opened nodes
-                const int cnt = open ? std::min(std::max(K.y, 0), 8) : 0;
-                int tot;
-                const int below = small_excl_scan(cnt, tot);
-                if (sp + tot > SCAP) {
-                    // move the bottom ks entries of the LDS stack to this wave's global region
-                    const int ks = spill_count(sp, tot);
-                    if (gsp + ks > A.gcap) {
-                        overflow = true;
+                    if (PASS != WHOLE && n_vis >= budget) {
+                        cut = true;
                         break;
                     }
-                    spill_bottom(L.stack, spill + gsp, sp, ks, lane);
-                    gsp += ks;
-                    sp -= ks;
-                    ghw = std::max(ghw, gsp);
-                }
-                {
-                    // unrolled: eight masked LDS stores with immediate offsets, no per-lane loop
-                    int *dst = &L.stack[sp + below];
-#pragma unroll
-                    for (int c = 0; c < 8; c++)
-                        if (c < cnt) dst[c] = K.x + c;
-                }
-                sp += tot;
-                __builtin_amdgcn_wave_barrier();
+                    const int k = std::min(sp, 64);
+                    const int base = sp - k;
+                    int e = lane < k ? L.stack[base + lane] : 0;
+                    const bool ve = lane < k && e >= 0 && e < A.nslots;  // a corrupt link is dropped, not followed
+                    if (!ve) e = 0;
+                    __builtin_amdgcn_wave_barrier();
+                    sp = base;
+                    n_vis += k;
+                    const V4<T> X = A.xyzm[e];
+                    const V4<T> X2 = A.aux[e];
+                    const int2 K = A.kids[e];
+                    const bool ispart = K.y == 0;
+                    // distance to the box per axis: max(bmin - x, x - bmax, 0), the same value as the
+                    // two-sided test (one max3 per axis)
+                    const T dxm = box_gap(X.x, bmin0, bmax0), dym = box_gap(X.y, bmin1, bmax1), dzm = box_gap(X.z, bmin2, bmax2);
+                    const T r2m = dxm * dxm + dym * dym + dzm * dzm;
+                    const T hh = X2.x > hmax ? X2.x : hmax;
+                    // the reference's test (treewalk.py:22-25) on squared distances (every threshold is >= 0),
+                    // with 1/theta; evaluated without branches (bitwise &) so the slot's aux record is one
+                    // load issued with the others, not a second round trip inside a branch
+                    const T c1 = X2.y * A.inv_theta + X2.z;
+                    const T c2 = hh + X2.y * T(0.6) + X2.z;
+                    const T c = c1 > c2 ? c1 : c2;
+                    bool acc_node = ve & !ispart & (r2m > c * c);
+                    // a particle farther from the group's box than every softening radius (and not
+                    // inside it) needs neither the softening nor the self test -> node list
+                    const bool far_part = ve & ispart & (r2m > hh * hh);
+                    if (A.crit == 1) {
+                        // error-bounded: also require the quadrupole term the monopole drops,
+                        // 3.5 |Q| / r^4, to stay below eps (theta is then only a loose cap)
+                        acc_node = acc_node & (X2.w < A.eps * r2m * r2m);
+                    } else if (A.crit == 2) {
+                        // learned: r_min beyond the node's predicted opening radius
+                        acc_node = acc_node & (r2m > X2.w * X2.w);
+                    }
+                    bool acc_part = ve && ispart && !far_part;
+                    acc_node = acc_node || far_part;
+                    bool open = ve && !ispart && !acc_node;
+                    if constexpr (EXP) {
+                        if (acc_node) {
+                            // accepted elements are outside every softening radius and r_min > 0,
+                            // so D >= r_min > 0; fold if the truncation bound is within the tolerance
+                            const T Dx = X.x - cx, Dy = X.y - cy, Dz = X.z - cz;
+                            T rinv;
+                            if (fold_test(X.w, Dx, Dy, Dz, rg, eps_x, A.exp_rel, rinv)) {
+                                exp_add(E, X.w, Dx, Dy, Dz, rinv);
+                                acc_node = false;
+                                n_exp++;
+                            }
+                        }
+                    }
 
-                if (nn >= LF) {
-                    const int c = nn & ~(LF - 1);  // c >= LF > nn - c
-                    flush_nodes<T, TPL, FIELDS, QUAD, LF>(L, c, acc, tx, ty, tz, th);
-                    __builtin_amdgcn_wave_barrier();
-                    if (lane < nn - c) {  // reads [c, nn) and writes [0, nn - c): disjoint
-                        L.nodes[lane] = L.nodes[c + lane];
-                        if (QUAD)
-                            for (int q = 0; q < 6; q++) L.nq[6 * lane + q] = L.nq[6 * (c + lane) + q];
+                    const uint64_t bp = ptg_ballot(acc_part), bn = ptg_ballot(acc_node);
+                    if (acc_part) {
+                        const int at = np + lanes_below(bp);
+                        L.parts[at] = X;
+                        L.ph[at] = X2.x;
                     }
+                    if (acc_node) {
+                        const int at = nn + lanes_below(bn);
+                        L.nodes[at] = X;
+                        if (QUAD) {
+                            const T *q = A.quad + 8 * (int64_t)e;
+#pragma unroll
+                            for (int c = 0; c < 6; c++) L.nq[6 * at + c] = q[c];
+                        }
+                    }
+                    const int addp = (int)__popcll(bp), addn = (int)__popcll(bn);
+                    np += addp;
+                    nn += addn;
+                    n_list += addp + addn;
+                    n_part += addp;
+
+                    // push the children of opened nodes
+                    const int cnt = open ? std::min(std::max(K.y, 0), 8) : 0;
+                    int tot;
+                    const int below = small_excl_scan(cnt, tot);
+                    if (sp + tot > SCAP) {
+                        // move the bottom ks entries of the LDS stack to this wave's global region
+                        const int ks = spill_count(sp, tot);
+                        if (gsp + ks > B.gcap) {
+                            overflow = true;
+                            break;
+                        }
+                        spill_bottom(L.stack, spill + gsp, sp, ks, lane);
+                        gsp += ks;
+                        sp -= ks;
+                        ghw = std::max(ghw, gsp);
+                    }
+                    {
+                        // unrolled: eight masked LDS stores with immediate offsets, no per-lane loop
+                        int *dst = &L.stack[sp + below];
+#pragma unroll
+                        for (int c = 0; c < 8; c++)
+                            if (c < cnt) dst[c] = K.x + c;
+                    }
+                    sp += tot;
                     __builtin_amdgcn_wave_barrier();
-                    nn -= c;
+
+                    if (nn >= LF) {
+                        const int c = nn & ~(LF - 1);  // c >= LF > nn - c
+                        flush_nodes<T, TPL, FIELDS, QUAD, LF>(L, c, acc, tx, ty, tz, th);
+                        __builtin_amdgcn_wave_barrier();
+                        if (lane < nn - c) {  // reads [c, nn) and writes [0, nn - c): disjoint
+                            L.nodes[lane] = L.nodes[c + lane];
+                            if (QUAD)
+                                for (int q = 0; q < 6; q++) L.nq[6 * lane + q] = L.nq[6 * (c + lane) + q];
+                        }
+                        __builtin_amdgcn_wave_barrier();
+                        nn -= c;
+                    }
+                    if (np >= LF) {
+                        const int c = np & ~(LF - 1);
+                        flush_parts<T, TPL, FIELDS, QUAD, LF>(L, c, acc, tx, ty, tz, th);
+                        __builtin_amdgcn_wave_barrier();
+                        if (lane < np - c) {  // disjoint ranges, as above
+                            L.parts[lane] = L.parts[c + lane];
+                            L.ph[lane] = L.ph[c + lane];
+                        }
+                        __builtin_amdgcn_wave_barrier();
+                        np -= c;
+                    }
                 }
-                if (np >= LF) {
-                    const int c = np & ~(LF - 1);
-                    flush_parts<T, TPL, FIELDS, QUAD, LF>(L, c, acc, tx, ty, tz, th);
-                    __builtin_amdgcn_wave_barrier();
-                    if (lane < np - c) {  // disjoint ranges, as above
-                        L.parts[lane] = L.parts[c + lane];
-                        L.ph[lane] = L.ph[c + lane];
-                    }
-                    __builtin_amdgcn_wave_barrier();
-                    np -= c;
+                if (PASS == WHOLE || !cut) break;
+                nchild = walk_cut<TASKS>(A.ctl, B, L.stack, sp, spill, gsp, lane, self, off, child0);
+                cut = nchild > 0;
+                if (cut) break;
+                budget = 0x7fffffff;
+            }
+            if (A.counters) {
+                if (EXP) {
+#pragma unroll
+                    for (int d = 32; d >= 1; d >>= 1) n_exp += __shfl_xor(n_exp, d, 64);  // lanes fold separately
+                }
+                if (lane == 0) {
+                    atomicAdd((unsigned long long *)&A.counters[0], (unsigned long long)n_list * (unsigned long long)mt);
+                    atomicAdd((unsigned long long *)&A.counters[1], (unsigned long long)n_vis);
+                    atomicAdd((unsigned long long *)&A.counters[2], (unsigned long long)n_part * (unsigned long long)mt);
+                    if (EXP) atomicAdd((unsigned long long *)&A.counters[3], (unsigned long long)n_exp);
                 }
             }
             if (overflow) {
                 if (lane == 0) atomicOr(&A.ctl->err, 1);
-                continue;
+                if (!TASKS) continue;
+                nn = np = 0;  // a task's row is written all the same: the sums read every task's
             }
             flush_nodes<T, TPL, FIELDS, QUAD, LF>(L, nn, acc, tx, ty, tz, th);
             flush_parts<T, TPL, FIELDS, QUAD, LF>(L, np, acc, tx, ty, tz, th);
@@ -620,12 +686,42 @@ void k_walk(WalkArgs<T> A)
                 for (int j = 0; j < TPL; j++) exp_eval<T, FIELDS>(acc[j], E, tx[j] - cx, ty[j] - cy, tz[j] - cz);
             }
 
-            // ---- write G * fields in the caller's order ----
-            constexpr int W = NW<FIELDS>::W;
+            // ---- G * fields in the caller's order, or the row of a deferred group or a task ----
+            constexpr int W = NW<FIELDS>::W, WI = NW<FIELDS>::POT + 3 * NW<FIELDS>::ACC + 6 * NW<FIELDS>::TID;
+            if (TASKS || cut) {
+#pragma unroll
+                for (int j = 0; j < TPL; j++) {
+                    if (!tval[j]) continue;
+                    T *o = (T *)B.partial + ((int64_t)self * A.gs + lane + 64 * j) * WI;
+                    int c = 0;
+                    if (NW<FIELDS>::POT) agent_store(&o[c++], acc[j].phi);
+                    if (NW<FIELDS>::ACC) {
+                        agent_store(&o[c++], acc[j].gx);
+                        agent_store(&o[c++], acc[j].gy);
+                        agent_store(&o[c++], acc[j].gz);
+                    }
+                    if (NW<FIELDS>::TID) {
+                        agent_store(&o[c++], acc[j].txx);
+                        agent_store(&o[c++], acc[j].txy);
+                        agent_store(&o[c++], acc[j].txz);
+                        agent_store(&o[c++], acc[j].tyy);
+                        agent_store(&o[c++], acc[j].tyz);
+                        agent_store(&o[c++], acc[j].tzz);
+                    }
+                }
+                if (cut) {
+                    wave_stores_done();
+                    walk_publish<TASKS>(A.ctl, B, g, gsp + sp, nchild, off, child0, self, lane);
+                } else {
+                    walk_add_up<FIELDS, T>(B, self, grp, A.gs, A.perm, A.G, A.out, lane);
+                }
+                if (TASKS) closed++;
+                continue;
+            }
 #pragma unroll
             for (int j = 0; j < TPL; j++) {
                 if (!tval[j]) continue;
-                double *o = A.out + tidx[j] * W;
+                double *o = A.out + (PASS == WHOLE ? tidx[j] : A.perm[a0 + lane + 64 * j]) * W;
                 int c = 0;
                 if (NW<FIELDS>::POT) o[c++] = A.G * (double)acc[j].phi;
                 if (NW<FIELDS>::ACC) {
@@ -644,23 +740,8 @@ void k_walk(WalkArgs<T> A)
         }
     }
     if (lane == 0 && ghw > 0) atomicMax(&A.ctl->hwm, ghw);
-    if (lane == 0 && A.counters) {
-        atomicAdd((unsigned long long *)&A.counters[0], (unsigned long long)n_int);
-        atomicAdd((unsigned long long *)&A.counters[1], (unsigned long long)n_vis);
-        atomicAdd((unsigned long long *)&A.counters[2], (unsigned long long)n_part);
-    }
-    if (EXP && A.counters) {
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) n_exp += __shfl_xor(n_exp, d, 64);  // lanes fold separately
-        if (lane == 0) atomicAdd((unsigned long long *)&A.counters[3], (unsigned long long)n_exp);
-    }
 }
 
-
-__global__ void k_walk_init(WalkCtl *ctl)
-{
-    for (int i = threadIdx.x; i < (int)(sizeof(WalkCtl) / 4); i += blockDim.x) ((int32_t *)ctl)[i] = 0;
-}
 
 // ============================================================================================
 // host side
@@ -689,23 +770,25 @@ static int64_t walk_grid_blocks(int variant = -1)
     return (int64_t)num_cus() * per;
 }
 
+#define WALK_POOL (96u << 20)  // for the deferred traversals
+
 extern "C" size_t ptg_walk_workspace_bytes(int64_t nt, int group_size)
 {
     (void)nt;
     (void)group_size;
     size_t waves = (size_t)walk_grid_blocks() * WALK_WAVES;
-    return ptg_align256(sizeof(WalkCtl)) + ptg_align256(waves * GCAP * sizeof(int));
+    return walk_control_bytes() + ptg_align256(waves * GCAP * sizeof(int)) + WALK_POOL;
 }
 
 // ---- static scratch of ptg_walk_noalloc ----
 // Callers that cannot allocate (code under HIP graph capture, serving loops, harnesses that forbid
 // hipMalloc) walk with this file-scope array as the workspace: the walk control block (per-XCD group
-// counters, overflow flag) and the per-wave global spill stacks.  Every GPU that runs the library
+// counters, overflow flag), the per-wave global spill stacks and the cut traversals.  Every GPU that runs the library
 // holds its own copy until the process ends; every call on a device shares it, so calls that
 // overlap on one device (different streams) race.  Host code never passes the array's name to a
 // kernel (that is a host-side stand-in): it uses the address hipGetSymbolAddress returns, looked up
 // once per device with that device current and kept per device.
-#define NOALLOC_BYTES ((80u << 20) + 8192u)  // 4096 spill entries per wave for 5120 resident waves
+#define NOALLOC_BYTES ((80u << 20) + (1u << 20) + WALK_POOL)  // 4096 spill entries per wave for 5120 resident waves
 #define NOALLOC_MIN_GCAP 2048  // spill entries per wave the static scratch must leave
 #define NOALLOC_MAX_DEVICES 64
 static __device__ __align__(256) char scratch[NOALLOC_BYTES];
@@ -740,7 +823,7 @@ static ptg_status noalloc_scratch(void **p)
 static int noalloc_gcap(int64_t blocks)
 {
     const int64_t waves = blocks * WALK_WAVES;
-    int64_t per = (int64_t)(NOALLOC_BYTES - ptg_align256(sizeof(WalkCtl))) / (waves * (int64_t)sizeof(int));
+    int64_t per = (int64_t)(NOALLOC_BYTES - WALK_POOL - walk_control_bytes()) / (waves * (int64_t)sizeof(int));
     per = std::min<int64_t>(per, GCAP) & ~(int64_t)63;
     return (int)per;
 }
@@ -750,20 +833,45 @@ __global__ void k_walk_err_out(const WalkCtl *ctl, int32_t *err)
     if (threadIdx.x == 0) *err = ctl->err;
 }
 
+struct WalkWs {  // a walk's workspace
+    char *p;
+    size_t bytes;
+    int gcap;  // global spill entries per wave (GCAP, or what the static scratch of ptg_walk_noalloc gives)
+};
+
+
 template <typename T, int TPL, int FIELDS, bool QUAD, bool EXP, int VAR = 0>
-static ptg_status launch_t(const WalkArgs<T> &a, int64_t max_blocks, hipStream_t s)
+static ptg_status launch_t(const WalkArgs<T> &a, int64_t max_blocks, const WalkWs &ws, hipStream_t s)
 {
     static int per_cu = 0;
     if (per_cu == 0) {
         int nb = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_walk<T, TPL, FIELDS, QUAD, EXP, VAR>,
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_walk<T, TPL, FIELDS, QUAD, EXP, VAR, CUT>,
                                                          64 * WALK_WAVES, 0) != hipSuccess ||
             nb < 1)
             nb = 1;
         per_cu = std::min(nb, WalkOcc<T, TPL, VAR>::blocks_per_cu);
     }
-    int64_t blocks = std::min<int64_t>(max_blocks, (int64_t)num_cus() * per_cu);
-    k_walk<T, TPL, FIELDS, QUAD, EXP, VAR><<<(unsigned)blocks, 64 * WALK_WAVES, 0, s>>>(a);
+    const int64_t blocks = std::min<int64_t>(max_blocks, (int64_t)num_cus() * per_cu);
+    constexpr int WI = NW<FIELDS>::POT + 3 * NW<FIELDS>::ACC + 6 * NW<FIELDS>::TID;
+    WalkPool b{};
+    const double open = a.theta < T(0.7) ? 0.49 / ((double)a.theta * a.theta) : 1.0;
+    b.budget = (int)std::min(1e8, BUDGET * open * TPL);
+    b.most0 = 16;
+    b.div0 = 4;
+    b.most = 128;
+    b.div = 2;
+    ptg_status st = b.carve(ws.p, ws.bytes, blocks * WALK_WAVES, ws.gcap, (size_t)a.gs * WI * sizeof(T));
+    if (st) return st;
+    // a traversal visits a slot once, and no system has more targets than there are: where none can be
+    // cut, the kernel without (its scalar registers do not spill; 2 to 7 % of the longest traversals)
+    if (b.tcount == 0 || a.nslots <= b.budget || a.nt / a.gs < cut_groups(FIELDS)) {
+        k_walk<T, TPL, FIELDS, QUAD, EXP, VAR, WHOLE><<<(unsigned)blocks, 64 * WALK_WAVES, 0, s>>>(a, b);
+    } else {
+        k_walk<T, TPL, FIELDS, QUAD, EXP, VAR, CUT><<<(unsigned)blocks, 64 * WALK_WAVES, 0, s>>>(a, b);
+        PTG_LAUNCH_CHECK();
+        k_walk<T, TPL, FIELDS, QUAD, EXP, VAR, TASK><<<(unsigned)blocks, 64 * WALK_WAVES, 0, s>>>(a, b);
+    }
     PTG_LAUNCH_CHECK();
     return PTG_OK;
 }
@@ -771,33 +879,33 @@ static ptg_status launch_t(const WalkArgs<T> &a, int64_t max_blocks, hipStream_t
 // the monopole potential/acceleration kernels of the one-target-per-lane FP32 walk come in
 // WALK_NVARIANTS variants; every other kernel in variant 0
 template <typename T, int TPL, int FIELDS, bool EXP>
-static ptg_status launch_var(const WalkArgs<T> &a, int variant, int64_t blocks, hipStream_t s)
+static ptg_status launch_var(const WalkArgs<T> &a, int variant, int64_t blocks, const WalkWs &ws, hipStream_t s)
 {
     if constexpr (sizeof(T) == 4 && TPL == 1) {
-        if (variant == 1) return launch_t<T, TPL, FIELDS, false, EXP, 1>(a, blocks, s);
-        if (variant == 2) return launch_t<T, TPL, FIELDS, false, EXP, 2>(a, blocks, s);
+        if (variant == 1) return launch_t<T, TPL, FIELDS, false, EXP, 1>(a, blocks, ws, s);
+        if (variant == 2) return launch_t<T, TPL, FIELDS, false, EXP, 2>(a, blocks, ws, s);
     }
-    return launch_t<T, TPL, FIELDS, false, EXP, 0>(a, blocks, s);
+    return launch_t<T, TPL, FIELDS, false, EXP, 0>(a, blocks, ws, s);
 }
 
 template <typename T, int TPL>
 static ptg_status launch_fq(const WalkArgs<T> &a, int fields, bool quad, bool expand, int variant, int64_t blocks,
-                            hipStream_t s)
+                            const WalkWs &ws, hipStream_t s)
 {
     if (expand) {  // checked by the caller: monopole, potential and/or acceleration
-        if (fields == PTG_POT) return launch_var<T, TPL, PTG_POT, true>(a, variant, blocks, s);
-        if (fields == PTG_ACC) return launch_var<T, TPL, PTG_ACC, true>(a, variant, blocks, s);
-        return launch_var<T, TPL, PTG_POT | PTG_ACC, true>(a, variant, blocks, s);
+        if (fields == PTG_POT) return launch_var<T, TPL, PTG_POT, true>(a, variant, blocks, ws, s);
+        if (fields == PTG_ACC) return launch_var<T, TPL, PTG_ACC, true>(a, variant, blocks, ws, s);
+        return launch_var<T, TPL, PTG_POT | PTG_ACC, true>(a, variant, blocks, ws, s);
     }
     if (!quad) {
-        if (fields == PTG_POT) return launch_var<T, TPL, PTG_POT, false>(a, variant, blocks, s);
-        if (fields == PTG_ACC) return launch_var<T, TPL, PTG_ACC, false>(a, variant, blocks, s);
-        if (fields == (PTG_POT | PTG_ACC)) return launch_var<T, TPL, PTG_POT | PTG_ACC, false>(a, variant, blocks, s);
+        if (fields == PTG_POT) return launch_var<T, TPL, PTG_POT, false>(a, variant, blocks, ws, s);
+        if (fields == PTG_ACC) return launch_var<T, TPL, PTG_ACC, false>(a, variant, blocks, ws, s);
+        if (fields == (PTG_POT | PTG_ACC)) return launch_var<T, TPL, PTG_POT | PTG_ACC, false>(a, variant, blocks, ws, s);
     }
 #define PTG_F(F)                                                              \
     case F:                                                                   \
-        return quad ? launch_t<T, TPL, F, true, false>(a, blocks, s)          \
-                    : launch_t<T, TPL, F, false, false>(a, blocks, s);
+        return quad ? launch_t<T, TPL, F, true, false>(a, blocks, ws, s)          \
+                    : launch_t<T, TPL, F, false, false>(a, blocks, ws, s);
     switch (fields) {
         PTG_F(1) PTG_F(2) PTG_F(3) PTG_F(4) PTG_F(5) PTG_F(6) PTG_F(7)
     }
@@ -808,11 +916,11 @@ static ptg_status launch_fq(const WalkArgs<T> &a, int fields, bool quad, bool ex
 
 template <typename T>
 static ptg_status launch_walk(const WalkArgs<T> &a, int fields, bool quad, bool expand, int variant, int64_t blocks,
-                              hipStream_t s)
+                              const WalkWs &ws, hipStream_t s)
 {
-    if (a.gs <= 64) return launch_fq<T, 1>(a, fields, quad, expand, variant, blocks, s);
-    if (a.gs <= 128) return launch_fq<T, 2>(a, fields, quad, expand, variant, blocks, s);
-    return launch_fq<T, 4>(a, fields, quad, expand, variant, blocks, s);
+    if (a.gs <= 64) return launch_fq<T, 1>(a, fields, quad, expand, variant, blocks, ws, s);
+    if (a.gs <= 128) return launch_fq<T, 2>(a, fields, quad, expand, variant, blocks, ws, s);
+    return launch_fq<T, 4>(a, fields, quad, expand, variant, blocks, ws, s);
 }
 
 // ptg_walk and ptg_walk_noalloc: ws/ws_bytes is the caller's workspace, or nullptr with noalloc set
@@ -925,25 +1033,23 @@ static ptg_status walk_impl(const ptg_walk_tree *wt, const ptg_forest *forest, c
         return PTG_ERR_WORKSPACE;
     }
     WalkCtl *ctl = (WalkCtl *)ws;
-    int *spill = (int *)((char *)ws + ptg_align256(sizeof(WalkCtl)));
     const int64_t fn = forest ? forest->nsys : 0;
     const int64_t *fo = forest ? forest->offsets : nullptr;
     const double *fc = forest ? forest->cubes : nullptr;
-    k_walk_init<<<1, 64, 0, s>>>(ctl);
-    PTG_LAUNCH_CHECK();
-    ptg_status st;
+    ptg_status st = walk_clear(ctl, s);
+    if (st) return st;
     if (wt->prec == PTG_F32) {
         WalkArgs<float> a{(const V4<float> *)wt->xyzm, (const V4<float> *)wt->aux, (const int2 *)wt->kids,
                           (const float *)wt->quad, pos, soft, perm, targets_sorted != 0, wt->nslots, nt, ptg_cdiv(nt, group_size), group_offsets, group_count,
                           group_size, (float)theta, (float)(1.0 / theta), crit, (float)eps, (float)eps_exp,
                           expand ? criterion->expansion_rel : 0.0f, eps_scale, G, wt->origin[0], wt->origin[1],
                           wt->origin[2],
-                          fn, fo, fc, out, counters, ctl, spill, gcap};
+                          fn, fo, fc, out, counters, ctl};
         if (exact) {
             ptg_set_error("ptg_walk: the exact branch set is evaluated in FP64; use prec=PTG_F64");
             return PTG_ERR_ARG;
         }
-        st = launch_walk<float>(a, fields, quadrupole != 0, expand, variant, blocks, s);
+        st = launch_walk<float>(a, fields, quadrupole != 0, expand, variant, blocks, WalkWs{(char *)ws, ws_bytes, gcap}, s);
     } else if (wt->prec == PTG_F64) {
         Walk64Args a{(const V4<double> *)wt->xyzm, (const V4<double> *)wt->aux, (const int2 *)wt->kids,
                      (const double *)wt->quad, pos, soft, perm, targets_sorted != 0, wt->nslots, nt,
@@ -1016,6 +1122,10 @@ extern "C" ptg_status ptg_walk_check(void *ws, void *stream)
     if (err & 4) {
         ptg_set_error("ptg_walk_subtree: the start element's slot is outside the walk tree (nothing was walked)");
         return PTG_ERR_ARG;
+    }
+    if (err & 8) {
+        ptg_set_error("ptg_walk: waves of the task pass gave up waiting for deferred traversals");
+        return PTG_ERR_OVERFLOW;
     }
     if (err) {
         ptg_set_error("ptg_walk: a traversal stack exceeded its spill capacity");

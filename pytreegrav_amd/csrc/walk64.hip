@@ -8,58 +8,26 @@
 // max(h_s, h_t) from them) and take one reciprocal square root; particles outside every softening
 // radius of the group join them (monopole walks).
 //
-// The reference's groups are runs of the Morton order.  A run that crosses a high-level cell boundary
-// in a sparse region has a box as wide as the domain, opens nearly every node, and one wave walking it
-// alone sets the kernel's time (1.48e6 of the 2.9e8 visits of a 1e6-particle Plummer sphere are one
-// group's).  A task past its budget of visits is therefore deferred: it saves its stack, cut into
-// interleaved shares, as tasks of the next round, and k_walk64_sum adds the shares' partial sums in
-// their order.  The cut depends only on the group's own traversal, so results do not depend on
-// scheduling (unless the task tables fill up: then the rest is walked in place, the same terms summed
-// in another order).
+// The reference's groups are runs of the Morton order; those that cross a high-level cell boundary in a
+// sparse region open nearly every node (1.48e6 of the 2.9e8 visits of a 1e6-particle Plummer sphere are
+// one group's) and are deferred (walk_shared.hpp).
 //
 // Bound: instruction issue, about 60 % of it the traversal (250 instructions per 64-element step).
 // Whole calls, against one wave per group evaluating every entry for 8 of its 64 lanes with IEEE
-// square roots and divisions: 1e6-particle Plummer sphere 333 -> 4.8 ms, uniform cube of 1e5 6.0 -> 0.83
-// ms, tidal tensors with quadrupoles of 6e4 23.3 -> 1.3 ms.  Angle-binned columns of 2e5 particles
-// against their own walk (two waves per SIMD, six selected adds and a division a pair): 4.9 -> 2.25 ms.
+// square roots and divisions: 1e6-particle Plummer sphere 333 -> 4.4 ms, uniform cube of 1e5 6.0 -> 0.79
+// ms, tidal tensors with quadrupoles of 6e4 23.3 -> 1.24 ms.  Angle-binned columns of 2e5 particles
+// against their own walk (two waves per SIMD, six selected adds and a division a pair): 4.9 -> 2.15 ms.
 
 #include "walk_shared.hpp"
 
 #define LIST 32           // a list is evaluated in multiples of LIST entries once it holds LIST
 #define ICAP (LIST + 64)  // LIST - 1 entries + one step's 64
-#define BUDGET 3072       // visits after which a task is deferred (not in the last round), at least
-#define SHARES0 64        // tasks a deferred group is cut into, at most (of DIV0 stack entries or more)
-#define DIV0 16
-#define SHARES 128        // tasks a deferred task is cut into, at most (of DIV stack entries or more)
-#define DIV 4
-#define SHARE_BYTES 262144  // of partial sums, past 16 tasks: large groups are cut into fewer
+#define BUDGET 3072  // visits after which a traversal is cut, at least
 #define MAX_BLOCKS_PER_CU 4
-#define MAX_TASKS 196608  // of round 1; a quarter of it in each later round, an eighth deferred groups
-
-struct Walk64Task {
-    int32_t group;
-    int32_t child0, nchild;      // its shares in the task tables (deferred tasks; else nchild 0)
-    int32_t off, stride, count;  // saved stack entries pool[off + i * stride], i < count
-};
-
-struct Walk64Pool {
-    int *spill;  // per-wave global stacks, gcap entries each
-    int gcap;
-    int *entries;  // saved stacks
-    int ecap;
-    Walk64Task *tasks;  // the deferred groups, then the tasks of rounds 1, 2, ..
-    double *partial;    // one row of gs * WI sums per entry of tasks
-    int budget, shares0, shares;
-    // this launch: its round (level of the sums), its table (cap entries of tasks from base on) and the
-    // next one's (next_cap 0: nothing is deferred).  Scalars: arrays indexed by the round would put the
-    // arguments into scratch memory.
-    int round, base, cap, next_base, next_cap;
-};
 
 // FIELDS of the angle-binned column density (treewalk.py:976-1028, :1197-1276): six sums per target, kept
 // in LDS, since which of them a pair adds to differs from lane to lane (one LDS add instead of six
 // selected ones)
-#define BINS 8
 #define SKY_BIN (4.0 * 3.14159265358979323846 / 6.0)  // solid angle of a bin
 
 template <int FIELDS, bool QUAD> struct Lds64 {
@@ -252,59 +220,15 @@ template <int FIELDS, typename F> __device__ __forceinline__ void each_sum(Acc<d
         f(a.tzz);
     }
 }
-template <int FIELDS> struct Sums {
-    static constexpr int WI = FIELDS == BINS ? 6 : NW<FIELDS>::POT + 3 * NW<FIELDS>::ACC + 6 * NW<FIELDS>::TID;
-    static constexpr int WO = FIELDS == BINS ? 6 : NW<FIELDS>::W;  // output row
-};
-
-// the output row o[] entries that sum c of a target fills (two for an off-diagonal tidal component)
-template <int FIELDS> __device__ __forceinline__ void store_sum(double *o, int c, double v)
-{
-    constexpr int PA = FIELDS == BINS ? 6 : NW<FIELDS>::POT + 3 * NW<FIELDS>::ACC;
-    if (!NW<FIELDS>::TID || c < PA) {
-        o[c] = v;
-        return;
-    }
-    const int k = c - PA;
-    const int i = k < 3 ? 0 : k < 5 ? 1 : 2, j = k < 3 ? k : k < 5 ? k - 2 : 2;
-    o[PA + 3 * i + j] = v;
-    o[PA + 3 * j + i] = v;
-}
-
-struct Group64 {
-    int64_t a0;  // first target
-    int mt;      // targets
-    int over;    // targets of a supplied group past gs (not evaluated)
-};
-
-__device__ __forceinline__ Group64 group_of(const Walk64Args &A, int64_t g)
-{
-    const int64_t a0 = A.goff ? (int64_t)A.goff[g] : g * A.gs;
-    const int64_t e0 = A.goff ? (int64_t)A.goff[g + 1] : A.nt;
-    const int64_t b0 = e0 < a0 + A.gs ? e0 : a0 + A.gs;
-    return Group64{a0, (int)(b0 - a0), A.goff && e0 > b0};
-}
-
-// n consecutive entries of a table of cap counted by *counter: the first one's index (one lane calls).
-// Past cap - n they do not fit: cap if nothing was taken, else the entries below cap are the caller's
-// all the same.  The counter is added to once and never taken back: when thousands of waves reach
-// their budgets together, compare-and-swap loops on it took 27 ms.
-__device__ __forceinline__ int take(int32_t *counter, int n, int cap)
-{
-    const int seen = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return seen > cap - n ? cap : atomicAdd(counter, n);
-}
-
 // waves per SIMD the registers are capped for: four where the LDS lets four blocks onto a CU
 template <int TPL, int FIELDS, bool QUAD> struct Occ64 {
     static constexpr int waves = FIELDS == BINS ? 3 : TPL == 1 && !QUAD && !NW<FIELDS>::TID ? 4 : 1;
 };
 
-template <int TPL, int FIELDS, bool QUAD>
+template <int TPL, int FIELDS, bool QUAD, bool TASKS>
 __global__ __launch_bounds__(64 * WALK_WAVES) __attribute__((amdgpu_waves_per_eu(Occ64<TPL, FIELDS, QUAD>::waves)))
-void k_walk64(const Walk64Args A, const Walk64Pool B)
+void k_walk64(const Walk64Args A, const WalkPool B)
 {
-    const int round = B.round;
     constexpr int WI = Sums<FIELDS>::WI;
     __shared__ Lds64<FIELDS, QUAD> lds[WALK_WAVES];
     const int wave = threadIdx.x >> 6, lane = ptg_lane();
@@ -314,35 +238,36 @@ void k_walk64(const Walk64Args A, const Walk64Pool B)
     int64_t n_int = 0, n_vis = 0, n_part = 0;
     int ghw = 0;
     const int64_t ngroups = A.goff ? (int64_t)__builtin_amdgcn_readfirstlane(*A.gcount) : A.ngroups;
-    const int ntask = round ? std::min(__builtin_amdgcn_readfirstlane(A.ctl->ntask[round]), B.cap) : 0;
-    if (round && ntask == 0) return;
+    int closed = 0;
+    if (TASKS && agent_load(&A.ctl->open) == 0) return;  // nothing was deferred, or all of it is done
     // targets per slice, a power of two
     int P = 64;
     if (TPL == 1)
         while (P > 1 && P / 2 >= A.gs) P /= 2;
     const int tl = lane & (P - 1), sl = lane / P, slices = 64 / P;
 
-    // groups (round 0) or tasks from per-XCD counters, as the FP32 walk takes its groups
-    const int64_t nwork = round ? ntask : ngroups;
-    int32_t *ctr = round ? A.ctl->tctr + (round - 1) * NXCD * CTR_STRIDE : A.ctl->ctr;
-    for (int attempt = 0; attempt < NXCD; attempt++) {
+    // groups from per-XCD counters, as the FP32 walk takes them; or tasks by ticket
+    for (int attempt = 0; attempt < (TASKS ? 1 : NXCD); attempt++) {
         const int x = (xcd + attempt) % NXCD;
-        const int64_t w_lo = nwork * x / NXCD, w_hi = nwork * (x + 1) / NXCD;
+        const int64_t w_lo = ngroups * x / NXCD, w_hi = ngroups * (x + 1) / NXCD;
         for (;;) {
-            int wi = 0;
-            if (lane == 0) wi = atomicAdd(&ctr[x * CTR_STRIDE], 1);
-            const int64_t work = w_lo + __builtin_amdgcn_readfirstlane(wi);
-            if (work >= w_hi) break;
-            int64_t g = work;
-            int t_off = 0, t_stride = 0, t_count = 0;
-            if (round) {
-                const Walk64Task *T = &B.tasks[B.base + work];
-                g = __builtin_amdgcn_readfirstlane(T->group);
-                t_off = __builtin_amdgcn_readfirstlane(T->off);
-                t_stride = __builtin_amdgcn_readfirstlane(T->stride);
-                t_count = __builtin_amdgcn_readfirstlane(T->count);
+            int self = -1, t_off = 0, t_stride = 0, t_count = 0;
+            int64_t g;
+            if (TASKS) {
+                self = walk_ticket(A.ctl, B, lane, closed);
+                if (self < 0) break;
+                const WalkTask *T = &B.tasks[self];
+                g = __builtin_amdgcn_readfirstlane(agent_load(&T->group));
+                t_off = __builtin_amdgcn_readfirstlane(agent_load(&T->off));
+                t_stride = __builtin_amdgcn_readfirstlane(agent_load(&T->stride));
+                t_count = __builtin_amdgcn_readfirstlane(agent_load(&T->count));
+            } else {
+                int wi = 0;
+                if (lane == 0) wi = atomicAdd(&A.ctl->ctr[x * CTR_STRIDE], 1);
+                g = w_lo + __builtin_amdgcn_readfirstlane(wi);
+                if (g >= w_hi) break;
             }
-            const Group64 grp = group_of(A, g);
+            const WalkSpan grp = walk_span(A.goff, A.gs, A.nt, g);
             const int64_t a0 = grp.a0;
             const int mt = grp.mt;
             if (grp.over && lane == 0) atomicOr(&A.ctl->err, 2);  // a supplied group larger than group_size
@@ -402,9 +327,9 @@ void k_walk64(const Walk64Args A, const Walk64Pool B)
 
             int sp = 1, gsp = 0, nn = 0, np = 0, visits = 0;
             bool overflow = false;
-            if (round) {
+            if (TASKS) {
                 sp = t_count;  // <= SCAP: deeper stacks are not deferred
-                for (int q = lane; q < sp; q += 64) L.stack[q] = B.entries[t_off + (int64_t)q * t_stride];
+                for (int q = lane; q < sp; q += 64) L.stack[q] = agent_load(&B.entries[t_off + (int64_t)q * t_stride]);
             } else {
                 // the root of system s occupies walk slot s; a subtree walk starts at its element's slot
                 // instead (wave-uniform; an out-of-range slot is reported, and dropped when popped like
@@ -418,177 +343,149 @@ void k_walk64(const Walk64Args A, const Walk64Pool B)
             }
             __builtin_amdgcn_wave_barrier();
             // The more groups share the device, the longer one may run alone, and the fewer should pay for
-            // being cut: budgets of 3072 against 8192 take 0.83 / 0.95 ms (walk and build, uniform 1e5), 3
-            // against 2 times 4096 6.8 / 8.0 (clumpy 6e5).  Counted per system, so that a system's cuts
+            // being cut: budgets of 3072 against 8192 take 0.79 / 0.95 ms (walk and build, uniform 1e5), 4
+            // against 3 times 3072 6.8 / 8.3 ms (clumpy 6e5).  Counted per system, so that a system's cuts
             // are those it has alone.
             const int64_t sg = (A.nsys > 0 ? A.soff[root + 1] - A.soff[root] : A.nt) / A.gs;
-            int budget = B.budget * (round || sg <= 16384 ? 1 : sg <= 65536 ? 2 : sg <= 262144 ? 3 : 16);
-            if (B.next_cap == 0) budget = 0x7fffffff;
-            int child0 = -1, nchild = 0, slot = round ? B.base + (int)work : -1;
+            int budget = B.budget * (TASKS || sg <= 16384 ? 1 : sg <= 65536 ? 2 : sg <= 262144 ? 4 : 16);
+            if (B.tcount == 0) budget = 0x7fffffff;
+            bool cut = false;
+            int nchild = 0, off = 0, child0 = 0;
 
-            for (;;) {
-                if (sp == 0) {
-                    if (gsp == 0) break;
-                    const int k = std::min(gsp, SPILL);
-                    for (int q = lane; q < k; q += 64) L.stack[q] = spill[gsp - k + q];
-                    __builtin_amdgcn_wave_barrier();
-                    gsp -= k;
-                    sp = k;
-                }
-                if (visits >= budget) {
-                    // save the stack as interleaved shares of the next round; out of room: go on here
-                    const int cnt = gsp + sp;
-                    const int most = round ? B.shares : B.shares0, part = round ? cnt / DIV : cnt / DIV0;
-                    nchild = part > most ? most : part < 1 ? 1 : part;
-                    const int cap = B.next_cap;
-                    int off = -1, at = cap;
-                    if (lane == 0 && cnt <= nchild * SCAP) {
-                        if (round == 0) slot = take(&A.ctl->ntask[0], 1, B.cap);  // table 0 starts at 0
-                        if (round || slot < B.cap) {
-                            at = take(&A.ctl->ntask[round + 1], nchild, cap);
-                            if (at <= cap - nchild) off = take(&A.ctl->npool, cnt, B.ecap);
-                            if (off > B.ecap - cnt) off = -1;
-                            if (off >= 0) child0 = B.next_base + at;
-                            // a record without shares, should there be no room
-                            B.tasks[slot].group = (int32_t)g;
-                            B.tasks[slot].child0 = child0;
-                            B.tasks[slot].nchild = off >= 0 ? nchild : 0;
-                        }
+            for (;;) {  // once more only where a deferred traversal finds no room
+                for (;;) {
+                    if (sp == 0) {
+                        if (gsp == 0) break;
+                        const int k = std::min(gsp, SPILL);
+                        for (int q = lane; q < k; q += 64) L.stack[q] = spill[gsp - k + q];
+                        __builtin_amdgcn_wave_barrier();
+                        gsp -= k;
+                        sp = k;
                     }
-                    slot = __builtin_amdgcn_readfirstlane(slot);
-                    at = __builtin_amdgcn_readfirstlane(at);
-                    off = __builtin_amdgcn_readfirstlane(off);
-                    child0 = __builtin_amdgcn_readfirstlane(child0);
-                    // the entries taken below cap are filled in any case: the next round reads all of them
-                    for (int q = lane; q < nchild && at + q < cap; q += 64) {
-                        Walk64Task &T = B.tasks[B.next_base + at + q];
-                        T.group = (int32_t)g;
-                        T.nchild = 0;
-                        T.off = off + q;
-                        T.stride = nchild;
-                        T.count = off >= 0 ? (cnt - q + nchild - 1) / nchild : 0;
-                    }
-                    if (child0 >= 0) {
-                        for (int q = lane; q < gsp; q += 64) B.entries[off + q] = spill[q];
-                        for (int q = lane; q < sp; q += 64) B.entries[off + gsp + q] = L.stack[q];
+                    if (visits >= budget) {
+                        cut = true;
                         break;
                     }
-                    budget = 0x7fffffff;
-                }
-                const int k = std::min(sp, 64);
-                const int base = sp - k;
-                int e = lane < k ? L.stack[base + lane] : 0;
-                const bool ve = lane < k && e >= 0 && e < A.nslots;  // a corrupt link is dropped, not followed
-                if (!ve) e = 0;
-                __builtin_amdgcn_wave_barrier();
-                sp = base;
-                visits += k;
-                const V4<double> X = A.xyzm[e];
-                const V4<double> X2 = A.aux[e];
-                const int2 K = A.kids[e];
-                const bool ispart = K.y == 0;
-                const double dxm = box_gap(X.x, bmin0, bmax0), dym = box_gap(X.y, bmin1, bmax1);
-                const double dzm = box_gap(X.z, bmin2, bmax2);
-                const double r2m = dxm * dxm + dym * dym + dzm * dzm;
-                const double hh = X2.x > hmax ? X2.x : hmax;
-                // the reference's test r_min > max(size/theta + delta, h + 0.6 size + delta): decided on
-                // the squares unless they agree to 1e-14 (or could underflow), then as written
-                const double c2 = hh + X2.y * 0.6 + X2.z;
-                const double cq = std::max(X2.y * A.inv_theta + X2.z, c2), cc = cq * cq;
-                bool acc_node = ve & !ispart & (r2m > cc);
-                const bool close = ve & !ispart & !(fabs(r2m - cc) > fma(1e-14, cc, 1e-290));
-                if (ptg_ballot(close)) {
-                    const double r_min = sqrt(r2m), c1 = X2.y / A.theta + X2.z;
-                    if (close) acc_node = r_min > (c1 > c2 ? c1 : c2);
-                }
-                // a particle farther from the box than every softening radius needs neither the softening
-                // nor the self test; with quadrupoles it stays a particle (no quadrupole terms)
-                const bool far_part = !QUAD & ve & ispart & (r2m > hh * hh);
-                const bool acc_part = ve & ispart & !far_part;
-                const bool open = ve & !ispart & !acc_node;
-                acc_node |= far_part;
-                const uint64_t bp = ptg_ballot(acc_part), bn = ptg_ballot(acc_node);
-                if (acc_part) {
-                    const int at = np + lanes_below(bp);
-                    L.parts[at] = X;
-                    L.ph[at] = X2.x;
-                }
-                if (acc_node) {
-                    const int at = nn + lanes_below(bn);
-                    L.nodes[at] = X;
-                    if (QUAD) {
-                        const double *q = A.quad + 8 * (int64_t)e;
-#pragma unroll
-                        for (int c = 0; c < 6; c++) L.nq[6 * at + c] = q[c];
+                    const int k = std::min(sp, 64);
+                    const int base = sp - k;
+                    int e = lane < k ? L.stack[base + lane] : 0;
+                    const bool ve = lane < k && e >= 0 && e < A.nslots;  // a corrupt link is dropped, not followed
+                    if (!ve) e = 0;
+                    __builtin_amdgcn_wave_barrier();
+                    sp = base;
+                    visits += k;
+                    const V4<double> X = A.xyzm[e];
+                    const V4<double> X2 = A.aux[e];
+                    const int2 K = A.kids[e];
+                    const bool ispart = K.y == 0;
+                    const double dxm = box_gap(X.x, bmin0, bmax0), dym = box_gap(X.y, bmin1, bmax1);
+                    const double dzm = box_gap(X.z, bmin2, bmax2);
+                    const double r2m = dxm * dxm + dym * dym + dzm * dzm;
+                    const double hh = X2.x > hmax ? X2.x : hmax;
+                    // the reference's test r_min > max(size/theta + delta, h + 0.6 size + delta): decided on
+                    // the squares unless they agree to 1e-14 (or could underflow), then as written
+                    const double c2 = hh + X2.y * 0.6 + X2.z;
+                    const double cq = std::max(X2.y * A.inv_theta + X2.z, c2), cc = cq * cq;
+                    bool acc_node = ve & !ispart & (r2m > cc);
+                    const bool close = ve & !ispart & !(fabs(r2m - cc) > fma(1e-14, cc, 1e-290));
+                    if (ptg_ballot(close)) {
+                        const double r_min = sqrt(r2m), c1 = X2.y / A.theta + X2.z;
+                        if (close) acc_node = r_min > (c1 > c2 ? c1 : c2);
                     }
-                }
-                np += (int)__popcll(bp);
-                nn += (int)__popcll(bn);
-                if (A.counters) {
-                    n_int += (int64_t)(__popcll(bp) + __popcll(bn)) * mt;
-                    n_part += (int64_t)(__popcll(bp) + __popcll(ptg_ballot(far_part))) * mt;
-                }
-
-                const int cnt = open ? std::min(std::max(K.y, 0), 8) : 0;
-                int tot;
-                const int below = small_excl_scan(cnt, tot);
-                if (sp + tot > SCAP) {
-                    const int ks = spill_count(sp, tot);
-                    if (gsp + ks > B.gcap) {
-                        overflow = true;
-                        break;
+                    // a particle farther from the box than every softening radius needs neither the softening
+                    // nor the self test; with quadrupoles it stays a particle (no quadrupole terms)
+                    const bool far_part = !QUAD & ve & ispart & (r2m > hh * hh);
+                    const bool acc_part = ve & ispart & !far_part;
+                    const bool open = ve & !ispart & !acc_node;
+                    acc_node |= far_part;
+                    const uint64_t bp = ptg_ballot(acc_part), bn = ptg_ballot(acc_node);
+                    if (acc_part) {
+                        const int at = np + lanes_below(bp);
+                        L.parts[at] = X;
+                        L.ph[at] = X2.x;
                     }
-                    spill_bottom(L.stack, spill + gsp, sp, ks, lane);
-                    gsp += ks;
-                    sp -= ks;
-                    ghw = std::max(ghw, gsp);
-                }
-                {
-                    int *dst = &L.stack[sp + below];
+                    if (acc_node) {
+                        const int at = nn + lanes_below(bn);
+                        L.nodes[at] = X;
+                        if (QUAD) {
+                            const double *q = A.quad + 8 * (int64_t)e;
 #pragma unroll
-                    for (int c = 0; c < 8; c++)
-                        if (c < cnt) dst[c] = K.x + c;
-                }
-                sp += tot;
-                __builtin_amdgcn_wave_barrier();
-
-                if (nn >= LIST) {
-                    const int c = nn & ~(LIST - 1);  // c >= LIST > nn - c
-                    for (int q = sl; q < c; q += slices) {
-                        const V4<double> s = L.nodes[q];
-#pragma unroll
-                        for (int j = 0; j < TPL; j++) {
-                            if constexpr (FIELDS == BINS) sky.node(s, tx[j], ty[j], tz[j]);
-                            else pair_node<FIELDS, QUAD>(acc[j], s, &L.nq[QUAD ? 6 * q : 0], tx[j], ty[j], tz[j]);
+                            for (int c = 0; c < 6; c++) L.nq[6 * at + c] = q[c];
                         }
                     }
-                    __builtin_amdgcn_wave_barrier();
-                    if (lane < nn - c) {  // reads [c, nn) and writes [0, nn - c): disjoint
-                        L.nodes[lane] = L.nodes[c + lane];
-                        if (QUAD)
-                            for (int q = 0; q < 6; q++) L.nq[6 * lane + q] = L.nq[6 * (c + lane) + q];
+                    np += (int)__popcll(bp);
+                    nn += (int)__popcll(bn);
+                    if (A.counters) {
+                        n_int += (int64_t)(__popcll(bp) + __popcll(bn)) * mt;
+                        n_part += (int64_t)(__popcll(bp) + __popcll(ptg_ballot(far_part))) * mt;
                     }
-                    __builtin_amdgcn_wave_barrier();
-                    nn -= c;
-                }
-                if (np >= LIST) {
-                    const int c = np & ~(LIST - 1);
-                    for (int q = sl; q < c; q += slices) {
-                        const V4<double> s = L.parts[q];
-#pragma unroll
-                        for (int j = 0; j < TPL; j++) {
-                            if constexpr (FIELDS == BINS) sky.part(s, L.ph[q], tx[j], ty[j], tz[j]);
-                            else pair_part<FIELDS>(acc[j], s, L.ph[q], tx[j], ty[j], tz[j], th[j]);
+
+                    const int cnt = open ? std::min(std::max(K.y, 0), 8) : 0;
+                    int tot;
+                    const int below = small_excl_scan(cnt, tot);
+                    if (sp + tot > SCAP) {
+                        const int ks = spill_count(sp, tot);
+                        if (gsp + ks > B.gcap) {
+                            overflow = true;
+                            break;
                         }
+                        spill_bottom(L.stack, spill + gsp, sp, ks, lane);
+                        gsp += ks;
+                        sp -= ks;
+                        ghw = std::max(ghw, gsp);
                     }
-                    __builtin_amdgcn_wave_barrier();
-                    if (lane < np - c) {  // disjoint ranges, as above
-                        L.parts[lane] = L.parts[c + lane];
-                        L.ph[lane] = L.ph[c + lane];
+                    {
+                        int *dst = &L.stack[sp + below];
+#pragma unroll
+                        for (int c = 0; c < 8; c++)
+                            if (c < cnt) dst[c] = K.x + c;
                     }
+                    sp += tot;
                     __builtin_amdgcn_wave_barrier();
-                    np -= c;
+
+                    if (nn >= LIST) {
+                        const int c = nn & ~(LIST - 1);  // c >= LIST > nn - c
+                        for (int q = sl; q < c; q += slices) {
+                            const V4<double> s = L.nodes[q];
+#pragma unroll
+                            for (int j = 0; j < TPL; j++) {
+                                if constexpr (FIELDS == BINS) sky.node(s, tx[j], ty[j], tz[j]);
+                                else pair_node<FIELDS, QUAD>(acc[j], s, &L.nq[QUAD ? 6 * q : 0], tx[j], ty[j], tz[j]);
+                            }
+                        }
+                        __builtin_amdgcn_wave_barrier();
+                        if (lane < nn - c) {  // reads [c, nn) and writes [0, nn - c): disjoint
+                            L.nodes[lane] = L.nodes[c + lane];
+                            if (QUAD)
+                                for (int q = 0; q < 6; q++) L.nq[6 * lane + q] = L.nq[6 * (c + lane) + q];
+                        }
+                        __builtin_amdgcn_wave_barrier();
+                        nn -= c;
+                    }
+                    if (np >= LIST) {
+                        const int c = np & ~(LIST - 1);
+                        for (int q = sl; q < c; q += slices) {
+                            const V4<double> s = L.parts[q];
+#pragma unroll
+                            for (int j = 0; j < TPL; j++) {
+                                if constexpr (FIELDS == BINS) sky.part(s, L.ph[q], tx[j], ty[j], tz[j]);
+                                else pair_part<FIELDS>(acc[j], s, L.ph[q], tx[j], ty[j], tz[j], th[j]);
+                            }
+                        }
+                        __builtin_amdgcn_wave_barrier();
+                        if (lane < np - c) {  // disjoint ranges, as above
+                            L.parts[lane] = L.parts[c + lane];
+                            L.ph[lane] = L.ph[c + lane];
+                        }
+                        __builtin_amdgcn_wave_barrier();
+                        np -= c;
+                    }
                 }
+                if (!cut) break;
+                nchild = walk_cut<TASKS>(A.ctl, B, L.stack, sp, spill, gsp, lane, self, off, child0);
+                cut = nchild > 0;
+                if (cut) break;
+                budget = 0x7fffffff;
             }
             n_vis += visits;
             if (overflow) {
@@ -627,7 +524,7 @@ void k_walk64(const Walk64Args A, const Walk64Pool B)
             }
 
             // ---- G * fields in the caller's order, or the task's row of partial sums ----
-            const bool whole = round == 0 && child0 < 0;
+            const bool whole = !TASKS && !cut;
 #pragma unroll
             for (int j = 0; j < TPL; j++) {
                 if (!tval[j] || sl != 0) continue;
@@ -640,14 +537,21 @@ void k_walk64(const Walk64Args A, const Walk64Pool B)
                         for (int q = 0; q < 6; q++) o[q] = A.G * bin[q];
                     }
                 } else {
-                    double *o = B.partial + ((int64_t)slot * A.gs + tl + 64 * j) * WI;
-                    each_sum<FIELDS>(acc[j], [&](double &v) { o[c++] = v; });
+                    double *o = (double *)B.partial + ((int64_t)self * A.gs + tl + 64 * j) * WI;
+                    each_sum<FIELDS>(acc[j], [&](double &v) { agent_store(&o[c++], v); });
                     if constexpr (FIELDS == BINS) {
 #pragma unroll
-                        for (int q = 0; q < 6; q++) o[q] = bin[q];
+                        for (int q = 0; q < 6; q++) agent_store(&o[q], bin[q]);
                     }
                 }
             }
+            if (cut) {
+                wave_stores_done();
+                walk_publish<TASKS>(A.ctl, B, g, gsp + sp, nchild, off, child0, self, lane);
+            } else if (TASKS) {
+                walk_add_up<FIELDS, double>(B, self, grp, A.gs, A.perm, A.G, A.out, lane);
+            }
+            if (TASKS) closed++;
         }
     }
     if (lane == 0 && ghw > 0) atomicMax(&A.ctl->hwm, ghw);
@@ -655,35 +559,6 @@ void k_walk64(const Walk64Args A, const Walk64Pool B)
         atomicAdd((unsigned long long *)&A.counters[0], (unsigned long long)n_int);
         atomicAdd((unsigned long long *)&A.counters[1], (unsigned long long)n_vis);
         if (FIELDS != BINS) atomicAdd((unsigned long long *)&A.counters[2], (unsigned long long)n_part);
-    }
-}
-
-// Adds to the row of each deferred task of round B.round the rows of its shares, in order; round 0:
-// the deferred groups, whose totals are the results.  One wave per deferred task, deepest level first.
-template <int FIELDS>
-__global__ __launch_bounds__(256) void k_walk64_sum(const Walk64Args A, const Walk64Pool B)
-{
-    constexpr int WI = Sums<FIELDS>::WI;
-    const int nt = std::min(__builtin_amdgcn_readfirstlane(A.ctl->ntask[B.round]), B.cap);
-    const int64_t rs = (int64_t)A.gs * WI;
-    for (int t = blockIdx.x * 4 + (threadIdx.x >> 6); t < nt; t += gridDim.x * 4) {
-        const Walk64Task T = B.tasks[B.base + t];
-        if (T.nchild == 0) continue;
-        const Group64 grp = group_of(A, T.group);
-        const int nv = grp.mt * WI;
-        double *row = B.partial + (int64_t)(B.base + t) * rs;
-        const double *kids = B.partial + T.child0 * rs;
-        for (int v = ptg_lane(); v < nv; v += 64) {
-            double s = row[v];
-#pragma unroll 8
-            for (int k = 0; k < T.nchild; k++) s += kids[k * rs + v];
-            if (B.round) {
-                row[v] = s;
-            } else {
-                const int64_t t = grp.a0 + v / WI, o = A.perm ? A.perm[t] : t;
-                store_sum<FIELDS>(A.out + o * Sums<FIELDS>::WO, v % WI, A.G * s);
-            }
-        }
     }
 }
 
@@ -696,66 +571,31 @@ static ptg_status launch(const Walk64Args &a, int cus, int gcap, char *ws, size_
     static int per_cu = 0;
     if (per_cu == 0) {
         int nb = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_walk64<TPL, FIELDS, QUAD>, 64 * WALK_WAVES, 0) !=
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_walk64<TPL, FIELDS, QUAD, false>, 64 * WALK_WAVES, 0) !=
                 hipSuccess ||
             nb < 1)
             nb = 1;
         per_cu = std::min(nb, MAX_BLOCKS_PER_CU);
     }
-    // the workspace after the control block: the spill stacks of the resident waves, then what deferral
-    // needs; none is left over only on a device with more waves than the workspace was sized for
-    Walk64Pool b{};
-    size_t at = ptg_align256(sizeof(WalkCtl));
-    auto carve = [&](size_t bytes) {
-        char *p = ws + at;
-        at += ptg_align256(bytes);
-        return p;
-    };
-    b.gcap = gcap;
-    b.spill = (int *)carve((size_t)cus * per_cu * WALK_WAVES * gcap * sizeof(int));
-    if (at > ws_bytes) {
-        ptg_set_error("FP64 walk: workspace too small (%zu < %zu)", ws_bytes, at);
-        return PTG_ERR_WORKSPACE;
-    }
-    const size_t left = ws_bytes - at;
-    const size_t pool = std::min<size_t>(left / 8 * 3, 48u << 20);
+    // an ordinary group's traversal stays well inside the budget: it grows as 1 / theta^2 and with the
+    // group; large groups (large rows of sums) are cut into fewer shares
     const size_t row = (size_t)a.gs * Sums<FIELDS>::WI * sizeof(double);
-    // an ordinary group's traversal stays well inside the budget: it grows as 1 / theta^2 and with the group
     const double open = a.theta < 0.7 ? 0.49 / (a.theta * a.theta) : 1.0;
+    const int share = (int)std::max<size_t>(16, 262144 / row);
+    WalkPool b{};
     b.budget = (int)std::min(1e8, BUDGET * open * (a.gs <= 16 ? 1 : a.gs <= 64 ? 2 : 4));
-    b.shares0 = (int)std::min<size_t>(SHARES0, std::max<size_t>(16, SHARE_BYTES / row));
-    b.shares = (int)std::min<size_t>(SHARES, std::max<size_t>(16, SHARE_BYTES / row));
-    const size_t nrows = left > pool + 1024 ? (left - pool - 1024) / (row + sizeof(Walk64Task)) : 0;
-    const int most = (int)std::min<size_t>(MAX_TASKS, nrows / 2);
-    int base[WALK_ROUNDS + 1] = {}, cap[WALK_ROUNDS + 1] = {}, n = 0;
-    if (most >= SHARES) {
-        b.ecap = (int)(pool / sizeof(int));
-        b.entries = (int *)carve(pool);
-        for (int k = 0; k < WALK_ROUNDS; k++) {  // nrows / 2 * (1/8 + 1 + 3 * 1/4) rows at most
-            base[k] = n;
-            n += cap[k] = k == 0 ? most / 8 : k == 1 ? most : most / 4;
-        }
-        b.tasks = (Walk64Task *)carve(n * sizeof(Walk64Task));
-        b.partial = (double *)carve(n * row);
-    }
+    b.most0 = std::min(64, share);
+    b.div0 = 4;
+    b.most = std::min(128, share);
+    b.div = 2;
     const int64_t blocks = (int64_t)cus * per_cu;
-    // a task of round r is what r budgets left of one traversal, which visits a slot once
-    const int rounds = n ? (int)std::min<int64_t>(WALK_ROUNDS, 1 + a.nslots / b.budget) : 1;
-    for (int round = 0; round < rounds; round++) {
-        const int64_t nb = round || a.goff ? blocks : std::min(blocks, ptg_cdiv(a.ngroups, WALK_WAVES));
-        b.round = round;
-        b.base = base[round];
-        b.cap = cap[round];
-        b.next_base = base[round + 1];
-        b.next_cap = cap[round + 1];
-        k_walk64<TPL, FIELDS, QUAD><<<(unsigned)nb, 64 * WALK_WAVES, 0, s>>>(a, b);
-        PTG_LAUNCH_CHECK();
-    }
-    for (int round = rounds - 2; round >= 0; round--) {
-        b.round = round;
-        b.base = base[round];
-        b.cap = cap[round];
-        k_walk64_sum<FIELDS><<<256, 256, 0, s>>>(a, b);
+    const ptg_status st = b.carve(ws, ws_bytes, blocks * WALK_WAVES, gcap, row);
+    if (st) return st;
+    const int64_t nb = a.goff ? blocks : std::min(blocks, ptg_cdiv(a.ngroups, WALK_WAVES));
+    k_walk64<TPL, FIELDS, QUAD, false><<<(unsigned)nb, 64 * WALK_WAVES, 0, s>>>(a, b);
+    PTG_LAUNCH_CHECK();
+    if (b.tcount && a.nslots > b.budget) {  // a traversal visits a slot once
+        k_walk64<TPL, FIELDS, QUAD, true><<<(unsigned)blocks, 64 * WALK_WAVES, 0, s>>>(a, b);
         PTG_LAUNCH_CHECK();
     }
     return PTG_OK;
