@@ -361,53 +361,11 @@ struct Geom {
     double center[3], size, cmin[3], inv;
 };
 
-__global__ __launch_bounds__(256) void k_bbox_partial(const double *pos, int64_t n, double *part)
+// box corners of a block of 256 threads, valid in thread 0
+__device__ __forceinline__ void block_corners(double lo[3], double hi[3], double sh[6][4])
 {
-    __shared__ double sh[6][4];
-    double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    const int wave = threadIdx.x >> 6, lane = ptg_lane();
 #pragma unroll
-        for (int k = 0; k < 3; k++) {
-            double x = pos[3 * i + k];
-            lo[k] = fmin(lo[k], x);
-            hi[k] = fmax(hi[k], x);
-        }
-    }
-    int wave = threadIdx.x >> 6, lane = ptg_lane();
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        lo[k] = ptg_wave_min(lo[k]);
-        hi[k] = ptg_wave_max(hi[k]);
-    }
-    if (lane == 0)
-        for (int k = 0; k < 3; k++) {
-            sh[k][wave] = lo[k];
-            sh[3 + k][wave] = hi[k];
-        }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int k = 0; k < 3; k++) {
-            double a = sh[k][0], b = sh[3 + k][0];
-            for (int w = 1; w < 4; w++) {
-                a = fmin(a, sh[k][w]);
-                b = fmax(b, sh[3 + k][w]);
-            }
-            part[6 * blockIdx.x + k] = a;
-            part[6 * blockIdx.x + 3 + k] = b;
-        }
-    }
-}
-
-__global__ __launch_bounds__(256) void k_bbox_final(const double *part, int nb, Geom *g)
-{
-    __shared__ double sh[6][4];
-    double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (int b = threadIdx.x; b < nb; b += blockDim.x)
-        for (int k = 0; k < 3; k++) {
-            lo[k] = fmin(lo[k], part[6 * b + k]);
-            hi[k] = fmax(hi[k], part[6 * b + 3 + k]);
-        }
-    int wave = threadIdx.x >> 6, lane = ptg_lane();
     for (int k = 0; k < 3; k++) {
         lo[k] = ptg_wave_min(lo[k]);
         hi[k] = ptg_wave_max(hi[k]);
@@ -422,11 +380,47 @@ __global__ __launch_bounds__(256) void k_bbox_final(const double *part, int nb, 
     for (int k = 0; k < 3; k++) {
         lo[k] = sh[k][0];
         hi[k] = sh[3 + k][0];
-        for (int w = 1; w < (int)(blockDim.x >> 6); w++) {
+        for (int w = 1; w < 4; w++) {
             lo[k] = fmin(lo[k], sh[k][w]);
             hi[k] = fmax(hi[k], sh[3 + k][w]);
         }
     }
+}
+
+__global__ __launch_bounds__(256) void k_bbox_partial(const double *pos, int64_t n, double *part)
+{
+    __shared__ double sh[6][4];
+    double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            double x = pos[3 * i + k];
+            lo[k] = fmin(lo[k], x);
+            hi[k] = fmax(hi[k], x);
+        }
+    }
+    block_corners(lo, hi, sh);
+    if (threadIdx.x == 0)
+        for (int k = 0; k < 3; k++) {
+            part[6 * blockIdx.x + k] = lo[k];
+            part[6 * blockIdx.x + 3 + k] = hi[k];
+        }
+}
+
+// block s: the cube g[s] of its nb partial boxes
+__global__ __launch_bounds__(256) void k_bbox_final(const double *part, int nb, Geom *g)
+{
+    __shared__ double sh[6][4];
+    part += 6 * (int64_t)blockIdx.x * nb;
+    g += blockIdx.x;
+    double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    for (int b = threadIdx.x; b < nb; b += blockDim.x)
+        for (int k = 0; k < 3; k++) {
+            lo[k] = fmin(lo[k], part[6 * b + k]);
+            hi[k] = fmax(hi[k], part[6 * b + 3 + k]);
+        }
+    block_corners(lo, hi, sh);
+    if (threadIdx.x != 0) return;
     for (int k = 0; k < 3; k++) g->center[k] = 0.5 * (hi[k] + lo[k]);
     double sz = hi[0] - lo[0];
     if (hi[1] - lo[1] > sz) sz = hi[1] - lo[1];
@@ -514,61 +508,53 @@ __global__ __launch_bounds__(256) void k_sys_of(const int64_t *offsets, int64_t 
     sys_in[i] = (uint32_t)lo;
 }
 
-// one block per system: its bounding cube (octree.py:539-574, per system)
-__global__ __launch_bounds__(256) void k_bbox_sys(const double *pos, const int64_t *offsets, Geom *geoms)
+// bounding cubes (octree.py:539-574, per system): `parts` blocks a system reduce its range to box corners,
+// one block a system reduces those.  One block a system alone read 2.6e6 particles of 128 systems at 0.6 TB/s
+// (104 us, the largest system setting the time).
+static int bbox_parts(int64_t nsys) { return (int)std::max<int64_t>(1, BB_BLOCKS / nsys); }
+
+__global__ __launch_bounds__(256) void k_bbox_sys_partial(const double *pos, const int64_t *offsets, int parts,
+                                                          double *part)
 {
     __shared__ double sh[6][4];
-    const int64_t a = offsets[blockIdx.x], b = offsets[blockIdx.x + 1];
+    const int64_t sys = blockIdx.x / parts;
+    const int64_t a = offsets[sys], b = offsets[sys + 1];
     double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (int64_t i = a + threadIdx.x; i < b; i += blockDim.x)
+    for (int64_t i = a + (int64_t)(blockIdx.x % parts) * blockDim.x + threadIdx.x; i < b;
+         i += (int64_t)parts * blockDim.x)
         for (int k = 0; k < 3; k++) {
             double x = pos[3 * i + k];
             lo[k] = fmin(lo[k], x);
             hi[k] = fmax(hi[k], x);
         }
-    int wave = threadIdx.x >> 6, lane = ptg_lane();
-    for (int k = 0; k < 3; k++) {
-        lo[k] = ptg_wave_min(lo[k]);
-        hi[k] = ptg_wave_max(hi[k]);
-    }
-    if (lane == 0)
+    block_corners(lo, hi, sh);
+    if (threadIdx.x == 0)
         for (int k = 0; k < 3; k++) {
-            sh[k][wave] = lo[k];
-            sh[3 + k][wave] = hi[k];
+            part[6 * (int64_t)blockIdx.x + k] = lo[k];
+            part[6 * (int64_t)blockIdx.x + 3 + k] = hi[k];
         }
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    for (int k = 0; k < 3; k++) {
-        lo[k] = sh[k][0];
-        hi[k] = sh[3 + k][0];
-        for (int w = 1; w < (int)(blockDim.x >> 6); w++) {
-            lo[k] = fmin(lo[k], sh[k][w]);
-            hi[k] = fmax(hi[k], sh[3 + k][w]);
-        }
-    }
-    Geom *g = geoms + blockIdx.x;
-    for (int k = 0; k < 3; k++) g->center[k] = 0.5 * (hi[k] + lo[k]);
-    double sz = hi[0] - lo[0];
-    if (hi[1] - lo[1] > sz) sz = hi[1] - lo[1];
-    if (hi[2] - lo[2] > sz) sz = hi[2] - lo[2];
-    g->size = sz;
-    g->inv = sz > 0 ? 1.0 / sz : 0.0;
-    for (int k = 0; k < 3; k++) g->cmin[k] = g->center[k] - 0.5 * sz;
 }
 
 __global__ __launch_bounds__(256) void k_keys_sys(const double *pos, const double *m, const double *h, int64_t n,
                                                   const Geom *geoms, const uint32_t *sys, uint64_t *keys,
-                                                  uint64_t *kU, uint32_t *vals, PartRec *rec)
+                                                  uint64_t *kU, uint32_t *vals, Counters *c, PartRec *rec)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const Geom *g = geoms + sys[i];
-    const double x = pos[3 * i], y = pos[3 * i + 1], z = pos[3 * i + 2];
-    uint64_t k = morton_key(x, y, z, g->cmin, g->inv);
-    keys[i] = k;
-    kU[i] = k;
-    vals[i] = (uint32_t)i;
-    if (rec) put_rec(rec, i, x, y, z, m[i], h[i]);
+    bool bad = false;
+    if (i < n) {
+        const Geom *g = geoms + sys[i];
+        const double x = pos[3 * i], y = pos[3 * i + 1], z = pos[3 * i + 2];
+        uint64_t k = morton_key(x, y, z, g->cmin, g->inv);
+        keys[i] = k;
+        kU[i] = k;
+        vals[i] = (uint32_t)i;
+        if (rec) {
+            const double mi = m[i], hi = h[i];
+            bad = !isfinite(x) || !isfinite(y) || !isfinite(z) || !isfinite(mi) || !isfinite(hi);
+            put_rec(rec, i, x, y, z, mi, hi);
+        }
+    }
+    if (ptg_ballot(bad) && ptg_lane() == 0) c->nonfinite = 1;
 }
 
 __global__ __launch_bounds__(256) void k_gather_sys_key(const uint32_t *sys, const uint32_t *vals, int64_t n,
@@ -597,18 +583,6 @@ __global__ __launch_bounds__(256) void k_forest_cubes(const Geom *geoms, int64_t
 // ============================================================================================
 // build workspace
 // ============================================================================================
-
-__global__ __launch_bounds__(256) void k_check_finite(const double *pos, const double *m, const double *h, int64_t n,
-                                                      Counters *c)
-{
-    bool bad = false;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        bad |= !isfinite(pos[3 * i]) || !isfinite(pos[3 * i + 1]) || !isfinite(pos[3 * i + 2]);
-        if (m) bad |= !isfinite(m[i]);
-        if (h) bad |= !isfinite(h[i]);
-    }
-    if (ptg_ballot(bad) && ptg_lane() == 0) c->nonfinite = 1;
-}
 
 struct BuildWS {
     double *part;
@@ -639,7 +613,7 @@ struct BuildWS {
 
 static bool carve_build(PtgArena &A, int64_t n, BuildWS &w, int64_t nsys = 1)
 {
-    w.part = A.take<double>(6 * BB_BLOCKS);
+    w.part = A.take<double>(6 * std::max<int64_t>(BB_BLOCKS, nsys));
     w.geom = A.take<Geom>(1);
     w.ctr = A.take<Counters>(1);
     w.kA = A.take<uint64_t>(n);
@@ -974,8 +948,11 @@ static ptg_status sort_by_keys_forest(const double *pos, const double *m, const 
                                       hipStream_t s)
 {
     k_sys_of<<<grid1(n), 256, 0, s>>>(w.soff, w.nsys, n, w.sys);
-    k_bbox_sys<<<(unsigned)w.nsys, 256, 0, s>>>(pos, w.soff, w.geoms);
-    k_keys_sys<<<grid1(n), 256, 0, s>>>(pos, m, h, n, w.geoms, w.sys, w.kA, w.kU, w.vA, m && h ? w.rec : nullptr);
+    const int parts = bbox_parts(w.nsys);
+    k_bbox_sys_partial<<<(unsigned)(w.nsys * parts), 256, 0, s>>>(pos, w.soff, parts, w.part);
+    k_bbox_final<<<(unsigned)w.nsys, 256, 0, s>>>(w.part, parts, w.geoms);
+    k_keys_sys<<<grid1(n), 256, 0, s>>>(pos, m, h, n, w.geoms, w.sys, w.kA, w.kU, w.vA, w.ctr,
+                                        m && h ? w.rec : nullptr);
     PTG_LAUNCH_CHECK();
     bool in_first;
     ptg_status st = radix_sort(w.kA, w.vA, w.kB, w.vB, n, 64, w.rs, &in_first, s);
@@ -1181,13 +1158,11 @@ extern "C" ptg_status ptg_build_sort(const double *pos, const double *m, const d
         return PTG_ERR_ARG;
     };
     if (forest) {
-        // forests: the offsets index the per-system kernels, so they (and the inputs) are checked
-        // before anything else runs; a single tree checks finiteness inside the key pass instead
-        k_check_finite<<<(unsigned)std::min<int64_t>(1024, ptg_cdiv(n, 256)), 256, 0, s>>>(pos, m, h, n, w.ctr);
-        if (forest) k_check_offsets<<<grid1(nsys + 1), 256, 0, s>>>(forest->offsets, nsys, n, w.ctr);
+        // the offsets index the per-system kernels, so they are checked before anything else runs
+        // (the key pass checks the inputs: a pass of its own took 107 of the 9500 us of a 1e7-particle step)
+        k_check_offsets<<<grid1(nsys + 1), 256, 0, s>>>(forest->offsets, nsys, n, w.ctr);
         PTG_HIP_CHECK(hipMemcpyAsync(&hc, w.ctr, sizeof(Counters), hipMemcpyDeviceToHost, s));
         PTG_HIP_CHECK(hipStreamSynchronize(s));
-        if (hc.nonfinite) return nonfinite();
         if (hc.badforest) {
             ptg_set_error("ptg_build_sort: forest offsets must start at 0, end at n and give every system >= 2 "
                           "particles");
@@ -2137,10 +2112,7 @@ extern "C" ptg_status ptg_build_deferred(const double *pos, const double *m, con
     if (st) return st;
     phase_mark(PTG_PHASE_SORT, s);
     if (!F) PTG_HIP_CHECK(hipMemcpyAsync(w.geoms, w.geom, sizeof(Geom), hipMemcpyDeviceToDevice, s));
-    if (forest) {
-        if (F) k_check_finite<<<(unsigned)std::min<int64_t>(1024, ptg_cdiv(n, 256)), 256, 0, s>>>(pos, m, h, n, w.ctr);
-        k_forest_cubes<<<grid1(nsys), 256, 0, s>>>(w.geoms, nsys, forest->cubes);
-    }
+    if (forest) k_forest_cubes<<<grid1(nsys), 256, 0, s>>>(w.geoms, nsys, forest->cubes);
     k_levels<<<lev_grid(n), 256, 0, s>>>(w.kA, w.sys, n, w.lev, w.ctr);
     // collision runs: re-keyed here; the stage's kernels read k_levels' count of colliding pairs and
     // return at once when it is 0 (nsub then stays 0 from the zeroed counters)
@@ -2568,7 +2540,7 @@ static int64_t group_tiles(int64_t n) { return std::max<int64_t>(1, ptg_cdiv(n, 
 static bool carve_groups(PtgArena &A, int64_t n, int64_t nsys, GroupWS &w)
 {
     const int64_t nt = group_tiles(n);
-    w.part = A.take<double>(6 * BB_BLOCKS);
+    w.part = A.take<double>(6 * std::max<int64_t>(BB_BLOCKS, nsys));
     w.geom = A.take<Geom>(nsys);
     w.keys = A.take<uint64_t>(n);
     w.gmask = A.take<uint64_t>(nt * GT_WORDS);
@@ -2619,7 +2591,9 @@ extern "C" ptg_status ptg_target_groups(const double *pos, const int64_t *perm, 
         if (nsys > 1) {
             // targets are the forest's own particles: system s owns input indices and sorted
             // positions [offsets[s], offsets[s+1])
-            k_bbox_sys<<<(unsigned)nsys, 256, 0, s>>>(pos, soff, w.geom);
+            const int parts = bbox_parts(nsys);
+            k_bbox_sys_partial<<<(unsigned)(nsys * parts), 256, 0, s>>>(pos, soff, parts, w.part);
+            k_bbox_final<<<(unsigned)nsys, 256, 0, s>>>(w.part, parts, w.geom);
         } else {
             int nb = (int)std::min<int64_t>(BB_BLOCKS, std::max<int64_t>(1, ptg_cdiv(n, 1024)));
             k_bbox_partial<<<nb, 256, 0, s>>>(pos, n, w.part);
