@@ -182,7 +182,7 @@ struct LoadArr {
 
 // ============================================================================================
 // LSD radix sort of (u64 key, u32 value) pairs, 8-bit digits.  Each 256-thread block owns a tile of
-// RS_TILE consecutive elements.  Per pass: a tile histogram, the offset of every (digit, tile) (one
+// 256 RS_ITEMS consecutive elements.  Per pass: a tile histogram, the offset of every (digit, tile) (one
 // block per digit scans that digit's tile counts and writes the digit's total; each scatter block
 // turns the 256 totals into digit starts itself), and a scatter that ranks the tile's keys stably
 // (ballot-based digit matching inside each wave, per-digit prefix over the waves), reorders the
@@ -194,18 +194,23 @@ struct LoadArr {
 // ============================================================================================
 #define RS_BITS 8
 #define RS_BINS 256
-#define RS_ITEMS 8
 #define RS_WAVES 4
 #define RS_THREADS (64 * RS_WAVES)
-#define RS_TILE (RS_THREADS * RS_ITEMS)
 
+// Keys a thread ranks, one after the other.  Long tiles write long runs, which is what a large sort needs; a
+// small one waits for the chain of a few blocks instead.  Whole builds with 1 / 2 / 4 / 8 keys a thread, us:
+// 5e3 particles 356 / 374 / 384 / 410, 5e4 393 / 401 / 419 / 437, 1e5 430 / 428 / 435 / 460, 2e5 489 / 479 /
+// 481 / 494, 7e5 721 / 656 / 617 / 639, 1e6 871 / 767 / 703 / 709, 2e6 1372 / 1154 / 1019 / 950.
+static int rs_items(int64_t n) { return n <= (1 << 16) ? 1 : n <= (1 << 18) ? 2 : n <= (1 << 20) ? 4 : 8; }
+
+template <int RS_ITEMS>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const uint64_t *keys, int64_t n, int shift, int64_t ntiles,
                                                         int32_t *hist)
 {
     __shared__ uint32_t cnt[RS_BINS];
     cnt[threadIdx.x] = 0;
     __syncthreads();
-    int64_t base = (int64_t)blockIdx.x * RS_TILE;
+    int64_t base = (int64_t)blockIdx.x * (RS_THREADS * RS_ITEMS);
 #pragma unroll 4
     for (int r = 0; r < RS_ITEMS; r++) {
         int64_t i = base + r * RS_THREADS + threadIdx.x;
@@ -215,10 +220,12 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const uint64_t *keys, in
     hist[(int64_t)threadIdx.x * ntiles + blockIdx.x] = (int32_t)cnt[threadIdx.x];
 }
 
+template <int RS_ITEMS>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint64_t *kin, const uint32_t *vin, int64_t n,
                                                            int shift, int64_t ntiles, const int32_t *offs,
                                                            const int32_t *dtot, uint64_t *kout, uint32_t *vout)
 {
+    constexpr int RS_TILE = RS_THREADS * RS_ITEMS;
     __shared__ uint64_t sk[RS_TILE];
     __shared__ uint32_t sv[RS_TILE];
     __shared__ uint32_t run[RS_WAVES][RS_BINS];
@@ -295,8 +302,8 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint64_t *kin, 
     }
 }
 
-// number of sort tiles (sizes the histogram array: RS_BINS entries per tile)
-static int64_t rs_nwt(int64_t n) { return std::max<int64_t>(1, ptg_cdiv(n, RS_TILE)); }
+// number of sort tiles of n keys (RS_BINS histogram entries each)
+static int64_t rs_tiles(int64_t n, int items) { return std::max<int64_t>(1, ptg_cdiv(n, RS_THREADS * items)); }
 
 struct RsWS {
     int32_t *hist;   // (RS_BINS, ntiles) tile counts, scanned in place per digit
@@ -306,7 +313,7 @@ struct RsWS {
 
 static void carve_rs(PtgArena &A, int64_t n, RsWS &w)
 {
-    w.hist = A.take<int32_t>((int64_t)RS_BINS * rs_nwt(n));
+    w.hist = A.take<int32_t>((int64_t)RS_BINS * rs_tiles(n, rs_items(n)));
     w.dtot = A.take<int32_t>(RS_BINS);
     w.cap = n;
 }
@@ -338,14 +345,26 @@ static ptg_status radix_sort(uint64_t *k0, uint32_t *v0, uint64_t *k1, uint32_t 
         ptg_set_error("radix_sort: %lld keys exceed the workspace's %lld", (long long)n, (long long)w.cap);
         return PTG_ERR_WORKSPACE;
     }
-    const int64_t ntiles = rs_nwt(n);
+    const int items = rs_items(w.cap);  // by what the histogram was sized for
+    const int64_t ntiles = rs_tiles(n, items);
     bool first = true;
     for (int shift = 0; shift < nbits; shift += RS_BITS) {
         uint64_t *ki = first ? k0 : k1, *ko = first ? k1 : k0;
         uint32_t *vi = first ? v0 : v1, *vo = first ? v1 : v0;
-        k_rs_hist<<<ntiles, RS_THREADS, 0, s>>>(ki, n, shift, ntiles, w.hist);
-        k_rs_tile_scan<<<RS_BINS, 256, 0, s>>>(w.hist, ntiles, w.dtot);
-        k_rs_scatter<<<ntiles, RS_THREADS, 0, s>>>(ki, vi, n, shift, ntiles, w.hist, w.dtot, ko, vo);
+#define RS_PASS(I)                                                                  \
+    k_rs_hist<I><<<ntiles, RS_THREADS, 0, s>>>(ki, n, shift, ntiles, w.hist);       \
+    k_rs_tile_scan<<<RS_BINS, 256, 0, s>>>(w.hist, ntiles, w.dtot);                 \
+    k_rs_scatter<I><<<ntiles, RS_THREADS, 0, s>>>(ki, vi, n, shift, ntiles, w.hist, w.dtot, ko, vo);
+        if (items == 1) {
+            RS_PASS(1)
+        } else if (items == 2) {
+            RS_PASS(2)
+        } else if (items == 4) {
+            RS_PASS(4)
+        } else {
+            RS_PASS(8)
+        }
+#undef RS_PASS
         PTG_LAUNCH_CHECK();
         first = !first;
     }
@@ -1751,7 +1770,7 @@ __device__ __forceinline__ void lane_moments(int64_t idx, int64_t n, int64_t ne,
 }
 
 #define MOM_THREADS 256
-#define MOM_DEFERRED_BLOCKS 2048  // grid of each level's launch in a deferred build (grid-stride over the level)
+#define MOM_BLOCKS 2048  // at most, for each level's launch (grid-stride over the level)
 
 // one level, one node per lane
 template <bool QUAD>
@@ -1934,11 +1953,12 @@ static ptg_status tree_phase(const double *pos, const double *m, const double *h
         // round trip for the level sizes; small levels cost a few microseconds of dispatch and load
         // latency each: running the levels nearest the root in one workgroup with barriers measured
         // no faster, as each level's chain of dependent loads remains)
+        const unsigned mb = (unsigned)std::min<int64_t>(MOM_BLOCKS, ptg_cdiv(nnodes, MOM_THREADS));
         for (int L = max_level; L >= 0; L--) {
             if (quadrupole)
-                k_moments_level<true><<<MOM_DEFERRED_BLOCKS, MOM_THREADS, 0, s>>>(n, nnodes, L, nw.lvstart, byid, t, nw);
+                k_moments_level<true><<<mb, MOM_THREADS, 0, s>>>(n, nnodes, L, nw.lvstart, byid, t, nw);
             else
-                k_moments_level<false><<<MOM_DEFERRED_BLOCKS, MOM_THREADS, 0, s>>>(n, nnodes, L, nw.lvstart, byid, t, nw);
+                k_moments_level<false><<<mb, MOM_THREADS, 0, s>>>(n, nnodes, L, nw.lvstart, byid, t, nw);
         }
     } else {
         k_fold_particles<<<grid1(nnodes), 256, 0, s>>>(n, nnodes, t);
