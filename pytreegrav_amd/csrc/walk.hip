@@ -158,41 +158,56 @@ __device__ __forceinline__ SplineFast<T> spline_fast(T r, T rinv, T h)
     return o;
 }
 
-// Particle on one target, fast path: point mass unless any lane is inside the softening radius,
-// in which case those lanes evaluate the spline (wave-uniform branch); r2 == 0 contributes zero.
-template <typename T, int FIELDS>
-__device__ __forceinline__ void interact_part_fast(Acc<T> &a, V4<T> s, T hs, T tx, T ty, T tz, T th)
+// Particle on one target, fast path: point mass unless any lane is inside the softening radius, in which
+// case those lanes evaluate the spline; r2 == 0 contributes zero.  part_pair says whether this lane's pair is
+// softened, part_add adds it (SOFT: with the spline branch).
+template <typename T> struct PartPair {
+    T dx, dy, dz, r2, ht;
+    bool nonzero, soft;
+};
+template <typename T>
+__device__ __forceinline__ PartPair<T> part_pair(const V4<T> &s, T hs, T tx, T ty, T tz, T th)
+{
+    PartPair<T> p;
+    p.dx = s.x - tx;
+    p.dy = s.y - ty;
+    p.dz = s.z - tz;
+    p.r2 = p.dx * p.dx + p.dy * p.dy + p.dz * p.dz;
+    p.ht = fmaxf(hs, th);
+    p.nonzero = p.r2 > T(0);
+    p.soft = p.nonzero && p.r2 < p.ht * p.ht;
+    return p;
+}
+template <typename T, int FIELDS, bool SOFT>
+__device__ __forceinline__ void part_add(Acc<T> &a, const PartPair<T> &p, T m)
 {
     constexpr bool P = NW<FIELDS>::POT, G = NW<FIELDS>::ACC, D = NW<FIELDS>::TID;
-    T dx = s.x - tx, dy = s.y - ty, dz = s.z - tz;
-    T r2 = dx * dx + dy * dy + dz * dz;
-    T ht = fmaxf(hs, th);
-    bool nonzero = r2 > T(0);
-    bool soft = nonzero && r2 < ht * ht;
-    T rinv = nonzero ? fast_rsqrt(r2) : T(0);
+    const T dx = p.dx, dy = p.dy, dz = p.dz;
+    T rinv = p.nonzero ? fast_rsqrt(p.r2) : T(0);
     T rinv2 = rinv * rinv;
-    T mr = s.w * rinv;
+    T mr = m * rinv;
     T phi = -mr;
     T K = mr * rinv2;
     T Q = T(3) * K * rinv2;
-    if (ptg_ballot(soft)) {
-        if (soft) {
-            SplineFast<T> sp = spline_fast<T, P, D>(r2 * rinv, rinv, ht);
-            if (P) phi = s.w * sp.phi;
-            K = s.w * sp.K;
-            if (D) Q = s.w * sp.Q;
-        }
+    if (SOFT && p.soft) {
+        SplineFast<T> sp = spline_fast<T, P, D>(p.r2 * rinv, rinv, p.ht);
+        if (P) phi = m * sp.phi;
+        K = m * sp.K;
+        if (D) Q = m * sp.Q;
     }
-    if (P) a.phi += phi;
+    if (P) {
+#pragma clang fp contract(off)  // rounded as in the soft branch, whichever other lanes and entries share the batch
+        a.phi += phi;
+    }
     if (G) {
         a.gx += K * dx;
         a.gy += K * dy;
         a.gz += K * dz;
     }
     if (D) {
-        a.txx += Q * dx * dx - K;
-        a.tyy += Q * dy * dy - K;
-        a.tzz += Q * dz * dz - K;
+        a.txx += fma(Q * dx, dx, -K);
+        a.tyy += fma(Q * dy, dy, -K);
+        a.tzz += fma(Q * dz, dz, -K);
         a.txy += Q * dx * dy;
         a.txz += Q * dx * dz;
         a.tyz += Q * dy * dz;
@@ -311,38 +326,85 @@ __device__ __forceinline__ void exp_eval(Acc<T> &a, const GroupExp<T> &E, T ux, 
     }
 }
 
-template <typename T, int TPL, int FIELDS, bool QUAD, int LF>
-__device__ __forceinline__ void flush_nodes(const WaveLds<T, QUAD, LF> &L, int cnt, Acc<T> (&acc)[TPL],
-                                            const T (&tx)[TPL], const T (&ty)[TPL], const T (&tz)[TPL],
-                                            const T (&th)[TPL])
+// U entries of a list are evaluated together: their LDS reads are issued at once and their chains overlap.  One
+// at a time, every entry waited for its read and 4 of a node's 19 instructions were the loop's; for particles the
+// spline was evaluated whether a lane was softened or not.  The terms are added in the order of the list.
+// Whole calls, one entry -> U: 1000 targets on 1e5 particles 2.43 -> 1.54 ms, FP32 acceleration of
+// 5e4 particles 0.93 -> 0.84, of 1e6 2.10 -> 1.95, a learned step of 1e7 9.57 -> 9.25.
+template <typename T, int TPL, int FIELDS, bool QUAD, int LF, int U>
+__device__ __forceinline__ void add_nodes(const WaveLds<T, QUAD, LF> &L, int k, Acc<T> (&acc)[TPL],
+                                          const T (&tx)[TPL], const T (&ty)[TPL], const T (&tz)[TPL])
 {
-    for (int k = 0; k < cnt; k++) {
-        V4<T> s = L.nodes[k];
-        T q[6];
+    V4<T> s[U];
+    T q[U][6];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        s[u] = L.nodes[k + u];
         if (QUAD) {
 #pragma unroll
-            for (int c = 0; c < 6; c++) q[c] = L.nq[6 * k + c];
+            for (int c = 0; c < 6; c++) q[u][c] = L.nq[6 * (k + u) + c];
         }
+    }
 #pragma unroll
-        for (int j = 0; j < TPL; j++) {
-            interact_node_fast<T, FIELDS, QUAD>(acc[j], s, q, tx[j], ty[j], tz[j]);
+    for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int j = 0; j < TPL; j++) interact_node_fast<T, FIELDS, QUAD>(acc[j], s[u], q[u], tx[j], ty[j], tz[j]);
+}
+
+template <int U, typename T, int TPL, int FIELDS, bool QUAD, int LF>
+__device__ __forceinline__ void flush_nodes(const WaveLds<T, QUAD, LF> &L, int cnt, Acc<T> (&acc)[TPL],
+                                            const T (&tx)[TPL], const T (&ty)[TPL], const T (&tz)[TPL])
+{
+    int k = 0;
+#pragma unroll 1
+    for (; k + U <= cnt; k += U) add_nodes<T, TPL, FIELDS, QUAD, LF, U>(L, k, acc, tx, ty, tz);
+#pragma unroll 1
+    for (; U > 1 && k < cnt; k++) add_nodes<T, TPL, FIELDS, QUAD, LF, 1>(L, k, acc, tx, ty, tz);
+}
+
+template <typename T, int TPL, int FIELDS, bool QUAD, int LF, int U>
+__device__ __forceinline__ void add_parts(const WaveLds<T, QUAD, LF> &L, int k, Acc<T> (&acc)[TPL],
+                                          const T (&tx)[TPL], const T (&ty)[TPL], const T (&tz)[TPL],
+                                          const T (&th)[TPL])
+{
+    V4<T> s[U];
+    T hs[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        s[u] = L.parts[k + u];
+        hs[u] = L.ph[k + u];
+    }
+#pragma unroll
+    for (int j = 0; j < TPL; j++) {
+        PartPair<T> p[U];
+        bool soft = false;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            p[u] = part_pair(s[u], hs[u], tx[j], ty[j], tz[j], th[j]);
+            soft |= p[u].soft;
+        }
+        if (U == 1 || ptg_ballot(soft)) {
+            // the barrier keeps this a branch: as selects, every pair went through the spline's 40 instructions
+            if (U > 1) __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int u = 0; u < U; u++) part_add<T, FIELDS, true>(acc[j], p[u], s[u].w);
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; u++) part_add<T, FIELDS, false>(acc[j], p[u], s[u].w);
         }
     }
 }
 
-template <typename T, int TPL, int FIELDS, bool QUAD, int LF>
+template <int U, typename T, int TPL, int FIELDS, bool QUAD, int LF>
 __device__ __forceinline__ void flush_parts(const WaveLds<T, QUAD, LF> &L, int cnt, Acc<T> (&acc)[TPL],
                                             const T (&tx)[TPL], const T (&ty)[TPL], const T (&tz)[TPL],
                                             const T (&th)[TPL])
 {
-    for (int k = 0; k < cnt; k++) {
-        V4<T> s = L.parts[k];
-        T hs = L.ph[k];
-#pragma unroll
-        for (int j = 0; j < TPL; j++) {
-            interact_part_fast<T, FIELDS>(acc[j], s, hs, tx[j], ty[j], tz[j], th[j]);
-        }
-    }
+    int k = 0;
+#pragma unroll 1
+    for (; k + U <= cnt; k += U) add_parts<T, TPL, FIELDS, QUAD, LF, U>(L, k, acc, tx, ty, tz, th);
+#pragma unroll 1
+    for (; U > 1 && k < cnt; k++) add_parts<T, TPL, FIELDS, QUAD, LF, 1>(L, k, acc, tx, ty, tz, th);
 }
 
 // Kernel variants of the FP32 one-target-per-lane walk (ptg_criterion.variant; the autotuner picks
@@ -371,6 +433,14 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
 {
     constexpr int LF = WalkOcc<T, TPL, VAR>::lf;
     constexpr bool TASKS = PASS == TASK;
+    // entries evaluated together (nodes, particles): 4 where the registers of five waves per SIMD hold them.
+    // The expansion's 16 sums leave room for 2 (with 4: 13 spilled registers), and in the six-wave variant for
+    // none; tidal or quadrupole particles take 2.  4 and 2 against 1 and 1 with quadrupoles: 2.20 against 2.33 ms
+    // for 1e6 particles, 2.89 against 3.60 with tidal tensors of 1e5 targets; 8 nodes were no faster than 4.  Two
+    // and four targets per lane fill the chain alone: 2 nodes 0.81 against 0.83 ms (groups of 128, 3e5
+    // particles), with quadrupoles 1 (2.75 ms for groups of 256; 2.89 with 2).
+    constexpr int UN = VAR == 2 ? (EXP ? 1 : 2) : TPL > 1 ? (QUAD ? 1 : 2) : EXP ? 2 : 4;
+    constexpr int UP = VAR == 2 ? UN : TPL > 1 ? 1 : EXP || QUAD || NW<FIELDS>::TID ? 2 : 4;
     static_assert(!EXP || (!QUAD && !NW<FIELDS>::TID), "the group expansion is a monopole potential/acceleration path");
     __shared__ WaveLds<T, QUAD, LF> lds[WALK_WAVES];
     const int wave = threadIdx.x >> 6, lane = ptg_lane();
@@ -632,7 +702,7 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
 
                     if (nn >= LF) {
                         const int c = nn & ~(LF - 1);  // c >= LF > nn - c
-                        flush_nodes<T, TPL, FIELDS, QUAD, LF>(L, c, acc, tx, ty, tz, th);
+                        flush_nodes<UN, T, TPL, FIELDS, QUAD, LF>(L, c, acc, tx, ty, tz);
                         __builtin_amdgcn_wave_barrier();
                         if (lane < nn - c) {  // reads [c, nn) and writes [0, nn - c): disjoint
                             L.nodes[lane] = L.nodes[c + lane];
@@ -644,7 +714,7 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
                     }
                     if (np >= LF) {
                         const int c = np & ~(LF - 1);
-                        flush_parts<T, TPL, FIELDS, QUAD, LF>(L, c, acc, tx, ty, tz, th);
+                        flush_parts<UP, T, TPL, FIELDS, QUAD, LF>(L, c, acc, tx, ty, tz, th);
                         __builtin_amdgcn_wave_barrier();
                         if (lane < np - c) {  // disjoint ranges, as above
                             L.parts[lane] = L.parts[c + lane];
@@ -677,8 +747,8 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
                 if (!TASKS) continue;
                 nn = np = 0;  // a task's row is written all the same: the sums read every task's
             }
-            flush_nodes<T, TPL, FIELDS, QUAD, LF>(L, nn, acc, tx, ty, tz, th);
-            flush_parts<T, TPL, FIELDS, QUAD, LF>(L, np, acc, tx, ty, tz, th);
+            flush_nodes<UN, T, TPL, FIELDS, QUAD, LF>(L, nn, acc, tx, ty, tz);
+            flush_parts<UP, T, TPL, FIELDS, QUAD, LF>(L, np, acc, tx, ty, tz, th);
             __builtin_amdgcn_wave_barrier();
             if constexpr (EXP) {
                 exp_wave_sum(E);
