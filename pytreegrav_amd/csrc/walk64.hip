@@ -136,27 +136,106 @@ __device__ __forceinline__ void spline64(double r, double rinv, double h, double
     }
 }
 
-template <int FIELDS>
-__device__ __forceinline__ void pair_part(Acc<double> &a, const V4<double> &s, double hs, double tx, double ty, double tz,
-                                          double th)
+// A particle's pair: the spline where it is softened, nothing where it coincides (SOFT: with that branch).
+struct Pair64 {
+    double dx, dy, dz, r2, h;
+    bool apart, soft;
+};
+__device__ __forceinline__ Pair64 part_pair(const V4<double> &s, double hs, double tx, double ty, double tz, double th)
 {
-    const double dx = s.x - tx, dy = s.y - ty, dz = s.z - tz;
-    const double r2 = fmin(dx * dx + dy * dy + dz * dz, R2_MAX);
-    const double h = fmax(hs, th);
-    const bool apart = r2 > 0.0;
-    const double rinv = apart ? rsqrt64(r2) : 0.0, rinv2 = rinv * rinv;
-    const double mr = s.w * rinv;
+    Pair64 p;
+    p.dx = s.x - tx;
+    p.dy = s.y - ty;
+    p.dz = s.z - tz;
+    p.r2 = fmin(p.dx * p.dx + p.dy * p.dy + p.dz * p.dz, R2_MAX);
+    p.h = fmax(hs, th);
+    p.apart = p.r2 > 0.0;
+    p.soft = p.apart && p.r2 < p.h * p.h;
+    return p;
+}
+template <int FIELDS, bool SOFT>
+__device__ __forceinline__ void part_add(Acc<double> &a, const Pair64 &p, double m)
+{
+    const double rinv = p.apart ? rsqrt64(p.r2) : 0.0, rinv2 = rinv * rinv;
+    const double mr = m * rinv;
     double phi = -mr, K = mr * rinv2, Q = 3.0 * K * rinv2;
-    const bool soft = apart && r2 < h * h;
-    if (ptg_ballot(soft)) {
-        if (soft) {
-            spline64<FIELDS>(r2 * rinv, rinv, h, phi, K, Q);
-            phi *= s.w;
-            K *= s.w;
-            Q *= s.w;
+    if (SOFT && p.soft) {
+        spline64<FIELDS>(p.r2 * rinv, rinv, p.h, phi, K, Q);
+        phi *= m;
+        K *= m;
+        Q *= m;
+    }
+    add_pair<FIELDS>(a, phi, K, Q, p.dx, p.dy, p.dz);
+}
+
+// U entries of a lane's slice of a list together: their LDS reads are issued at once and their chains
+// overlap, and the spline is evaluated only where a pair of the batch is softened.  The terms are added in
+// the order of the list.
+template <int U, int TPL, int FIELDS, bool QUAD, typename L>
+__device__ __forceinline__ void add_nodes(const L &l, int at, int step, Acc<double> (&acc)[TPL], const double (&tx)[TPL],
+                                          const double (&ty)[TPL], const double (&tz)[TPL])
+{
+    V4<double> s[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) s[u] = l.nodes[at + u * step];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int j = 0; j < TPL; j++)
+            pair_node<FIELDS, QUAD>(acc[j], s[u], &l.nq[QUAD ? 6 * (at + u * step) : 0], tx[j], ty[j], tz[j]);
+}
+template <int U, int TPL, int FIELDS, typename L>
+__device__ __forceinline__ void add_parts(const L &l, int at, int step, Acc<double> (&acc)[TPL], const double (&tx)[TPL],
+                                          const double (&ty)[TPL], const double (&tz)[TPL], const double (&th)[TPL])
+{
+    V4<double> s[U];
+    double hs[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        s[u] = l.parts[at + u * step];
+        hs[u] = l.ph[at + u * step];
+    }
+#pragma unroll
+    for (int j = 0; j < TPL; j++) {
+        Pair64 p[U];
+        bool soft = false;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            p[u] = part_pair(s[u], hs[u], tx[j], ty[j], tz[j], th[j]);
+            soft |= p[u].soft;
+        }
+        if (ptg_ballot(soft)) {
+            // the barrier keeps this a branch: as selects, every pair went through the spline's 27 instructions
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int u = 0; u < U; u++) part_add<FIELDS, true>(acc[j], p[u], s[u].w);
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; u++) part_add<FIELDS, false>(acc[j], p[u], s[u].w);
         }
     }
-    add_pair<FIELDS>(a, phi, K, Q, dx, dy, dz);
+}
+// entries [0, c) of the lists, this lane's slice of them
+template <int U, int TPL, int FIELDS, bool QUAD, typename L>
+__device__ __forceinline__ void sum_nodes(const L &l, int sl, int slices, int c, Acc<double> (&acc)[TPL],
+                                          const double (&tx)[TPL], const double (&ty)[TPL], const double (&tz)[TPL])
+{
+    int q = sl;
+#pragma unroll 1
+    for (; q + (U - 1) * slices < c; q += U * slices) add_nodes<U, TPL, FIELDS, QUAD>(l, q, slices, acc, tx, ty, tz);
+#pragma unroll 1
+    for (; U > 1 && q < c; q += slices) add_nodes<1, TPL, FIELDS, QUAD>(l, q, slices, acc, tx, ty, tz);
+}
+template <int U, int TPL, int FIELDS, typename L>
+__device__ __forceinline__ void sum_parts(const L &l, int sl, int slices, int c, Acc<double> (&acc)[TPL],
+                                          const double (&tx)[TPL], const double (&ty)[TPL], const double (&tz)[TPL],
+                                          const double (&th)[TPL])
+{
+    int q = sl;
+#pragma unroll 1
+    for (; q + (U - 1) * slices < c; q += U * slices) add_parts<U, TPL, FIELDS>(l, q, slices, acc, tx, ty, tz, th);
+#pragma unroll 1
+    for (; U > 1 && q < c; q += slices) add_parts<1, TPL, FIELDS>(l, q, slices, acc, tx, ty, tz, th);
 }
 
 // angle-binned columns of one lane: LDS sums bins[64 * bin] (units of mass / distance^2) and the part
@@ -230,6 +309,11 @@ __global__ __launch_bounds__(64 * WALK_WAVES) __attribute__((amdgpu_waves_per_eu
 void k_walk64(const Walk64Args A, const WalkPool B)
 {
     constexpr int WI = Sums<FIELDS>::WI;
+    // entries evaluated together (nodes, particles).  Quadrupoles, three waves per SIMD, have the registers for 4
+    // and 2: acceleration of 2e5 particles 2.31 -> 2.11 ms, of 1e5 in groups of 256 2.29 -> 2.06 (2 and 2: 2.19,
+    // 2.40).  Monopole sums at four waves have not: 4 and 2 spill 10 registers, 2 and 2 took the time of 1 and 1,
+    // which gain from the spline's branch alone (1e6 particles 4.45 -> 4.34 ms).
+    constexpr int UN = QUAD ? 4 : 1, UP = QUAD || NW<FIELDS>::TID ? 2 : 1;
     __shared__ Lds64<FIELDS, QUAD> lds[WALK_WAVES];
     const int wave = threadIdx.x >> 6, lane = ptg_lane();
     Lds64<FIELDS, QUAD> &L = lds[wave];
@@ -445,13 +529,10 @@ void k_walk64(const Walk64Args A, const WalkPool B)
 
                     if (nn >= LIST) {
                         const int c = nn & ~(LIST - 1);  // c >= LIST > nn - c
-                        for (int q = sl; q < c; q += slices) {
-                            const V4<double> s = L.nodes[q];
-#pragma unroll
-                            for (int j = 0; j < TPL; j++) {
-                                if constexpr (FIELDS == BINS) sky.node(s, tx[j], ty[j], tz[j]);
-                                else pair_node<FIELDS, QUAD>(acc[j], s, &L.nq[QUAD ? 6 * q : 0], tx[j], ty[j], tz[j]);
-                            }
+                        if constexpr (FIELDS == BINS) {
+                            for (int q = sl; q < c; q += slices) sky.node(L.nodes[q], tx[0], ty[0], tz[0]);
+                        } else {
+                            sum_nodes<UN, TPL, FIELDS, QUAD>(L, sl, slices, c, acc, tx, ty, tz);
                         }
                         __builtin_amdgcn_wave_barrier();
                         if (lane < nn - c) {  // reads [c, nn) and writes [0, nn - c): disjoint
@@ -464,13 +545,10 @@ void k_walk64(const Walk64Args A, const WalkPool B)
                     }
                     if (np >= LIST) {
                         const int c = np & ~(LIST - 1);
-                        for (int q = sl; q < c; q += slices) {
-                            const V4<double> s = L.parts[q];
-#pragma unroll
-                            for (int j = 0; j < TPL; j++) {
-                                if constexpr (FIELDS == BINS) sky.part(s, L.ph[q], tx[j], ty[j], tz[j]);
-                                else pair_part<FIELDS>(acc[j], s, L.ph[q], tx[j], ty[j], tz[j], th[j]);
-                            }
+                        if constexpr (FIELDS == BINS) {
+                            for (int q = sl; q < c; q += slices) sky.part(L.parts[q], L.ph[q], tx[0], ty[0], tz[0]);
+                        } else {
+                            sum_parts<UP, TPL, FIELDS>(L, sl, slices, c, acc, tx, ty, tz, th);
                         }
                         __builtin_amdgcn_wave_barrier();
                         if (lane < np - c) {  // disjoint ranges, as above
@@ -492,21 +570,15 @@ void k_walk64(const Walk64Args A, const WalkPool B)
                 if (lane == 0) atomicOr(&A.ctl->err, 1);
                 nn = np = 0;  // a task's row is still written: the sums read every task's
             }
-            for (int q = sl; q < nn; q += slices) {
-                const V4<double> s = L.nodes[q];
-#pragma unroll
-                for (int j = 0; j < TPL; j++) {
-                    if constexpr (FIELDS == BINS) sky.node(s, tx[j], ty[j], tz[j]);
-                    else pair_node<FIELDS, QUAD>(acc[j], s, &L.nq[QUAD ? 6 * q : 0], tx[j], ty[j], tz[j]);
-                }
+            if constexpr (FIELDS == BINS) {
+                for (int q = sl; q < nn; q += slices) sky.node(L.nodes[q], tx[0], ty[0], tz[0]);
+            } else {
+                sum_nodes<UN, TPL, FIELDS, QUAD>(L, sl, slices, nn, acc, tx, ty, tz);
             }
-            for (int q = sl; q < np; q += slices) {
-                const V4<double> s = L.parts[q];
-#pragma unroll
-                for (int j = 0; j < TPL; j++) {
-                    if constexpr (FIELDS == BINS) sky.part(s, L.ph[q], tx[j], ty[j], tz[j]);
-                    else pair_part<FIELDS>(acc[j], s, L.ph[q], tx[j], ty[j], tz[j], th[j]);
-                }
+            if constexpr (FIELDS == BINS) {
+                for (int q = sl; q < np; q += slices) sky.part(L.parts[q], L.ph[q], tx[0], ty[0], tz[0]);
+            } else {
+                sum_parts<UP, TPL, FIELDS>(L, sl, slices, np, acc, tx, ty, tz, th);
             }
             __builtin_amdgcn_wave_barrier();
             [[maybe_unused]] double bin[FIELDS == BINS ? 6 : 1];

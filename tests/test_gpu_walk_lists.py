@@ -1,11 +1,12 @@
-"""Interaction lists of the FP32 walk at every remainder of the batches that it evaluates together, with
+"""Interaction lists of the walks at every remainder of the batches that it evaluates together, with
 softened, unsoftened and coincident pairs in one batch, against the FP64 direct sum in numpy.
 
 theta = 1e-3 opens every node, so the lists hold the particles alone: the group of near targets lists them as
 particles, the far group as unsoftened ones.  Bound: 4e-5 of the sum of the pairs' magnitudes m / s^k with
 s = max(r, 0.05), the particles' least distance (3 for the two terms of a tidal tensor).  A pair's offset is
 off by 1e-7 (coordinates below 4 in FP32), relative to s 2e-6, up to five times that in the tidal tensor; the
-spline's polynomials cancel from about 100 to 1 in a few operations of 6e-8 (2e-5); 200 sums add 1e-5."""
+spline's polynomials cancel from about 100 to 1 in a few operations of 6e-8 (2e-5); 200 sums add 1e-5.  FP64: the same times 2^-29, doubled for
+reciprocals of two units in the last place and again for the reference's own rounding."""
 
 import numpy as np
 import pytest
@@ -16,24 +17,20 @@ from pytreegrav_amd import ConstructTree, engine
 pytestmark = pytest.mark.gpu
 
 
-def _spline(r, h):
+def _spline(r, h):  # kernel.py:4-75, with its decimal constants
     q = np.where(h > 0, r / np.where(h > 0, h, 1.0), 2.0)
     qs, hs = np.maximum(q, 1e-30), np.where(h > 0, h, 1.0)
     phi = np.where(q <= 0.5, -2.8 + q**2 * (16 / 3 + q**2 * (6.4 * q - 9.6)),
                    -3.2 + 1 / (15 * qs) + q**2 * (32 / 3 + q * (-16 + q * (9.6 - 32 / 15 * q)))) / hs
     K = np.where(q <= 0.5, 32 / 3 + q**2 * (32 * q - 38.4),
-                 64 / 3 - 48 * q + 38.4 * q**2 - 32 / 3 * q**3 - 1 / (15 * qs**3)) / hs**3
+                 21.333333333333 - 48 * q + 38.4 * q**2 - 10.666666666667 * q**3 - 0.066666666667 / qs**3) / hs**3
     Q = np.where(q <= 0.5, 76.8 - 96 * q, 48 / qs - 76.8 + 32 * q - 0.2 / qs**5) / hs**5
     far = (q >= 1) & (r > 0)
     rs = np.where(r > 0, r, 1.0)
     return np.where(far, -1 / rs, phi), np.where(far, rs**-3, K), np.where(far, 3 * rs**-5, Q)
 
 
-@pytest.mark.parametrize("n", [1, 2, 3, 5, 6, 31, 64, 65, 67, 130, 199])
-@pytest.mark.parametrize("mask,quad,gs,variant", [(1, False, 64, 0), (3, False, 64, 1), (2, False, 64, 2),
-                                                  (7, False, 64, 0), (3, True, 64, 0), (7, True, 64, 0),
-                                                  (2, False, 128, 0), (3, True, 256, 0)])
-def test_list_remainders(n, mask, quad, gs, variant):
+def _check(n, mask, quad, gs, variant, precision, tol):
     rng = np.random.default_rng(n)
     cells = rng.permutation(1000)[:n]  # one particle in the middle half of a cell of 0.1: at least 0.05 apart
     x = 0.1 * (np.stack([cells // 100, cells // 10 % 10, cells % 10], 1) + 0.25 + 0.5 * rng.random((n, 3)))
@@ -43,7 +40,7 @@ def test_list_remainders(n, mask, quad, gs, variant):
     tree = ConstructTree(x, m, h, quadrupole=quad)
     perm = torch.arange(len(t), dtype=torch.int64, device=engine.device())
     out = engine.walk(tree.dev, t, np.zeros(len(t)), perm, mask, quadrupole=quad, group_size=gs, theta=1e-3,
-                      precision="float32", grouping="fixed", variant=variant)
+                      precision=precision, grouping="fixed", variant=variant)
     d = x[None] - t[:, None]
     r = np.sqrt((d**2).sum(2))
     phi, K, Q = _spline(r, np.broadcast_to(h, r.shape))
@@ -55,4 +52,19 @@ def test_list_remainders(n, mask, quad, gs, variant):
         p = {"potential": 1, "accel": 2, "tidal": 3}[k]
         size = (1.0 if p < 3 else 3.0) * (w / s**p).sum(1)
         err = np.abs(v.cpu().numpy() - ref[k]).reshape(len(t), -1).max(1)
-        assert (err <= 4e-5 * size + 1e-30).all(), (k, (err / np.maximum(size, 1e-30)).max())
+        assert (err <= tol * size + 1e-30).all(), (k, (err / np.maximum(size, 1e-30)).max())
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 6, 31, 64, 65, 67, 130, 199])
+@pytest.mark.parametrize("mask,quad,gs,variant", [(1, False, 64, 0), (3, False, 64, 1), (2, False, 64, 2),
+                                                  (7, False, 64, 0), (3, True, 64, 0), (7, True, 64, 0),
+                                                  (2, False, 128, 0), (3, True, 256, 0)])
+def test_fp32_list_remainders(n, mask, quad, gs, variant):
+    _check(n, mask, quad, gs, variant, "float32", 4e-5)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 6, 31, 64, 65, 67, 130, 199])
+@pytest.mark.parametrize("mask,quad,gs", [(3, False, 1), (2, False, 8), (3, True, 8), (7, True, 16), (4, False, 64),
+                                          (2, True, 128), (3, True, 256)])
+def test_fp64_list_remainders(n, mask, quad, gs):
+    _check(n, mask, quad, gs, 0, "float64", 4 * 4e-5 * 2.0**-29)
