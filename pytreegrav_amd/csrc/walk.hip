@@ -445,6 +445,11 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
     __shared__ WaveLds<T, QUAD, LF> lds[WALK_WAVES];
     const int wave = threadIdx.x >> 6, lane = ptg_lane();
     WaveLds<T, QUAD, LF> &L = lds[wave];
+    // each wave's counts, added to the caller's when it ends: added per group they serialised on one line
+    // (the learned walk of 1e7 particles took 10.3 ms with counters, 4.1 without)
+    __shared__ unsigned long long counts[WALK_WAVES][4];
+    if (lane < 4) counts[wave][lane] = 0;
+    __builtin_amdgcn_wave_barrier();
     int *spill = B.spill + ((int64_t)blockIdx.x * WALK_WAVES + wave) * (int64_t)B.gcap;
     const int xcd = blockIdx.x % NXCD;
     int ghw = 0;  // this wave's deepest spill
@@ -736,10 +741,10 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
                     for (int d = 32; d >= 1; d >>= 1) n_exp += __shfl_xor(n_exp, d, 64);  // lanes fold separately
                 }
                 if (lane == 0) {
-                    atomicAdd((unsigned long long *)&A.counters[0], (unsigned long long)n_list * (unsigned long long)mt);
-                    atomicAdd((unsigned long long *)&A.counters[1], (unsigned long long)n_vis);
-                    atomicAdd((unsigned long long *)&A.counters[2], (unsigned long long)n_part * (unsigned long long)mt);
-                    if (EXP) atomicAdd((unsigned long long *)&A.counters[3], (unsigned long long)n_exp);
+                    counts[wave][0] += (unsigned long long)n_list * mt;
+                    counts[wave][1] += n_vis;
+                    counts[wave][2] += (unsigned long long)n_part * mt;
+                    if (EXP) counts[wave][3] += n_exp;
                 }
             }
             if (overflow) {
@@ -810,6 +815,9 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
         }
     }
     if (lane == 0 && ghw > 0) atomicMax(&A.ctl->hwm, ghw);
+    __builtin_amdgcn_wave_barrier();
+    if (A.counters && lane < (EXP ? 4 : 3) && counts[wave][lane])
+        atomicAdd((unsigned long long *)&A.counters[lane], counts[wave][lane]);
 }
 
 
