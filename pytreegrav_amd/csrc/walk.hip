@@ -455,7 +455,7 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
     int ghw = 0;  // this wave's deepest spill
     const int64_t ngroups = A.goff ? (int64_t)__builtin_amdgcn_readfirstlane(*A.gcount) : A.ngroups;
 
-    int closed = 0;
+    int ticket = -1, closed = 0;
     if (TASKS && agent_load(&A.ctl->open) == 0) return;  // nothing was deferred, or all of it is done
 
     for (int attempt = 0; attempt < (TASKS ? 1 : NXCD); attempt++) {
@@ -465,7 +465,7 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
             int self = -1, t_off = 0, t_stride = 0, t_count = 0;
             int64_t g;
             if (TASKS) {
-                self = walk_ticket(A.ctl, B, lane, closed);
+                self = walk_ticket(A.ctl, B, lane, ticket, closed);
                 if (self < 0) break;
                 const WalkTask *W = &B.tasks[self];
                 g = __builtin_amdgcn_readfirstlane(agent_load(&W->group));
@@ -786,7 +786,7 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
                 }
                 if (cut) {
                     wave_stores_done();
-                    walk_publish<TASKS>(A.ctl, B, g, gsp + sp, nchild, off, child0, self, lane);
+                    walk_publish<AgentMem>(A.ctl, B, TASKS, (int)g, gsp + sp, nchild, off, child0, self, lane);
                 } else {
                     walk_add_up<FIELDS, T>(B, self, grp, A.gs, A.perm, A.G, A.out, lane);
                 }
@@ -939,7 +939,7 @@ static ptg_status launch_t(const WalkArgs<T> &a, int64_t max_blocks, const WalkW
     b.div0 = 4;
     b.most = 128;
     b.div = 2;
-    ptg_status st = b.carve(ws.p, ws.bytes, blocks * WALK_WAVES, ws.gcap, (size_t)a.gs * WI * sizeof(T));
+    ptg_status st = walk_carve(b, ws.p, ws.bytes, blocks * WALK_WAVES, ws.gcap, (size_t)a.gs * WI * sizeof(T));
     if (st) return st;
     // a traversal visits a slot once, and no system has more targets than there are: where none can be
     // cut, the kernel without (its scalar registers do not spill; 2 to 7 % of the longest traversals)

@@ -322,7 +322,7 @@ void k_walk64(const Walk64Args A, const WalkPool B)
     int64_t n_int = 0, n_vis = 0, n_part = 0;
     int ghw = 0;
     const int64_t ngroups = A.goff ? (int64_t)__builtin_amdgcn_readfirstlane(*A.gcount) : A.ngroups;
-    int closed = 0;
+    int ticket = -1, closed = 0;
     if (TASKS && agent_load(&A.ctl->open) == 0) return;  // nothing was deferred, or all of it is done
     // targets per slice, a power of two
     int P = 64;
@@ -338,7 +338,7 @@ void k_walk64(const Walk64Args A, const WalkPool B)
             int self = -1, t_off = 0, t_stride = 0, t_count = 0;
             int64_t g;
             if (TASKS) {
-                self = walk_ticket(A.ctl, B, lane, closed);
+                self = walk_ticket(A.ctl, B, lane, ticket, closed);
                 if (self < 0) break;
                 const WalkTask *T = &B.tasks[self];
                 g = __builtin_amdgcn_readfirstlane(agent_load(&T->group));
@@ -619,7 +619,7 @@ void k_walk64(const Walk64Args A, const WalkPool B)
             }
             if (cut) {
                 wave_stores_done();
-                walk_publish<TASKS>(A.ctl, B, g, gsp + sp, nchild, off, child0, self, lane);
+                walk_publish<AgentMem>(A.ctl, B, TASKS, (int)g, gsp + sp, nchild, off, child0, self, lane);
             } else if (TASKS) {
                 walk_add_up<FIELDS, double>(B, self, grp, A.gs, A.perm, A.G, A.out, lane);
             }
@@ -661,7 +661,7 @@ static ptg_status launch(const Walk64Args &a, int cus, int gcap, char *ws, size_
     b.most = std::min(128, share);
     b.div = 2;
     const int64_t blocks = (int64_t)cus * per_cu;
-    const ptg_status st = b.carve(ws, ws_bytes, blocks * WALK_WAVES, gcap, row);
+    const ptg_status st = walk_carve(b, ws, ws_bytes, blocks * WALK_WAVES, gcap, row);
     if (st) return st;
     const int64_t nb = a.goff ? blocks : std::min(blocks, ptg_cdiv(a.ngroups, WALK_WAVES));
     k_walk64<TPL, FIELDS, QUAD, false><<<(unsigned)nb, 64 * WALK_WAVES, 0, s>>>(a, b);

@@ -6,30 +6,16 @@
 
 #include "ptg_common.hpp"
 
+#define WALK_FN static __device__ __forceinline__
+#include "walk_tasks.hpp"
+
 #define WALK_WAVES 4
 #define SCAP 768       // LDS traversal stack entries per wave (>= 512, the most children one step pushes)
 #define SPILL 256      // entries refilled from global memory at a time (<= SCAP - 512)
 #define GCAP 16384     // global spill entries per wave
-#define NXCD 8
-#define CTR_STRIDE 32  // int32 words between per-XCD counters (128 B)
 
 template <typename T> struct alignas(4 * sizeof(T)) V4 {
     T x, y, z, w;
-};
-
-#define WALK_DONE 16  // copies of the word that ends the task pass, each on its own line
-
-struct WalkCtl {
-    int32_t ctr[NXCD * CTR_STRIDE];   // per-XCD group counters
-    int32_t err;
-    int32_t hwm;  // deepest global spill stack (entries) any wave reached in the last walk
-    int32_t pad[30];
-    // deferral: entries taken of the deferred groups, of the tasks and of the saved stacks; tasks not yet
-    // finished; tickets drawn by the task pass, per XCD
-    int32_t ngroup, ntask, npool, pad2[29];
-    int32_t open, pad3[31];
-    int32_t ticket[NXCD * CTR_STRIDE];
-    int32_t done[WALK_DONE * 32];
 };
 
 template <int FIELDS> struct NW {
@@ -128,63 +114,42 @@ template <int FIELDS> __device__ __forceinline__ void store_sum(double *o, int c
 // same terms summed in another order).
 //
 // The second launch costs 3 us where nothing was deferred; a launch per generation of tasks and one per
-// level of sums cost 30.  Its waves end when no task is open: running waves wait for nothing, so the open
-// count falls to zero.  What one wave writes and another reads within it (records, stacks, rows) goes
+// level of sums cost 30.  Its waves end when no task is open; which wave walks which task is in
+// walk_tasks.hpp.  What one wave writes and another reads within it (records, stacks, rows) goes
 // through agent-scope accesses, ordered by the writer's wait before it publishes or counts down.
-struct WalkTask {
-    int32_t group;
-    int32_t parent;              // entry of tasks (-1: a deferred group)
-    int32_t off, stride, count;  // saved stack entries entries[off + i * stride], i < count
-    int32_t child0, nchild;      // its shares (a group or a task that was cut)
-    int32_t wait;                // shares not yet added
-};
+#define WALK_LOOKS (1 << 26)  // a wave gives up after a minute without a task and reports it
 
-#define WALK_MAX_TASKS 196608
-#define WALK_POLLS (1 << 26)  // a wave gives up after a minute without a task and reports it
-
-struct WalkPool {
-    int *spill;  // per-wave global stacks, gcap entries each
-    int gcap;
-    int *entries;  // saved stacks
-    int ecap;
-    WalkTask *tasks;  // gcount deferred groups, then tcount tasks
-    int32_t *ready;   // [WALK_MAX_TASKS] task published (cleared before the walk)
-    int gcount, tcount;  // 0: nothing is deferred
-    void *partial;    // one row of gs * (sums per target) per entry of tasks, in the walk's type
-    int budget, most0, div0, most, div;  // shares of a deferred group (task): stack >> div0 (div), at most most0 (most)
-
-    // the workspace behind the control block: the spill stacks of `waves` waves, then what deferral needs.
-    // row: bytes of one partial row
-    ptg_status carve(char *ws, size_t ws_bytes, int64_t waves, int gcap_, size_t row)
-    {
-        size_t at = ptg_align256(sizeof(WalkCtl));
-        auto take = [&](size_t bytes) {
-            char *p = ws + at;
-            at += ptg_align256(bytes);
-            return p;
-        };
-        ready = (int32_t *)take(WALK_MAX_TASKS * sizeof(int32_t));  // where the control block's clearing expects it
-        gcap = gcap_;
-        spill = (int *)take((size_t)waves * gcap * sizeof(int));
-        if (at > ws_bytes) {
-            ptg_set_error("ptg_walk: workspace too small (%zu < %zu)", ws_bytes, at);
-            return PTG_ERR_WORKSPACE;
-        }
-        const size_t left = ws_bytes - at;
-        const size_t ebytes = std::min<size_t>(left / 8 * 3, 48u << 20);
-        const size_t nrows = left > ebytes + 1024 ? (left - ebytes - 1024) / (row + sizeof(WalkTask)) : 0;
-        gcount = tcount = 0;
-        if (nrows >= 1024) {
-            ecap = (int)(ebytes / sizeof(int));
-            entries = (int *)take(ebytes);
-            tcount = (int)std::min<size_t>(WALK_MAX_TASKS, nrows / 8 * 7);
-            gcount = tcount / 8;
-            tasks = (WalkTask *)take((size_t)(gcount + tcount) * sizeof(WalkTask));
-            partial = take((size_t)(gcount + tcount) * row);
-        }
-        return PTG_OK;
+// the workspace behind the control block: the spill stacks of `waves` waves, then what deferral needs.
+// row: bytes of one partial row
+static ptg_status walk_carve(WalkPool &b, char *ws, size_t ws_bytes, int64_t waves, int gcap, size_t row)
+{
+    size_t at = ptg_align256(sizeof(WalkCtl));
+    auto take = [&](size_t bytes) {
+        char *p = ws + at;
+        at += ptg_align256(bytes);
+        return p;
+    };
+    b.ready = (int32_t *)take(WALK_MAX_TASKS * sizeof(int32_t));  // where the control block's clearing expects it
+    b.gcap = gcap;
+    b.spill = (int *)take((size_t)waves * gcap * sizeof(int));
+    if (at > ws_bytes) {
+        ptg_set_error("ptg_walk: workspace too small (%zu < %zu)", ws_bytes, at);
+        return PTG_ERR_WORKSPACE;
     }
-};
+    const size_t left = ws_bytes - at;
+    const size_t ebytes = std::min<size_t>(left / 8 * 3, 48u << 20);
+    const size_t nrows = left > ebytes + 1024 ? (left - ebytes - 1024) / (row + sizeof(WalkTask)) : 0;
+    b.gcount = b.tcount = 0;
+    if (nrows >= 1024) {
+        b.ecap = (int)(ebytes / sizeof(int));
+        b.entries = (int *)take(ebytes);
+        b.tcount = (int)std::min<size_t>(WALK_MAX_TASKS, nrows / 8 * 7);
+        b.gcount = b.tcount / 8;
+        b.tasks = (WalkTask *)take((size_t)(b.gcount + b.tcount) * sizeof(WalkTask));
+        b.partial = take((size_t)(b.gcount + b.tcount) * row);
+    }
+    return PTG_OK;
+}
 
 static inline size_t walk_control_bytes()
 {
@@ -234,15 +199,16 @@ __device__ __forceinline__ WalkSpan walk_span(const int32_t *goff, int gs, int64
     return WalkSpan{a0, (int)(b0 - a0), goff && e0 > b0};
 }
 
-// n entries of a table of cap counted by *counter: the first one's index, or -1 (one lane calls).  The
-// counter is added to once and never taken back: when thousands of waves reach their budgets together,
-// compare-and-swap loops on it took 27 ms.
-__device__ __forceinline__ int walk_take(int32_t *counter, int n, int cap)
-{
-    if (agent_load(counter) > cap - n) return -1;
-    const int at = atomicAdd(counter, n);
-    return at > cap - n ? -1 : at;
-}
+// the memory of the task pass (walk_tasks.hpp)
+struct AgentMem {
+    static constexpr int LANES = 64;
+    static __device__ __forceinline__ int32_t load(const int32_t *p) { return agent_load(p); }
+    static __device__ __forceinline__ void store(int32_t *p, int32_t v) { agent_store(p, v); }
+    static __device__ __forceinline__ int32_t add(int32_t *p, int32_t v) { return atomicAdd(p, v); }
+    static __device__ __forceinline__ int32_t sub(int32_t *p, int32_t v) { return atomicSub(p, v); }
+    static __device__ __forceinline__ bool cas(int32_t *p, int32_t is, int32_t v) { return atomicCAS(p, is, v) == is; }
+    static __device__ __forceinline__ void settle() { wave_stores_done(); }
+};
 
 // Cuts a traversal: takes room for its shares (gsp spilled entries below sp in LDS) and saves the stack.
 // `self` is the task's entry of tasks (a group's is taken here).  Returns the number of shares, 0 if
@@ -257,9 +223,9 @@ __device__ __forceinline__ int walk_cut(WalkCtl *ctl, const WalkPool &B, const i
     off = -1;
     if (lane == 0 && cnt <= nchild * SCAP) {
         // tasks last: one that was taken is published (a ticket would wait for it)
-        if (!TASKS) self = walk_take(&ctl->ngroup, 1, B.gcount);
-        off = self >= 0 ? walk_take(&ctl->npool, cnt, B.ecap) : -1;
-        child0 = off >= 0 ? walk_take(&ctl->ntask, nchild, B.tcount) : -1;
+        if (!TASKS) self = walk_take<AgentMem>(&ctl->ngroup, 1, B.gcount);
+        off = self >= 0 ? walk_take<AgentMem>(&ctl->npool, cnt, B.ecap) : -1;
+        child0 = off >= 0 ? walk_take<AgentMem>(&ctl->ntask, nchild, B.tcount) : -1;
         if (child0 < 0) off = -1;
         child0 += B.gcount;
     }
@@ -274,61 +240,18 @@ __device__ __forceinline__ int walk_cut(WalkCtl *ctl, const WalkPool &B, const i
     return nchild;
 }
 
-// after the row of `self` is stored: its record, then its shares' records, then their flags
-template <bool TASKS>
-__device__ __forceinline__ void walk_publish(WalkCtl *ctl, const WalkPool &B, int64_t g, int cnt, int nchild, int off,
-                                             int child0, int self, int lane)
+// The next task of the task pass (its entry of tasks), or -1 when none is open any more.  Block b is of
+// class b mod 8, as it runs on XCD b mod 8.  ticket, closed: the wave's (task_look), uniform.
+__device__ __forceinline__ int walk_ticket(WalkCtl *ctl, const WalkPool &B, int lane, int &ticket, int &closed)
 {
-    if (lane == 0) {
-        WalkTask *T = &B.tasks[self];
-        if (!TASKS) {
-            agent_store(&T->group, (int32_t)g);
-            agent_store(&T->parent, -1);
-        }
-        agent_store(&T->child0, child0);
-        agent_store(&T->nchild, nchild);
-        agent_store(&T->wait, nchild);
-        atomicAdd(&ctl->open, nchild);
-    }
-#pragma unroll 1
-    for (int q = lane; q < nchild; q += 64) {
-        WalkTask *T = &B.tasks[child0 + q];
-        agent_store(&T->group, (int32_t)g);
-        agent_store(&T->parent, self);
-        agent_store(&T->off, off + q);
-        agent_store(&T->stride, nchild);
-        agent_store(&T->count, (cnt - q + nchild - 1) / nchild);
-    }
-    wave_stores_done();
-#pragma unroll 1
-    for (int q = lane; q < nchild; q += 64) agent_store(&B.ready[child0 - B.gcount + q], 1);
-}
-
-// The next task of the task pass (its entry of tasks), or -1 when none is open any more.  Task t is drawn
-// by XCD t mod 8 (block b runs on XCD b mod 8; the grid holds blocks of each).  closed: tasks this wave has
-// finished since it last counted them off, which it does before it waits: a count per task on one word
-// would take milliseconds.
-__device__ __forceinline__ int walk_ticket(WalkCtl *ctl, const WalkPool &B, int lane, int &closed)
-{
-    const int x = blockIdx.x % NXCD;
-    int t = 0;
-    if (lane == 0) t = x + NXCD * atomicAdd(&ctl->ticket[x * CTR_STRIDE], 1);
-    t = __builtin_amdgcn_readfirstlane(t);
-    for (int polls = 0; polls < WALK_POLLS; polls++) {
-        int r = 0, d = 0;
-        if (lane == 0) {
-            if (t < B.tcount) r = agent_load(&B.ready[t]);
-            if (polls) d = agent_load(&ctl->done[(blockIdx.x % WALK_DONE) * 32]);
-        }
-        if (__builtin_amdgcn_readfirstlane(r)) return B.gcount + t;
-        if (__builtin_amdgcn_readfirstlane(d)) return -1;
-        if (closed) {
-            int o = 0;
-            if (lane == 0) o = atomicSub(&ctl->open, closed);
-            if (__builtin_amdgcn_readfirstlane(o) == closed && lane < WALK_DONE) agent_store(&ctl->done[lane * 32], 1);
-            closed = 0;
-        }
-        if (t >= B.tcount) return -1;  // all that there can be have been drawn
+    for (int looks = 0; looks < WALK_LOOKS; looks++) {
+        int t = TASK_NONE;
+        if (lane == 0)
+            t = task_look<AgentMem>(ctl, B, blockIdx.x % NXCD, blockIdx.x % WALK_DONE, looks, ticket, closed);
+        t = __builtin_amdgcn_readfirstlane(t);
+        ticket = __builtin_amdgcn_readfirstlane(ticket);
+        closed = __builtin_amdgcn_readfirstlane(closed);
+        if (t != TASK_NONE) return t == TASK_END ? -1 : B.gcount + t;
         __builtin_amdgcn_s_sleep(32);  // 0.9 us
     }
     if (lane == 0) atomicOr(&ctl->err, 8);
