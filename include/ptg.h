@@ -329,9 +329,10 @@ ptg_status ptg_walk_subtree(const ptg_walk_tree *wt, const int32_t *start_slot, 
 /* ptg_walk without a workspace, for callers that cannot allocate (code under HIP graph capture,
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  The same
  * kernels and results as ptg_walk; the walk control block and the per-wave spill stacks live in a
- * static device array of the library (177 MiB per GPU, held until the process ends: 4096 spill
+ * static device array of the library (133 MiB per GPU, held until the process ends: 4096 spill
  * entries per wave for the 5120 waves of a 256-CU grid, of which measured walks need at most 1344,
- * and 96 MiB for traversals that are cut and finished in shares).
+ * and 52 MiB for traversals that are cut and finished in shares; walks of more than 3.3e7 groups are
+ * not cut).
  * Nothing is allocated and nothing synchronises.  err (device int32, required) receives the
  * walk's flags instead of ptg_walk_check: 0 fine, bit 0 a traversal stack exceeded the spill
  * capacity, bit 1 a supplied group held more than group_size targets, bit 3 a share of a cut

@@ -520,7 +520,6 @@ __global__ __launch_bounds__(CD_THREADS) void k_column_binned(const ptg_tree_arr
 
 // ---- wavefront-per-group binned walk: k_walk64's traversal (walk64.hip) with six sums per target ----
 #define CB_GCAP 10240  // global spill entries per wave (a step leaves at most 448 a level of the 21 levels)
-#define CB_POOL (96u << 20)  // for the deferred traversals
 
 static int cb_cus()
 {
@@ -535,7 +534,7 @@ static int cb_cus()
 extern "C" size_t ptg_column_workspace_bytes(int64_t group_size)
 {
     (void)group_size;
-    return walk_control_bytes() + (size_t)cb_cus() * 3 * WALK_WAVES * CB_GCAP * sizeof(int) + CB_POOL;
+    return walk_control_bytes() + (size_t)cb_cus() * 3 * WALK_WAVES * CB_GCAP * sizeof(int) + WALK_POOL;
 }
 
 // the walk's flags as ptg_column_binned reports them
@@ -721,13 +720,13 @@ extern "C" ptg_status ptg_column_binned(const ptg_tree_arrays *tree, int64_t n, 
             return PTG_ERR_ARG;
         }
         WalkCtl *ctl = (WalkCtl *)ws;
-        st = walk_clear(ctl, s);
+        st = walk_clear(ctl, ptg_cdiv(nt, group_size), WALK_AGAIN, s);
         if (st) return st;
         const Walk64Args a{(const V4<double> *)wt->xyzm, (const V4<double> *)wt->aux, (const int2 *)wt->kids, nullptr,
                            targets, nullptr, nullptr, 1, wt->nslots, nt, ptg_cdiv(nt, group_size), nullptr, nullptr,
                            (int)group_size, theta, 1.0 / theta, 6.0 / (4.0 * 3.14159265358979323846), 0.0, 0.0, 0.0, 0,
                            nullptr, out, counters, ctl, nullptr};
-        st = ptg_walk64_bins(a, cb_cus(), CB_GCAP, (char *)ws, ws_bytes, s);
+        st = ptg_walk64_bins(a, cb_cus(), CB_GCAP, WALK_AGAIN, (char *)ws, ws_bytes, s);
         if (st) return st;
         k_column_err_out<<<1, 1, 0, s>>>(ctl, err);
         PTG_LAUNCH_CHECK();

@@ -429,7 +429,7 @@ enum { WHOLE, CUT, TASK };
 
 template <typename T, int TPL, int FIELDS, bool QUAD, bool EXP, int VAR, int PASS>
 __global__ __launch_bounds__(64 * WALK_WAVES) __attribute__((amdgpu_waves_per_eu(WalkOcc<T, TPL, VAR>::waves)))
-void k_walk(const WalkArgs<T> A, const WalkPool B)
+void k_walk(const WalkArgs<T> A, const WalkHot H, const WalkPool pool)
 {
     constexpr int LF = WalkOcc<T, TPL, VAR>::lf;
     constexpr bool TASKS = PASS == TASK;
@@ -450,28 +450,28 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
     __shared__ unsigned long long counts[WALK_WAVES][4];
     if (lane < 4) counts[wave][lane] = 0;
     __builtin_amdgcn_wave_barrier();
-    int *spill = B.spill + ((int64_t)blockIdx.x * WALK_WAVES + wave) * (int64_t)B.gcap;
+    int *spill = H.spill + ((int64_t)blockIdx.x * WALK_WAVES + wave) * (int64_t)H.gcap;
     const int xcd = blockIdx.x % NXCD;
     int ghw = 0;  // this wave's deepest spill
     const int64_t ngroups = A.goff ? (int64_t)__builtin_amdgcn_readfirstlane(*A.gcount) : A.ngroups;
 
     int ticket = -1, closed = 0;
+    if (!TASKS && blockIdx.x == 0 && threadIdx.x == 0) A.ctl->words = (int32_t)walk_words(ngroups);
     if (TASKS && agent_load(&A.ctl->open) == 0) return;  // nothing was deferred, or all of it is done
 
     for (int attempt = 0; attempt < (TASKS ? 1 : NXCD); attempt++) {
         const int x = (xcd + attempt) % NXCD;
         const int64_t g_lo = ngroups * x / NXCD, g_hi = ngroups * (x + 1) / NXCD;
         for (;;) {
-            int self = -1, t_off = 0, t_stride = 0, t_count = 0;
+            int self = -1, parent = -1;
             int64_t g;
+            TaskWords rec;  // the parent's
             if (TASKS) {
-                self = walk_ticket(A.ctl, B, lane, ticket, closed);
+                const WalkPool B = walk_pool<TASKS>(A.ctl, H, pool);
+                self = walk_ticket(A.ctl, B, lane, ticket, closed, parent);
                 if (self < 0) break;
-                const WalkTask *W = &B.tasks[self];
-                g = __builtin_amdgcn_readfirstlane(agent_load(&W->group));
-                t_off = __builtin_amdgcn_readfirstlane(agent_load(&W->off));
-                t_stride = __builtin_amdgcn_readfirstlane(agent_load(&W->stride));
-                t_count = __builtin_amdgcn_readfirstlane(agent_load(&W->count));
+                rec = TaskWords(&B.tasks[parent], lane);
+                g = rec.get<&WalkTask::group>();
             } else {
                 int gi = 0;
                 if (lane == 0) gi = atomicAdd(&A.ctl->ctr[x * CTR_STRIDE], 1);
@@ -560,9 +560,14 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
 
             int sp = 1, gsp = 0, nn = 0, np = 0;
             bool overflow = false, cut = false;
-            if (TASKS) {
-                sp = t_count;  // <= SCAP: deeper stacks are not deferred
-                for (int q = lane; q < sp; q += 64) L.stack[q] = agent_load(&B.entries[t_off + (int64_t)q * t_stride]);
+            const bool share = TASKS && rec.get<&WalkTask::off>() >= 0;  // else a group from its root
+            if (share) {
+                const WalkPool B = walk_pool<TASKS>(A.ctl, H, pool);
+                const int stride = rec.get<&WalkTask::nchild>(), q0 = self - B.gcount - rec.get<&WalkTask::child0>();
+                const int share_no = q0 < 0 ? q0 + B.tcount : q0;
+                const int *entries = B.entries + rec.get<&WalkTask::off>() + share_no;
+                sp = share_count(rec.get<&WalkTask::count>(), stride, share_no);  // <= SCAP: deeper stacks are not cut
+                for (int q = lane; q < sp; q += 64) L.stack[q] = agent_load(&entries[(int64_t)q * stride]);
             } else if (lane == 0) {
                 L.stack[0] = root;  // the root of system s occupies walk slot s
             }
@@ -576,18 +581,19 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
             // BUDGET; 2.2e6: 36 ms, 42 with BUDGET).  By the targets of the group's own system, so that a
             // system's cuts are those it has alone.
             int budget = 0x7fffffff;
-            if (PASS == TASK) {
-                budget = B.budget;
-            } else if (PASS == CUT) {
+            if (share) {
+                budget = H.budget;
+            } else if (PASS != WHOLE) {
                 const int64_t sg = (A.nsys > 0 ? A.soff[root + 1] - A.soff[root] : A.nt) / A.gs;
                 const float many = fmaxf(1.0f, (float)sg * (1.0f / 5120));
-                if (sg >= cut_groups(FIELDS)) budget = (int)fminf((float)B.budget * many * sqrtf(many), 2e9f);
+                if (sg >= cut_groups(FIELDS)) budget = (int)fminf((float)H.budget * many * sqrtf(many), 2e9f);
             }
-            int nchild = 0, off = 0, child0 = 0;
+            if (TASKS) budget = walk_budget(budget, rec.get<&WalkTask::level>());
+            int nchild = 0, off = 0, child0 = 0, troot = -1;
             // counts of this traversal: elements visited, listed, listed as particles; folded (per lane)
             int n_vis = 0, n_list = 0, n_part = 0, n_exp = 0;
 
-            for (;;) {  // once more only where a deferred traversal finds no room
+            for (;;) {  // once more only for a traversal that is not cut
                 for (;;) {
                     // pop up to 64 stack entries, one per lane, refilling the LDS stack from the spill
                     // region when it is empty
@@ -686,7 +692,7 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
                     if (sp + tot > SCAP) {
                         // move the bottom ks entries of the LDS stack to this wave's global region
                         const int ks = spill_count(sp, tot);
-                        if (gsp + ks > B.gcap) {
+                        if (gsp + ks > H.gcap) {
                             overflow = true;
                             break;
                         }
@@ -730,10 +736,22 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
                     }
                 }
                 if (PASS == WHOLE || !cut) break;
-                nchild = walk_cut<TASKS>(A.ctl, B, L.stack, sp, spill, gsp, lane, self, off, child0);
+                nchild = walk_cut<TASKS>(A.ctl, H, pool, share, L.stack, sp, spill, gsp, lane, self, off, child0);
                 cut = nchild > 0;
-                if (cut) break;
+                if (nchild) break;
                 budget = 0x7fffffff;
+            }
+            if (TASKS) troot = parent < walk_pool<TASKS>(A.ctl, H, pool).gcount ? parent : rec.get<&WalkTask::root>();
+            if (PASS != WHOLE && nchild < 0) {  // no room: the group is walked again
+                const WalkPool B = walk_pool<TASKS>(A.ctl, H, pool);
+                if (!TASKS) {
+                    if (lane == 0) walk_put_back<AgentMem>(A.ctl, B, false, (int)g);
+                    continue;
+                }
+                if (lane == 0) agent_store(&B.tasks[troot].root, 1);
+                walk_add_up<FIELDS, T>(A.ctl, B, parent, grp, A.gs, A.perm, A.G, A.out, lane);
+                closed++;
+                continue;
             }
             if (A.counters) {
                 if (EXP) {
@@ -741,10 +759,12 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
                     for (int d = 32; d >= 1; d >>= 1) n_exp += __shfl_xor(n_exp, d, 64);  // lanes fold separately
                 }
                 if (lane == 0) {
-                    counts[wave][0] += (unsigned long long)n_list * mt;
-                    counts[wave][1] += n_vis;
-                    counts[wave][2] += (unsigned long long)n_part * mt;
-                    if (EXP) counts[wave][3] += n_exp;
+                    const int64_t n[4] = {(int64_t)n_list * mt, n_vis, (int64_t)n_part * mt, n_exp};
+                    for (int q = 0; q < (EXP ? 4 : 3); q++) {
+                        if (PASS == CUT && cut) agent_store(&walk_pool<TASKS>(A.ctl, H, pool).counts[4 * self + q], n[q]);
+                        else if (TASKS) atomicAdd((unsigned long long *)&walk_pool<TASKS>(A.ctl, H, pool).counts[4 * troot + q], (unsigned long long)n[q]);
+                        else counts[wave][q] += (unsigned long long)n[q];
+                    }
                 }
             }
             if (overflow) {
@@ -764,6 +784,7 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
             // ---- G * fields in the caller's order, or the row of a deferred group or a task ----
             constexpr int W = NW<FIELDS>::W, WI = NW<FIELDS>::POT + 3 * NW<FIELDS>::ACC + 6 * NW<FIELDS>::TID;
             if (TASKS || cut) {
+                const WalkPool B = walk_pool<TASKS>(A.ctl, H, pool);
 #pragma unroll
                 for (int j = 0; j < TPL; j++) {
                     if (!tval[j]) continue;
@@ -785,10 +806,13 @@ void k_walk(const WalkArgs<T> A, const WalkPool B)
                     }
                 }
                 if (cut) {
-                    wave_stores_done();
-                    walk_publish<AgentMem>(A.ctl, B, TASKS, (int)g, gsp + sp, nchild, off, child0, self, lane);
+                    const WalkPool P = walk_pool<TASKS>(A.ctl, H, pool);
+                    walk_publish<AgentMem>(A.ctl, P, WalkTask{(int)g, parent, TASKS ? troot : 0, TASKS ? rec.get<&WalkTask::level>() : 0, off,
+                                                         gsp + sp, child0 % P.tcount, nchild, nchild, {}}, child0, self, lane);
                 } else {
-                    walk_add_up<FIELDS, T>(B, self, grp, A.gs, A.perm, A.G, A.out, lane);
+                    const int p = walk_add_up<FIELDS, T>(A.ctl, B, parent, grp, A.gs, A.perm, A.G, A.out, lane);
+                    if (p >= 0 && A.counters && lane < (EXP ? 4 : 3))
+                        counts[wave][lane] += (unsigned long long)agent_load(&B.counts[4 * p + lane]);
                 }
                 if (TASKS) closed++;
                 continue;
@@ -848,14 +872,17 @@ static int64_t walk_grid_blocks(int variant = -1)
     return (int64_t)num_cus() * per;
 }
 
-#define WALK_POOL (96u << 20)  // for the deferred traversals
+// bytes of the bits of a walk's groups, at most one per target
+static size_t walk_again_bytes(int64_t nt)
+{
+    return std::max<size_t>(WALK_AGAIN, walk_words(nt) * sizeof(int32_t));
+}
 
 extern "C" size_t ptg_walk_workspace_bytes(int64_t nt, int group_size)
 {
-    (void)nt;
     (void)group_size;
     size_t waves = (size_t)walk_grid_blocks() * WALK_WAVES;
-    return walk_control_bytes() + ptg_align256(waves * GCAP * sizeof(int)) + WALK_POOL;
+    return walk_control_bytes(walk_again_bytes(nt)) + ptg_align256(waves * GCAP * sizeof(int)) + WALK_POOL;
 }
 
 // ---- static scratch of ptg_walk_noalloc ----
@@ -866,7 +893,8 @@ extern "C" size_t ptg_walk_workspace_bytes(int64_t nt, int group_size)
 // overlap on one device (different streams) race.  Host code never passes the array's name to a
 // kernel (that is a host-side stand-in): it uses the address hipGetSymbolAddress returns, looked up
 // once per device with that device current and kept per device.
-#define NOALLOC_BYTES ((80u << 20) + (1u << 20) + WALK_POOL)  // 4096 spill entries per wave for 5120 resident waves
+// 4096 spill entries per wave for 5120 resident waves
+#define NOALLOC_BYTES ((80u << 20) + (1u << 20) + WALK_AGAIN + WALK_POOL)
 #define NOALLOC_MIN_GCAP 2048  // spill entries per wave the static scratch must leave
 #define NOALLOC_MAX_DEVICES 64
 static __device__ __align__(256) char scratch[NOALLOC_BYTES];
@@ -914,6 +942,7 @@ __global__ void k_walk_err_out(const WalkCtl *ctl, int32_t *err)
 struct WalkWs {  // a walk's workspace
     char *p;
     size_t bytes;
+    size_t again;  // bytes of the bits of the groups put back
     int gcap;  // global spill entries per wave (GCAP, or what the static scratch of ptg_walk_noalloc gives)
 };
 
@@ -932,23 +961,22 @@ static ptg_status launch_t(const WalkArgs<T> &a, int64_t max_blocks, const WalkW
     }
     const int64_t blocks = std::min<int64_t>(max_blocks, (int64_t)num_cus() * per_cu);
     constexpr int WI = NW<FIELDS>::POT + 3 * NW<FIELDS>::ACC + 6 * NW<FIELDS>::TID;
-    WalkPool b{};
+    WalkHot b{};
     const double open = a.theta < T(0.7) ? 0.49 / ((double)a.theta * a.theta) : 1.0;
     b.budget = (int)std::min(1e8, BUDGET * open * TPL);
     b.most0 = 16;
-    b.div0 = 4;
     b.most = 128;
-    b.div = 2;
-    ptg_status st = walk_carve(b, ws.p, ws.bytes, blocks * WALK_WAVES, ws.gcap, (size_t)a.gs * WI * sizeof(T));
+    ptg_status st = walk_carve(b, ws.p, ws.bytes, a.goff ? a.nt : a.ngroups, ws.again, blocks * WALK_WAVES, ws.gcap,
+                               (size_t)a.gs * WI * sizeof(T));
     if (st) return st;
     // a traversal visits a slot once, and no system has more targets than there are: where none can be
     // cut, the kernel without (its scalar registers do not spill; 2 to 7 % of the longest traversals)
     if (b.tcount == 0 || a.nslots <= b.budget || a.nt / a.gs < cut_groups(FIELDS)) {
-        k_walk<T, TPL, FIELDS, QUAD, EXP, VAR, WHOLE><<<(unsigned)blocks, 64 * WALK_WAVES, 0, s>>>(a, b);
+        k_walk<T, TPL, FIELDS, QUAD, EXP, VAR, WHOLE><<<(unsigned)blocks, 64 * WALK_WAVES, 0, s>>>(a, b, walk_pool(a.ctl, b));
     } else {
-        k_walk<T, TPL, FIELDS, QUAD, EXP, VAR, CUT><<<(unsigned)blocks, 64 * WALK_WAVES, 0, s>>>(a, b);
+        k_walk<T, TPL, FIELDS, QUAD, EXP, VAR, CUT><<<(unsigned)blocks, 64 * WALK_WAVES, 0, s>>>(a, b, walk_pool(a.ctl, b));
         PTG_LAUNCH_CHECK();
-        k_walk<T, TPL, FIELDS, QUAD, EXP, VAR, TASK><<<(unsigned)blocks, 64 * WALK_WAVES, 0, s>>>(a, b);
+        k_walk<T, TPL, FIELDS, QUAD, EXP, VAR, TASK><<<(unsigned)blocks, 64 * WALK_WAVES, 0, s>>>(a, b, walk_pool(a.ctl, b));
     }
     PTG_LAUNCH_CHECK();
     return PTG_OK;
@@ -1114,7 +1142,8 @@ static ptg_status walk_impl(const ptg_walk_tree *wt, const ptg_forest *forest, c
     const int64_t fn = forest ? forest->nsys : 0;
     const int64_t *fo = forest ? forest->offsets : nullptr;
     const double *fc = forest ? forest->cubes : nullptr;
-    ptg_status st = walk_clear(ctl, s);
+    const size_t again = noalloc ? WALK_AGAIN : walk_again_bytes(nt);
+    ptg_status st = walk_clear(ctl, group_offsets ? nt : ptg_cdiv(nt, group_size), again, s);
     if (st) return st;
     if (wt->prec == PTG_F32) {
         WalkArgs<float> a{(const V4<float> *)wt->xyzm, (const V4<float> *)wt->aux, (const int2 *)wt->kids,
@@ -1127,13 +1156,13 @@ static ptg_status walk_impl(const ptg_walk_tree *wt, const ptg_forest *forest, c
             ptg_set_error("ptg_walk: the exact branch set is evaluated in FP64; use prec=PTG_F64");
             return PTG_ERR_ARG;
         }
-        st = launch_walk<float>(a, fields, quadrupole != 0, expand, variant, blocks, WalkWs{(char *)ws, ws_bytes, gcap}, s);
+        st = launch_walk<float>(a, fields, quadrupole != 0, expand, variant, blocks, WalkWs{(char *)ws, ws_bytes, again, gcap}, s);
     } else if (wt->prec == PTG_F64) {
         Walk64Args a{(const V4<double> *)wt->xyzm, (const V4<double> *)wt->aux, (const int2 *)wt->kids,
                      (const double *)wt->quad, pos, soft, perm, targets_sorted != 0, wt->nslots, nt,
                      ptg_cdiv(nt, group_size), group_offsets, group_count, group_size, theta, 1.0 / theta, G,
                      wt->origin[0], wt->origin[1], wt->origin[2], fn, fo, out, counters, ctl, start_slot};
-        st = ptg_walk64_launch(a, fields, quadrupole != 0, num_cus(), gcap, (char *)ws, ws_bytes, s);
+        st = ptg_walk64_launch(a, fields, quadrupole != 0, num_cus(), gcap, again, (char *)ws, ws_bytes, s);
     } else {
         ptg_set_error("ptg_walk: prec must be PTG_F32 or PTG_F64");
         return PTG_ERR_ARG;

@@ -299,14 +299,16 @@ template <int FIELDS, typename F> __device__ __forceinline__ void each_sum(Acc<d
         f(a.tzz);
     }
 }
-// waves per SIMD the registers are capped for: four where the LDS lets four blocks onto a CU
+// waves per SIMD the registers are capped for: as many as the sums leave room for and the LDS lets onto a CU
 template <int TPL, int FIELDS, bool QUAD> struct Occ64 {
-    static constexpr int waves = FIELDS == BINS ? 3 : TPL == 1 && !QUAD && !NW<FIELDS>::TID ? 4 : 1;
+    static constexpr int sums = TPL * Sums<FIELDS>::WI;
+    static constexpr int waves = FIELDS == BINS ? 3 : !QUAD && TPL == 1 ? (sums <= 4 ? 4 : sums <= 9 ? 3 : 1)
+                                                 : sums >= 12 && sums <= 24 ? 2 : 1;
 };
 
 template <int TPL, int FIELDS, bool QUAD, bool TASKS>
 __global__ __launch_bounds__(64 * WALK_WAVES) __attribute__((amdgpu_waves_per_eu(Occ64<TPL, FIELDS, QUAD>::waves)))
-void k_walk64(const Walk64Args A, const WalkPool B)
+void k_walk64(const Walk64Args A, const WalkHot H, const WalkPool pool)
 {
     constexpr int WI = Sums<FIELDS>::WI;
     // entries evaluated together (nodes, particles).  Quadrupoles, three waves per SIMD, have the registers for 4
@@ -317,12 +319,13 @@ void k_walk64(const Walk64Args A, const WalkPool B)
     __shared__ Lds64<FIELDS, QUAD> lds[WALK_WAVES];
     const int wave = threadIdx.x >> 6, lane = ptg_lane();
     Lds64<FIELDS, QUAD> &L = lds[wave];
-    int *spill = B.spill + ((int64_t)blockIdx.x * WALK_WAVES + wave) * (int64_t)B.gcap;
+    int *spill = H.spill + ((int64_t)blockIdx.x * WALK_WAVES + wave) * (int64_t)H.gcap;
     const int xcd = blockIdx.x % NXCD;
-    int64_t n_int = 0, n_vis = 0, n_part = 0;
+    int64_t total[3] = {0, 0, 0};  // interactions, visits, particle interactions of the groups this wave finished
     int ghw = 0;
     const int64_t ngroups = A.goff ? (int64_t)__builtin_amdgcn_readfirstlane(*A.gcount) : A.ngroups;
     int ticket = -1, closed = 0;
+    if (!TASKS && blockIdx.x == 0 && threadIdx.x == 0) A.ctl->words = (int32_t)walk_words(ngroups);
     if (TASKS && agent_load(&A.ctl->open) == 0) return;  // nothing was deferred, or all of it is done
     // targets per slice, a power of two
     int P = 64;
@@ -335,16 +338,15 @@ void k_walk64(const Walk64Args A, const WalkPool B)
         const int x = (xcd + attempt) % NXCD;
         const int64_t w_lo = ngroups * x / NXCD, w_hi = ngroups * (x + 1) / NXCD;
         for (;;) {
-            int self = -1, t_off = 0, t_stride = 0, t_count = 0;
+            int self = -1, parent = -1;
             int64_t g;
+            TaskWords rec;  // the parent's
             if (TASKS) {
-                self = walk_ticket(A.ctl, B, lane, ticket, closed);
+                const WalkPool B = walk_pool<TASKS>(A.ctl, H, pool);
+                self = walk_ticket(A.ctl, B, lane, ticket, closed, parent);
                 if (self < 0) break;
-                const WalkTask *T = &B.tasks[self];
-                g = __builtin_amdgcn_readfirstlane(agent_load(&T->group));
-                t_off = __builtin_amdgcn_readfirstlane(agent_load(&T->off));
-                t_stride = __builtin_amdgcn_readfirstlane(agent_load(&T->stride));
-                t_count = __builtin_amdgcn_readfirstlane(agent_load(&T->count));
+                rec = TaskWords(&B.tasks[parent], lane);
+                g = rec.get<&WalkTask::group>();
             } else {
                 int wi = 0;
                 if (lane == 0) wi = atomicAdd(&A.ctl->ctr[x * CTR_STRIDE], 1);
@@ -409,11 +411,16 @@ void k_walk64(const Walk64Args A, const WalkPool B)
             if (FIELDS == BINS)
                 for (int q = 0; q < 6; q++) L.bins[64 * q + lane] = 0.0;
 
-            int sp = 1, gsp = 0, nn = 0, np = 0, visits = 0;
+            int sp = 1, gsp = 0, nn = 0, np = 0, visits = 0, n_list = 0, n_part = 0;
             bool overflow = false;
-            if (TASKS) {
-                sp = t_count;  // <= SCAP: deeper stacks are not deferred
-                for (int q = lane; q < sp; q += 64) L.stack[q] = agent_load(&B.entries[t_off + (int64_t)q * t_stride]);
+            const bool share = TASKS && rec.get<&WalkTask::off>() >= 0;  // else a group from its root
+            if (share) {
+                const WalkPool B = walk_pool<TASKS>(A.ctl, H, pool);
+                const int stride = rec.get<&WalkTask::nchild>(), q0 = self - B.gcount - rec.get<&WalkTask::child0>();
+                const int share_no = q0 < 0 ? q0 + B.tcount : q0;
+                const int *entries = B.entries + rec.get<&WalkTask::off>() + share_no;
+                sp = share_count(rec.get<&WalkTask::count>(), stride, share_no);  // <= SCAP: deeper stacks are not cut
+                for (int q = lane; q < sp; q += 64) L.stack[q] = agent_load(&entries[(int64_t)q * stride]);
             } else {
                 // the root of system s occupies walk slot s; a subtree walk starts at its element's slot
                 // instead (wave-uniform; an out-of-range slot is reported, and dropped when popped like
@@ -431,12 +438,13 @@ void k_walk64(const Walk64Args A, const WalkPool B)
             // against 3 times 3072 6.8 / 8.3 ms (clumpy 6e5).  Counted per system, so that a system's cuts
             // are those it has alone.
             const int64_t sg = (A.nsys > 0 ? A.soff[root + 1] - A.soff[root] : A.nt) / A.gs;
-            int budget = B.budget * (TASKS || sg <= 16384 ? 1 : sg <= 65536 ? 2 : sg <= 262144 ? 4 : 16);
-            if (B.tcount == 0) budget = 0x7fffffff;
+            int budget = H.budget * (share || sg <= 16384 ? 1 : sg <= 65536 ? 2 : sg <= 262144 ? 4 : 16);
+            if (TASKS) budget = walk_budget(budget, rec.get<&WalkTask::level>());
+            if (H.tcount == 0) budget = 0x7fffffff;
             bool cut = false;
-            int nchild = 0, off = 0, child0 = 0;
+            int nchild = 0, off = 0, child0 = 0, troot = -1;
 
-            for (;;) {  // once more only where a deferred traversal finds no room
+            for (;;) {  // once more only for a traversal that is not cut
                 for (;;) {
                     if (sp == 0) {
                         if (gsp == 0) break;
@@ -500,8 +508,8 @@ void k_walk64(const Walk64Args A, const WalkPool B)
                     np += (int)__popcll(bp);
                     nn += (int)__popcll(bn);
                     if (A.counters) {
-                        n_int += (int64_t)(__popcll(bp) + __popcll(bn)) * mt;
-                        n_part += (int64_t)(__popcll(bp) + __popcll(ptg_ballot(far_part))) * mt;
+                        n_list += (int)(__popcll(bp) + __popcll(bn));
+                        n_part += (int)(__popcll(bp) + __popcll(ptg_ballot(far_part)));
                     }
 
                     const int cnt = open ? std::min(std::max(K.y, 0), 8) : 0;
@@ -509,7 +517,7 @@ void k_walk64(const Walk64Args A, const WalkPool B)
                     const int below = small_excl_scan(cnt, tot);
                     if (sp + tot > SCAP) {
                         const int ks = spill_count(sp, tot);
-                        if (gsp + ks > B.gcap) {
+                        if (gsp + ks > H.gcap) {
                             overflow = true;
                             break;
                         }
@@ -560,12 +568,33 @@ void k_walk64(const Walk64Args A, const WalkPool B)
                     }
                 }
                 if (!cut) break;
-                nchild = walk_cut<TASKS>(A.ctl, B, L.stack, sp, spill, gsp, lane, self, off, child0);
+                nchild = walk_cut<TASKS>(A.ctl, H, pool, share, L.stack, sp, spill, gsp, lane, self, off, child0);
                 cut = nchild > 0;
-                if (cut) break;
+                if (nchild) break;
                 budget = 0x7fffffff;
             }
-            n_vis += visits;
+            if (TASKS) troot = parent < walk_pool<TASKS>(A.ctl, H, pool).gcount ? parent : rec.get<&WalkTask::root>();
+            if (nchild < 0) {  // no room: the group is walked again
+                const WalkPool B = walk_pool<TASKS>(A.ctl, H, pool);
+                if (!TASKS) {
+                    if (lane == 0) walk_put_back<AgentMem>(A.ctl, B, false, (int)g);
+                    continue;
+                }
+                if (lane == 0) agent_store(&B.tasks[troot].root, 1);
+                walk_add_up<FIELDS, double>(A.ctl, B, parent, grp, A.gs, A.perm, A.G, A.out, lane);
+                closed++;
+                continue;
+            }
+            if (A.counters) {
+                const int64_t n[3] = {(int64_t)n_list * mt, visits, (int64_t)n_part * mt};
+#pragma unroll
+                for (int q = 0; q < 3; q++) {
+                    if (!TASKS && !cut) total[q] += n[q];
+                    else if (lane != 0) continue;
+                    else if (TASKS) atomicAdd((unsigned long long *)&walk_pool<TASKS>(A.ctl, H, pool).counts[4 * troot + q], (unsigned long long)n[q]);
+                    else agent_store(&walk_pool<TASKS>(A.ctl, H, pool).counts[4 * self + q], n[q]);
+                }
+            }
             if (overflow) {
                 if (lane == 0) atomicOr(&A.ctl->err, 1);
                 nn = np = 0;  // a task's row is still written: the sums read every task's
@@ -609,7 +638,7 @@ void k_walk64(const Walk64Args A, const WalkPool B)
                         for (int q = 0; q < 6; q++) o[q] = A.G * bin[q];
                     }
                 } else {
-                    double *o = (double *)B.partial + ((int64_t)self * A.gs + tl + 64 * j) * WI;
+                    double *o = (double *)walk_pool<TASKS>(A.ctl, H, pool).partial + ((int64_t)self * A.gs + tl + 64 * j) * WI;
                     each_sum<FIELDS>(acc[j], [&](double &v) { agent_store(&o[c++], v); });
                     if constexpr (FIELDS == BINS) {
 #pragma unroll
@@ -618,19 +647,27 @@ void k_walk64(const Walk64Args A, const WalkPool B)
                 }
             }
             if (cut) {
-                wave_stores_done();
-                walk_publish<AgentMem>(A.ctl, B, TASKS, (int)g, gsp + sp, nchild, off, child0, self, lane);
+                const WalkPool P = walk_pool<TASKS>(A.ctl, H, pool);
+                walk_publish<AgentMem>(A.ctl, P, WalkTask{(int)g, parent, TASKS ? troot : 0, TASKS ? rec.get<&WalkTask::level>() : 0, off,
+                                                     gsp + sp, child0 % P.tcount, nchild, nchild, {}}, child0, self, lane);
             } else if (TASKS) {
-                walk_add_up<FIELDS, double>(B, self, grp, A.gs, A.perm, A.G, A.out, lane);
+                const WalkPool B = walk_pool<TASKS>(A.ctl, H, pool);
+                const int p = walk_add_up<FIELDS, double>(A.ctl, B, parent, grp, A.gs, A.perm, A.G, A.out, lane);
+                if (p >= 0 && A.counters)
+#pragma unroll
+                    for (int q = 0; q < 3; q++) {
+                        const int64_t n = agent_load(&walk_pool<TASKS>(A.ctl, H, pool).counts[4 * p + q]);
+                        total[q] += (int64_t)__builtin_amdgcn_readfirstlane((int)(n >> 32)) << 32 |
+                                    (uint32_t)__builtin_amdgcn_readfirstlane((int)n);
+                    }
             }
             if (TASKS) closed++;
         }
     }
     if (lane == 0 && ghw > 0) atomicMax(&A.ctl->hwm, ghw);
     if (lane == 0 && A.counters) {
-        atomicAdd((unsigned long long *)&A.counters[0], (unsigned long long)n_int);
-        atomicAdd((unsigned long long *)&A.counters[1], (unsigned long long)n_vis);
-        if (FIELDS != BINS) atomicAdd((unsigned long long *)&A.counters[2], (unsigned long long)n_part);
+        for (int q = 0; q < (FIELDS == BINS ? 2 : 3); q++)
+            atomicAdd((unsigned long long *)&A.counters[q], (unsigned long long)total[q]);
     }
 }
 
@@ -638,7 +675,7 @@ void k_walk64(const Walk64Args A, const WalkPool B)
 // host side
 // ============================================================================================
 template <int TPL, int FIELDS, bool QUAD>
-static ptg_status launch(const Walk64Args &a, int cus, int gcap, char *ws, size_t ws_bytes, hipStream_t s)
+static ptg_status launch(const Walk64Args &a, int cus, int gcap, size_t again, char *ws, size_t ws_bytes, hipStream_t s)
 {
     static int per_cu = 0;
     if (per_cu == 0) {
@@ -654,33 +691,31 @@ static ptg_status launch(const Walk64Args &a, int cus, int gcap, char *ws, size_
     const size_t row = (size_t)a.gs * Sums<FIELDS>::WI * sizeof(double);
     const double open = a.theta < 0.7 ? 0.49 / (a.theta * a.theta) : 1.0;
     const int share = (int)std::max<size_t>(16, 262144 / row);
-    WalkPool b{};
+    WalkHot b{};
     b.budget = (int)std::min(1e8, BUDGET * open * (a.gs <= 16 ? 1 : a.gs <= 64 ? 2 : 4));
     b.most0 = std::min(64, share);
-    b.div0 = 4;
     b.most = std::min(128, share);
-    b.div = 2;
     const int64_t blocks = (int64_t)cus * per_cu;
-    const ptg_status st = walk_carve(b, ws, ws_bytes, blocks * WALK_WAVES, gcap, row);
+    const ptg_status st = walk_carve(b, ws, ws_bytes, a.goff ? a.nt : a.ngroups, again, blocks * WALK_WAVES, gcap, row);
     if (st) return st;
     const int64_t nb = a.goff ? blocks : std::min(blocks, ptg_cdiv(a.ngroups, WALK_WAVES));
-    k_walk64<TPL, FIELDS, QUAD, false><<<(unsigned)nb, 64 * WALK_WAVES, 0, s>>>(a, b);
+    k_walk64<TPL, FIELDS, QUAD, false><<<(unsigned)nb, 64 * WALK_WAVES, 0, s>>>(a, b, walk_pool(a.ctl, b));
     PTG_LAUNCH_CHECK();
     if (b.tcount && a.nslots > b.budget) {  // a traversal visits a slot once
-        k_walk64<TPL, FIELDS, QUAD, true><<<(unsigned)blocks, 64 * WALK_WAVES, 0, s>>>(a, b);
+        k_walk64<TPL, FIELDS, QUAD, true><<<(unsigned)blocks, 64 * WALK_WAVES, 0, s>>>(a, b, walk_pool(a.ctl, b));
         PTG_LAUNCH_CHECK();
     }
     return PTG_OK;
 }
 
 template <int TPL>
-static ptg_status launch_fields(const Walk64Args &a, int fields, bool quad, int cus, int gcap, char *ws, size_t ws_bytes,
+static ptg_status launch_fields(const Walk64Args &a, int fields, bool quad, int cus, int gcap, size_t again, char *ws, size_t ws_bytes,
                                 hipStream_t s)
 {
 #define PTG_F(F)                                                             \
     case F:                                                                  \
-        return quad ? launch<TPL, F, true>(a, cus, gcap, ws, ws_bytes, s)    \
-                    : launch<TPL, F, false>(a, cus, gcap, ws, ws_bytes, s);
+        return quad ? launch<TPL, F, true>(a, cus, gcap, again, ws, ws_bytes, s)    \
+                    : launch<TPL, F, false>(a, cus, gcap, again, ws, ws_bytes, s);
     switch (fields) {
         PTG_F(1) PTG_F(2) PTG_F(3) PTG_F(4) PTG_F(5) PTG_F(6) PTG_F(7)
     }
@@ -689,15 +724,15 @@ static ptg_status launch_fields(const Walk64Args &a, int fields, bool quad, int 
     return PTG_ERR_ARG;
 }
 
-ptg_status ptg_walk64_launch(const Walk64Args &a, int fields, bool quad, int cus, int gcap, char *ws, size_t ws_bytes,
+ptg_status ptg_walk64_launch(const Walk64Args &a, int fields, bool quad, int cus, int gcap, size_t again, char *ws, size_t ws_bytes,
                              hipStream_t s)
 {
-    if (a.gs <= 64) return launch_fields<1>(a, fields, quad, cus, gcap, ws, ws_bytes, s);
-    if (a.gs <= 128) return launch_fields<2>(a, fields, quad, cus, gcap, ws, ws_bytes, s);
-    return launch_fields<4>(a, fields, quad, cus, gcap, ws, ws_bytes, s);
+    if (a.gs <= 64) return launch_fields<1>(a, fields, quad, cus, gcap, again, ws, ws_bytes, s);
+    if (a.gs <= 128) return launch_fields<2>(a, fields, quad, cus, gcap, again, ws, ws_bytes, s);
+    return launch_fields<4>(a, fields, quad, cus, gcap, again, ws, ws_bytes, s);
 }
 
-ptg_status ptg_walk64_bins(const Walk64Args &a, int cus, int gcap, char *ws, size_t ws_bytes, hipStream_t s)
+ptg_status ptg_walk64_bins(const Walk64Args &a, int cus, int gcap, size_t again, char *ws, size_t ws_bytes, hipStream_t s)
 {
-    return launch<1, BINS, false>(a, cus, gcap, ws, ws_bytes, s);
+    return launch<1, BINS, false>(a, cus, gcap, again, ws, ws_bytes, s);
 }

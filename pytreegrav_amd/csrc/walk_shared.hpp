@@ -109,9 +109,8 @@ template <int FIELDS> __device__ __forceinline__ void store_sum(double *o, int c
 // the sums it has (a row) and saves its stack as interleaved shares, tasks of a second launch.  There the
 // waves draw tickets for the tasks; a task past the budget is cut again, its shares published for the
 // waves that wait, and whoever finishes the last share of a task or group adds the shares' rows to it in
-// their order.  Where a traversal is cut depends on the group alone, so results do not depend on
-// scheduling or on what else is walked (unless the tables fill up: then the rest is walked in place, the
-// same terms summed in another order).
+// their order.  Where a traversal is cut depends on the group alone, also where the tables fill up
+// (walk_tasks.hpp), so results do not depend on scheduling or on what else is walked.
 //
 // The second launch costs 3 us where nothing was deferred; a launch per generation of tasks and one per
 // level of sums cost 30.  Its waves end when no task is open; which wave walks which task is in
@@ -119,52 +118,91 @@ template <int FIELDS> __device__ __forceinline__ void store_sum(double *o, int c
 // through agent-scope accesses, ordered by the writer's wait before it publishes or counts down.
 #define WALK_LOOKS (1 << 26)  // a wave gives up after a minute without a task and reports it
 
-// the workspace behind the control block: the spill stacks of `waves` waves, then what deferral needs.
-// row: bytes of one partial row
-static ptg_status walk_carve(WalkPool &b, char *ws, size_t ws_bytes, int64_t waves, int gcap, size_t row)
+// The workspace: the control block, the flags of the task slots and the bits of the groups put back (these
+// cleared before each walk), the spill stacks of the waves, and WALK_POOL bytes for what deferral needs.  The
+// tables are sized by the row alone, so that what fits does not depend on the call.
+#define WALK_AGAIN (4u << 20)  // bytes of the bits: 3.4e7 groups
+#define WALK_POOL (48u << 20)  // the listed and drawn cases use at most a third
+#define WALK_ENTRIES (WALK_POOL / 4)
+#define WALK_COUNTS (WALK_MAX_TASKS / 8 * 4 * sizeof(int64_t))
+
+// words of the bits of `groups` groups
+static __host__ __device__ __forceinline__ int64_t walk_words(int64_t groups) { return (groups + 255) / 256 * 8; }
+
+static constexpr size_t walk_align(size_t x) { return (x + 255) & ~(size_t)255; }
+#define WALK_READY_AT walk_align(sizeof(WalkCtl))
+#define WALK_AGAIN_AT (WALK_READY_AT + walk_align(WALK_MAX_TASKS * sizeof(int64_t)))
+
+static inline size_t walk_control_bytes(size_t again = WALK_AGAIN) { return WALK_AGAIN_AT + walk_align(again); }
+
+// A walk's workspace as its kernels take it: few words, since they are held in scalar registers through the
+// traversal.  The tables behind it are found where they are needed (walk_pool).
+struct WalkHot {
+    int *spill;  // per-wave global stacks, gcap entries each
+    int gcap;
+    int budget;       // of visits, before a traversal is cut
+    int most0, most;  // shares of a deferred group: stack >> WALK_DIV0, at most most0; of a task: >> WALK_DIV, most
+    int tcount;       // slots of the task table, 8 per entry for groups (0: nothing is deferred)
+    uint32_t pool_at;  // of the tables, from the control block, in units of 256 bytes
+};
+#define WALK_DIV0 4
+#define WALK_DIV 2
+
+static __host__ __device__ __forceinline__ WalkPool walk_pool(WalkCtl *ctl, const WalkHot &h)
 {
-    size_t at = ptg_align256(sizeof(WalkCtl));
-    auto take = [&](size_t bytes) {
-        char *p = ws + at;
-        at += ptg_align256(bytes);
-        return p;
-    };
-    b.ready = (int32_t *)take(WALK_MAX_TASKS * sizeof(int32_t));  // where the control block's clearing expects it
-    b.gcap = gcap;
-    b.spill = (int *)take((size_t)waves * gcap * sizeof(int));
-    if (at > ws_bytes) {
-        ptg_set_error("ptg_walk: workspace too small (%zu < %zu)", ws_bytes, at);
+    char *ws = (char *)ctl, *p = ws + (size_t)h.pool_at * 256;
+    WalkPool b;
+    b.ready = (int64_t *)(ws + WALK_READY_AT);
+    b.again = (int32_t *)(ws + WALK_AGAIN_AT);
+    b.entries = (int *)p;
+    b.ecap = (int)(WALK_ENTRIES / sizeof(int));
+    b.counts = (int64_t *)(p + WALK_ENTRIES);
+    b.tasks = (WalkTask *)(p + WALK_ENTRIES + WALK_COUNTS);
+    b.tcount = h.tcount;
+    b.gcount = h.tcount / 8;
+    b.partial = p + WALK_ENTRIES + WALK_COUNTS + walk_align((size_t)(b.gcount + b.tcount) * sizeof(WalkTask));
+    return b;
+}
+// The pool within a walk: the barrier keeps the addresses where they are used, moved out of the traversal they are
+// scalar registers again.  The task pass, which uses them between any two traversals, takes them as an argument.
+template <bool TASKS>
+__device__ __forceinline__ WalkPool walk_pool(WalkCtl *ctl, const WalkHot &h, const WalkPool &arg)
+{
+    if (TASKS) return arg;
+    asm volatile("" : "+s"(ctl));
+    return walk_pool(ctl, h);
+}
+
+// groups: at most, again: bytes of their bits (too few: nothing is deferred), gcap: spill entries per wave,
+// row: bytes of one partial row
+static ptg_status walk_carve(WalkHot &h, char *ws, size_t ws_bytes, int64_t groups, size_t again, int64_t waves, int gcap,
+                             size_t row)
+{
+    const size_t spill_at = walk_control_bytes(again), at = spill_at + walk_align((size_t)waves * gcap * sizeof(int));
+    if (at + WALK_POOL > ws_bytes) {
+        ptg_set_error("ptg_walk: workspace too small (%zu < %zu)", ws_bytes, at + WALK_POOL);
         return PTG_ERR_WORKSPACE;
     }
-    const size_t left = ws_bytes - at;
-    const size_t ebytes = std::min<size_t>(left / 8 * 3, 48u << 20);
-    const size_t nrows = left > ebytes + 1024 ? (left - ebytes - 1024) / (row + sizeof(WalkTask)) : 0;
-    b.gcount = b.tcount = 0;
-    if (nrows >= 1024) {
-        b.ecap = (int)(ebytes / sizeof(int));
-        b.entries = (int *)take(ebytes);
-        b.tcount = (int)std::min<size_t>(WALK_MAX_TASKS, nrows / 8 * 7);
-        b.gcount = b.tcount / 8;
-        b.tasks = (WalkTask *)take((size_t)(b.gcount + b.tcount) * sizeof(WalkTask));
-        b.partial = take((size_t)(b.gcount + b.tcount) * row);
-    }
+    h.spill = (int *)(ws + spill_at);
+    h.gcap = gcap;
+    h.pool_at = (uint32_t)(at / 256);
+    const int64_t left = WALK_POOL - WALK_ENTRIES - WALK_COUNTS - 256, nine = 9 * (int64_t)(row + sizeof(WalkTask));
+    h.tcount = 8 * (int)std::min<int64_t>(WALK_MAX_TASKS / 8, left / nine);
+    if (walk_words(groups) * (int64_t)sizeof(int32_t) > (int64_t)again) h.tcount = 0;
     return PTG_OK;
 }
 
-static inline size_t walk_control_bytes()
+// clears the control block, the task flags and the bits of the groups: n int4
+__global__ static void k_walk_init(int4 *ws, int64_t n)
 {
-    return ptg_align256(sizeof(WalkCtl)) + ptg_align256(WALK_MAX_TASKS * sizeof(int32_t));
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        ws[i] = int4{0, 0, 0, 0};
 }
-
-// clears the control block and the task flags behind it
-__global__ static void k_walk_init(int4 *ws, int n)
+static inline ptg_status walk_clear(void *ws, int64_t groups, size_t again, hipStream_t s)
 {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) ws[i] = int4{0, 0, 0, 0};
-}
-static inline ptg_status walk_clear(void *ws, hipStream_t s)
-{
-    const int n = (int)(walk_control_bytes() / sizeof(int4));
-    k_walk_init<<<(n + 1023) / 1024, 256, 0, s>>>((int4 *)ws, n);
+    const size_t bits = std::min<size_t>(again, walk_words(groups) * sizeof(int32_t));
+    const int64_t n = (int64_t)((WALK_AGAIN_AT + bits) / sizeof(int4));
+    k_walk_init<<<(unsigned)std::min<int64_t>(2048, (n + 1023) / 1024), 256, 0, s>>>((int4 *)ws, n);
     PTG_LAUNCH_CHECK();
     return PTG_OK;
 }
@@ -207,32 +245,41 @@ struct AgentMem {
     static __device__ __forceinline__ int32_t add(int32_t *p, int32_t v) { return atomicAdd(p, v); }
     static __device__ __forceinline__ int32_t sub(int32_t *p, int32_t v) { return atomicSub(p, v); }
     static __device__ __forceinline__ bool cas(int32_t *p, int32_t is, int32_t v) { return atomicCAS(p, is, v) == is; }
+    static __device__ __forceinline__ void max(int32_t *p, int32_t v) { atomicMax(p, v); }
+    static __device__ __forceinline__ void set(int32_t *p, int32_t bits) { atomicOr(p, bits); }
+    static __device__ __forceinline__ int64_t load(const int64_t *p) { return agent_load(p); }
+    static __device__ __forceinline__ void store(int64_t *p, int64_t v) { agent_store(p, v); }
+    // one store of the wave
+    static __device__ __forceinline__ void record(WalkTask *p, const WalkTask &T, int lane)
+    {
+        const int32_t v[WALK_TASK_WORDS] = {T.group, T.parent, T.root, T.level, T.off, T.count, T.child0, T.nchild, T.wait};
+        int32_t w = v[0];
+#pragma unroll
+        for (int i = 1; i < WALK_TASK_WORDS; i++) w = lane == i ? v[i] : w;
+        if (lane < WALK_TASK_WORDS) agent_store((int32_t *)p + lane, w);
+    }
     static __device__ __forceinline__ void settle() { wave_stores_done(); }
 };
 
 // Cuts a traversal: takes room for its shares (gsp spilled entries below sp in LDS) and saves the stack.
-// `self` is the task's entry of tasks (a group's is taken here).  Returns the number of shares, 0 if
-// there is no room (the wave goes on); the row is stored next, then walk_publish makes the shares tasks.
+// share: as a share of a group is cut, not as a group.  `self` is the task's entry of tasks (a group's is taken
+// here where it is negative).  Returns the number of shares, 0 if the traversal is one that is not cut, -1 if
+// there is no room; the row is stored next, then walk_publish makes the shares tasks.
 template <bool TASKS>
-__device__ __forceinline__ int walk_cut(WalkCtl *ctl, const WalkPool &B, const int *stack, int sp, const int *spill,
-                                        int gsp, int lane, int &self, int &off, int &child0)
+__device__ __forceinline__ int walk_cut(WalkCtl *ctl, const WalkHot &h, const WalkPool &arg, bool share, const int *stack, int sp,
+                                        const int *spill, int gsp, int lane, int &self, int &off, int &child0)
 {
+    const WalkPool B = walk_pool<TASKS>(ctl, h, arg);
     const int cnt = gsp + sp;
-    const int most = TASKS ? B.most : B.most0, part = cnt >> (TASKS ? B.div : B.div0);
+    const int most = share ? h.most : h.most0, part = cnt >> (share ? WALK_DIV : WALK_DIV0);
     const int nchild = part > most ? most : part < 1 ? 1 : part;
-    off = -1;
-    if (lane == 0 && cnt <= nchild * SCAP) {
-        // tasks last: one that was taken is published (a ticket would wait for it)
-        if (!TASKS) self = walk_take<AgentMem>(&ctl->ngroup, 1, B.gcount);
-        off = self >= 0 ? walk_take<AgentMem>(&ctl->npool, cnt, B.ecap) : -1;
-        child0 = off >= 0 ? walk_take<AgentMem>(&ctl->ntask, nchild, B.tcount) : -1;
-        if (child0 < 0) off = -1;
-        child0 += B.gcount;
-    }
+    if (cnt > nchild * SCAP) return 0;
+    int room = 0;
+    if (lane == 0) room = walk_room<AgentMem>(ctl, B, cnt, nchild, self, off, child0);
+    if (!__builtin_amdgcn_readfirstlane(room)) return -1;
     self = __builtin_amdgcn_readfirstlane(self);
     off = __builtin_amdgcn_readfirstlane(off);
     child0 = __builtin_amdgcn_readfirstlane(child0);
-    if (off < 0) return 0;
 #pragma unroll 1
     for (int q = lane; q < gsp; q += 64) agent_store(&B.entries[off + q], spill[q]);
 #pragma unroll 1
@@ -240,15 +287,22 @@ __device__ __forceinline__ int walk_cut(WalkCtl *ctl, const WalkPool &B, const i
     return nchild;
 }
 
+// a budget of visits at a level
+__device__ __forceinline__ int walk_budget(int budget, int level)
+{
+    return level == 0 ? budget : level < 8 && budget < 0x7fffffff >> 3 * level ? budget << 3 * level : 0x7fffffff;
+}
+
 // The next task of the task pass (its entry of tasks), or -1 when none is open any more.  Block b is of
 // class b mod 8, as it runs on XCD b mod 8.  ticket, closed: the wave's (task_look), uniform.
-__device__ __forceinline__ int walk_ticket(WalkCtl *ctl, const WalkPool &B, int lane, int &ticket, int &closed)
+__device__ __forceinline__ int walk_ticket(WalkCtl *ctl, const WalkPool &B, int lane, int &ticket, int &closed, int &parent)
 {
     for (int looks = 0; looks < WALK_LOOKS; looks++) {
         int t = TASK_NONE;
         if (lane == 0)
-            t = task_look<AgentMem>(ctl, B, blockIdx.x % NXCD, blockIdx.x % WALK_DONE, looks, ticket, closed);
+            t = task_look<AgentMem>(ctl, B, blockIdx.x % NXCD, blockIdx.x % WALK_DONE, looks, ticket, closed, parent);
         t = __builtin_amdgcn_readfirstlane(t);
+        parent = __builtin_amdgcn_readfirstlane(parent);
         ticket = __builtin_amdgcn_readfirstlane(ticket);
         closed = __builtin_amdgcn_readfirstlane(closed);
         if (t != TASK_NONE) return t == TASK_END ? -1 : B.gcount + t;
@@ -258,11 +312,26 @@ __device__ __forceinline__ int walk_ticket(WalkCtl *ctl, const WalkPool &B, int 
     return -1;
 }
 
-// the row of task `self` is stored: counts its parent's shares down; the last share's wave adds them up,
-// and so on up to the group, whose total is the result
+// a record of the task table in the wave's lanes: one load, where a load per field waited for each in turn
+struct TaskWords {
+    int32_t word = 0;
+    TaskWords() = default;
+    __device__ __forceinline__ TaskWords(const WalkTask *T, int lane)
+    {
+        word = agent_load((const int32_t *)T + (lane < WALK_TASK_WORDS ? lane : 0));
+    }
+    template <int32_t WalkTask::*F> __device__ __forceinline__ int get() const
+    {
+        constexpr WalkTask T{};
+        return __builtin_amdgcn_readlane(word, (int)(&(T.*F) - &T.group));
+    }
+};
+
+// the row of a share of entry p is stored: counts p's shares down; the last share's wave adds them up,
+// and so on up to the group, whose total is the result.  Returns the group's entry then, or -1.
 template <int FIELDS, typename R>
-__device__ __forceinline__ void walk_add_up(const WalkPool &B, int self, const WalkSpan &grp, int gs, const int64_t *perm,
-                                            double G, double *out, int lane)
+__device__ __forceinline__ int walk_add_up(WalkCtl *ctl, const WalkPool &B, int p, const WalkSpan &grp, int gs,
+                                           const int64_t *perm, double G, double *out, int lane)
 {
     constexpr int WI = Sums<FIELDS>::WI;
     const int nv = grp.mt * WI;
@@ -270,19 +339,33 @@ __device__ __forceinline__ void walk_add_up(const WalkPool &B, int self, const W
     R *rows = (R *)B.partial;
     for (;;) {
         wave_stores_done();
-        const int p = __builtin_amdgcn_readfirstlane(agent_load(&B.tasks[self].parent));
-        WalkTask *T = &B.tasks[p];
-        int w = 0;
-        if (lane == 0) w = atomicSub(&T->wait, 1);
-        if (__builtin_amdgcn_readfirstlane(w) != 1) return;
+        int last = 0;
+        if (lane == 0) last = task_close<AgentMem>(B, p);
+        if (!__builtin_amdgcn_readfirstlane(last)) return -1;
         asm volatile("" ::: "memory");
-        const int nchild = __builtin_amdgcn_readfirstlane(agent_load(&T->nchild));
-        const int64_t kids = __builtin_amdgcn_readfirstlane(agent_load(&T->child0)) * rs;
+        const TaskWords T(&B.tasks[p], lane);
+        const int nchild = T.get<&WalkTask::nchild>(), kid0 = T.get<&WalkTask::child0>();
+        const bool own = T.get<&WalkTask::off>() >= 0;  // p has a row
+        if (p < B.gcount && T.get<&WalkTask::root>()) {  // a share found no room
+            if (lane == 0) walk_put_back<AgentMem>(ctl, B, true, T.word);  // lane 0: the group
+            return -1;
+        }
+        const R *slots = rows + B.gcount * rs;
 #pragma unroll 1
         for (int v = lane; v < nv; v += 64) {
-            R s = agent_load(&rows[p * rs + v]);
-#pragma unroll 4
-            for (int k = 0; k < nchild; k++) s += agent_load(&rows[kids + k * rs + v]);
+            R s = agent_load(own ? &rows[p * rs + v] : &slots[kid0 * rs + v]);
+#pragma unroll 1
+            for (int k0 = own ? 0 : 1; k0 < nchild; k0 += 16) {
+                R t[16];  // the loads go out together
+#pragma unroll
+                for (int u = 0; u < 16; u++) {
+                    const int e = kid0 + (k0 + u < nchild ? k0 + u : nchild - 1);
+                    t[u] = agent_load(&slots[(e < B.tcount ? e : e - B.tcount) * rs + v]);  // the slots go round
+                }
+#pragma unroll
+                for (int u = 0; u < 16; u++)
+                    if (k0 + u < nchild) s += t[u];
+            }
             if (p >= B.gcount) {
                 agent_store(&rows[p * rs + v], s);
             } else {
@@ -290,8 +373,8 @@ __device__ __forceinline__ void walk_add_up(const WalkPool &B, int self, const W
                 store_sum<FIELDS>(out + o * Sums<FIELDS>::WO, v % WI, G * (double)s);
             }
         }
-        if (p < B.gcount) return;
-        self = p;
+        if (p < B.gcount) return p;
+        p = T.get<&WalkTask::parent>();
     }
 }
 
@@ -326,6 +409,6 @@ struct Walk64Args {
 // spill entries per wave; cus = the device's compute units
 // angle-binned column density (colden.hip): groups of gs <= 64 sorted targets, six sums each (soft and
 // perm NULL: no softening, rows in target order), scaled by G
-ptg_status ptg_walk64_bins(const Walk64Args &a, int cus, int gcap, char *ws, size_t ws_bytes, hipStream_t s);
-ptg_status ptg_walk64_launch(const Walk64Args &a, int fields, bool quad, int cus, int gcap, char *ws, size_t ws_bytes,
+ptg_status ptg_walk64_bins(const Walk64Args &a, int cus, int gcap, size_t again, char *ws, size_t ws_bytes, hipStream_t s);
+ptg_status ptg_walk64_launch(const Walk64Args &a, int fields, bool quad, int cus, int gcap, size_t again, char *ws, size_t ws_bytes,
                              hipStream_t s);
