@@ -18,6 +18,8 @@
 // ms, tidal tensors with quadrupoles of 6e4 23.3 -> 1.24 ms.  Angle-binned columns of 2e5 particles
 // against their own walk (two waves per SIMD, six selected adds and a division a pair): 4.9 -> 2.15 ms.
 
+#include <cfloat>
+
 #include "walk_shared.hpp"
 
 #define LIST 32           // a list is evaluated in multiples of LIST entries once it holds LIST
@@ -39,22 +41,26 @@ template <int FIELDS, bool QUAD> struct Lds64 {
     double bins[FIELDS == BINS ? 6 * 64 : 1];  // [bin][lane]
 };
 
-// 1/sqrt(x) and 1/x: the hardware estimate (2^-24) with one cubic step, 1-2 ulp
-__device__ __forceinline__ double rsqrt64(double x)
+// 1/sqrt(x) and 1/x of x > 0: the hardware estimate (2^-24) with one cubic step, 1-2 ulp.  WIDE: the step's own
+// terms stay finite for every x, so that infinity gives 0, what is too small for a reciprocal infinity, and a nan nan.
+template <bool WIDE> __device__ __forceinline__ double rsqrt64(double x)
 {
     const double y = __builtin_amdgcn_rsq(x);
-    const double e = fma(-x * y, y, 1.0);
+    const double e = fma(-(WIDE ? fmin(x, DBL_MAX) : x) * y, y, 1.0);
     return fma(y * e, fma(0.375, e, 0.5), y);
 }
-__device__ __forceinline__ double rcp64(double x)
+template <bool WIDE> __device__ __forceinline__ double rcp64(double x)
 {
-    const double y = __builtin_amdgcn_rcp(x);
-    const double e = fma(-x, y, 1.0);
+    const double y = __builtin_amdgcn_rcp(x), f = WIDE ? fmin(y, DBL_MAX) : y;
+    const double e = fma(-(WIDE ? fmin(x, DBL_MAX) : x), f, 1.0);
     return fma(y, fma(e, e, e), y);
 }
 
-// squared distances are capped so that the refinement of 1/sqrt stays finite (r2 = inf gives nan)
-#define R2_MAX 1e300
+// A group is walked WIDE where a coordinate of it or of its tree is not at most this large, or a target's softening: no
+// other squared distance can overflow.  Caps in every pair cost 6 to 18 % of the walk (groups of 64 to 256).
+#define ORDINARY 1e153
+
+__device__ __forceinline__ bool is_nan3(double x, double y, double z) { return !(x == x) | !(y == y) | !(z == z); }
 
 template <int FIELDS>
 __device__ __forceinline__ void add_pair(Acc<double> &a, double phi, double K, double Q, double dx, double dy, double dz)
@@ -76,13 +82,13 @@ __device__ __forceinline__ void add_pair(Acc<double> &a, double phi, double K, d
     }
 }
 
-template <int FIELDS, bool QUAD>
+template <int FIELDS, bool QUAD, bool WIDE>
 __device__ __forceinline__ void pair_node(Acc<double> &a, const V4<double> &s, const double *q, double tx, double ty,
                                           double tz)
 {
     const double dx = s.x - tx, dy = s.y - ty, dz = s.z - tz;
-    const double r2 = fmin(dx * dx + dy * dy + dz * dz, R2_MAX);
-    const double rinv = rsqrt64(r2), rinv2 = rinv * rinv;
+    const double r2 = dx * dx + dy * dy + dz * dz;
+    const double rinv = rsqrt64<WIDE>(r2), rinv2 = rinv * rinv;
     const double mr = s.w * rinv, K = mr * rinv2;
     add_pair<FIELDS>(a, -mr, K, 3.0 * K * rinv2, dx, dy, dz);
     if (QUAD) {
@@ -114,10 +120,10 @@ __device__ __forceinline__ void pair_node(Acc<double> &a, const V4<double> &s, c
 }
 
 // the M4 spline softening of kernel.py:4-75 at 0 < r < h
-template <int FIELDS>
+template <int FIELDS, bool WIDE>
 __device__ __forceinline__ void spline64(double r, double rinv, double h, double &phi, double &K, double &Q)
 {
-    const double hinv = rcp64(h), q = r * hinv;
+    const double hinv = rcp64<WIDE>(h), q = r * hinv;
     const double hinv2 = hinv * hinv, hinv3 = hinv2 * hinv;
     if (q <= 0.5) {
         const double q2 = q * q;
@@ -141,26 +147,27 @@ struct Pair64 {
     double dx, dy, dz, r2, h;
     bool apart, soft;
 };
+template <bool WIDE>
 __device__ __forceinline__ Pair64 part_pair(const V4<double> &s, double hs, double tx, double ty, double tz, double th)
 {
     Pair64 p;
     p.dx = s.x - tx;
     p.dy = s.y - ty;
     p.dz = s.z - tz;
-    p.r2 = fmin(p.dx * p.dx + p.dy * p.dy + p.dz * p.dz, R2_MAX);
+    p.r2 = p.dx * p.dx + p.dy * p.dy + p.dz * p.dz;
     p.h = fmax(hs, th);
     p.apart = p.r2 > 0.0;
-    p.soft = p.apart && p.r2 < p.h * p.h;
+    p.soft = p.apart & (!WIDE | (th == th)) & (p.r2 < p.h * p.h);  // a target whose softening is a nan is never softened
     return p;
 }
-template <int FIELDS, bool SOFT>
+template <int FIELDS, bool SOFT, bool WIDE>
 __device__ __forceinline__ void part_add(Acc<double> &a, const Pair64 &p, double m)
 {
-    const double rinv = p.apart ? rsqrt64(p.r2) : 0.0, rinv2 = rinv * rinv;
+    const double rinv = p.apart ? rsqrt64<WIDE>(p.r2) : 0.0, rinv2 = rinv * rinv;
     const double mr = m * rinv;
     double phi = -mr, K = mr * rinv2, Q = 3.0 * K * rinv2;
     if (SOFT && p.soft) {
-        spline64<FIELDS>(p.r2 * rinv, rinv, p.h, phi, K, Q);
+        spline64<FIELDS, WIDE>(p.r2 * rinv, rinv, p.h, phi, K, Q);
         phi *= m;
         K *= m;
         Q *= m;
@@ -171,7 +178,7 @@ __device__ __forceinline__ void part_add(Acc<double> &a, const Pair64 &p, double
 // U entries of a lane's slice of a list together: their LDS reads are issued at once and their chains
 // overlap, and the spline is evaluated only where a pair of the batch is softened.  The terms are added in
 // the order of the list.
-template <int U, int TPL, int FIELDS, bool QUAD, typename L>
+template <int U, int TPL, int FIELDS, bool QUAD, bool WIDE, typename L>
 __device__ __forceinline__ void add_nodes(const L &l, int at, int step, Acc<double> (&acc)[TPL], const double (&tx)[TPL],
                                           const double (&ty)[TPL], const double (&tz)[TPL])
 {
@@ -182,9 +189,9 @@ __device__ __forceinline__ void add_nodes(const L &l, int at, int step, Acc<doub
     for (int u = 0; u < U; u++)
 #pragma unroll
         for (int j = 0; j < TPL; j++)
-            pair_node<FIELDS, QUAD>(acc[j], s[u], &l.nq[QUAD ? 6 * (at + u * step) : 0], tx[j], ty[j], tz[j]);
+            pair_node<FIELDS, QUAD, WIDE>(acc[j], s[u], &l.nq[QUAD ? 6 * (at + u * step) : 0], tx[j], ty[j], tz[j]);
 }
-template <int U, int TPL, int FIELDS, typename L>
+template <int U, int TPL, int FIELDS, bool WIDE, typename L>
 __device__ __forceinline__ void add_parts(const L &l, int at, int step, Acc<double> (&acc)[TPL], const double (&tx)[TPL],
                                           const double (&ty)[TPL], const double (&tz)[TPL], const double (&th)[TPL])
 {
@@ -201,41 +208,41 @@ __device__ __forceinline__ void add_parts(const L &l, int at, int step, Acc<doub
         bool soft = false;
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            p[u] = part_pair(s[u], hs[u], tx[j], ty[j], tz[j], th[j]);
+            p[u] = part_pair<WIDE>(s[u], hs[u], tx[j], ty[j], tz[j], th[j]);
             soft |= p[u].soft;
         }
         if (ptg_ballot(soft)) {
             // the barrier keeps this a branch: as selects, every pair went through the spline's 27 instructions
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
-            for (int u = 0; u < U; u++) part_add<FIELDS, true>(acc[j], p[u], s[u].w);
+            for (int u = 0; u < U; u++) part_add<FIELDS, true, WIDE>(acc[j], p[u], s[u].w);
         } else {
 #pragma unroll
-            for (int u = 0; u < U; u++) part_add<FIELDS, false>(acc[j], p[u], s[u].w);
+            for (int u = 0; u < U; u++) part_add<FIELDS, false, WIDE>(acc[j], p[u], s[u].w);
         }
     }
 }
 // entries [0, c) of the lists, this lane's slice of them
-template <int U, int TPL, int FIELDS, bool QUAD, typename L>
+template <int U, int TPL, int FIELDS, bool QUAD, bool WIDE, typename L>
 __device__ __forceinline__ void sum_nodes(const L &l, int sl, int slices, int c, Acc<double> (&acc)[TPL],
                                           const double (&tx)[TPL], const double (&ty)[TPL], const double (&tz)[TPL])
 {
     int q = sl;
 #pragma unroll 1
-    for (; q + (U - 1) * slices < c; q += U * slices) add_nodes<U, TPL, FIELDS, QUAD>(l, q, slices, acc, tx, ty, tz);
+    for (; q + (U - 1) * slices < c; q += U * slices) add_nodes<U, TPL, FIELDS, QUAD, WIDE>(l, q, slices, acc, tx, ty, tz);
 #pragma unroll 1
-    for (; U > 1 && q < c; q += slices) add_nodes<1, TPL, FIELDS, QUAD>(l, q, slices, acc, tx, ty, tz);
+    for (; U > 1 && q < c; q += slices) add_nodes<1, TPL, FIELDS, QUAD, WIDE>(l, q, slices, acc, tx, ty, tz);
 }
-template <int U, int TPL, int FIELDS, typename L>
+template <int U, int TPL, int FIELDS, bool WIDE, typename L>
 __device__ __forceinline__ void sum_parts(const L &l, int sl, int slices, int c, Acc<double> (&acc)[TPL],
                                           const double (&tx)[TPL], const double (&ty)[TPL], const double (&tz)[TPL],
                                           const double (&th)[TPL])
 {
     int q = sl;
 #pragma unroll 1
-    for (; q + (U - 1) * slices < c; q += U * slices) add_parts<U, TPL, FIELDS>(l, q, slices, acc, tx, ty, tz, th);
+    for (; q + (U - 1) * slices < c; q += U * slices) add_parts<U, TPL, FIELDS, WIDE>(l, q, slices, acc, tx, ty, tz, th);
 #pragma unroll 1
-    for (; U > 1 && q < c; q += slices) add_parts<1, TPL, FIELDS>(l, q, slices, acc, tx, ty, tz, th);
+    for (; U > 1 && q < c; q += slices) add_parts<1, TPL, FIELDS, WIDE>(l, q, slices, acc, tx, ty, tz, th);
 }
 
 // angle-binned columns of one lane: LDS sums bins[64 * bin] (units of mass / distance^2) and the part
@@ -254,24 +261,24 @@ struct Sky {
         __hip_atomic_fetch_add(bins + 64 * bin, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
     }
     // an element farther than its radius: a point mass
-    __device__ __forceinline__ void node(const V4<double> &s, double tx, double ty, double tz)
+    template <bool WIDE> __device__ __forceinline__ void node(const V4<double> &s, double tx, double ty, double tz)
     {
         const double dx = s.x - tx, dy = s.y - ty, dz = s.z - tz;
-        add(dx, dy, dz, s.w * rcp64(fmin(dx * dx + dy * dy + dz * dz, R2_MAX)));
+        add(dx, dy, dz, s.w * rcp64<WIDE>(dx * dx + dy * dy + dz * dz));
     }
     // a particle: a point mass outside its radius h, a blend of the isotropic and directed limits inside
-    __device__ __forceinline__ void part(const V4<double> &s, double h, double tx, double ty, double tz)
+    template <bool WIDE> __device__ __forceinline__ void part(const V4<double> &s, double h, double tx, double ty, double tz)
     {
         const double dx = s.x - tx, dy = s.y - ty, dz = s.z - tz;
-        const double r2 = fmin(dx * dx + dy * dy + dz * dz, R2_MAX), hh = h * h;
+        const double r2 = dx * dx + dy * dy + dz * dz, hh = h * h;
         const bool out = r2 > hh;
-        double v = s.w * rcp64(out ? r2 : 1.0);
+        double v = s.w * rcp64<WIDE>(out ? r2 : 1.0);
         if (ptg_ballot(!out)) {
             if (!out) {
                 v = 0.0;
                 if (h > 0) {
-                    const double hinv = rcp64(h), col0 = s.w * (3.0 / (4.0 * 3.14159265358979323846) * SKY_BIN) * hinv * hinv;
-                    const double fac = r2 > 0 ? r2 * rsqrt64(r2) * hinv : 0.0;
+                    const double hinv = rcp64<WIDE>(h), col0 = s.w * (3.0 / (4.0 * 3.14159265358979323846) * SKY_BIN) * hinv * hinv;
+                    const double fac = r2 == 0 ? 0.0 : r2 * rsqrt64<WIDE>(r2) * hinv;
                     iso += (1.0 - fac) * col0;
                     v = 2.0 * col0 * fac;
                 }
@@ -404,12 +411,54 @@ void k_walk64(const Walk64Args A, const WalkHot H, const WalkPool pool)
             bmax1 = ptg_wave_max(bmax1);
             bmax2 = ptg_wave_max(bmax2);
             hmax = ptg_wave_max(hmax);
+            // a target with a nan coordinate bounds nothing; of binned columns it gets what the particles' own radii
+            // give it, so none of its group's particles is taken for a far one
+            const bool near_all = FIELDS == BINS && ptg_ballot(is_nan3(tx[0], ty[0], tz[0])) != 0;
+            const V4<double> top = A.xyzm[root];
+            const double far = fmax(fmax(fabs(top.x), fabs(top.y)), fabs(top.z)) + A.aux[root].y;
+            bool odd = !(far <= ORDINARY);
+#pragma unroll
+            for (int j = 0; j < TPL; j++)
+                odd |= !(fabs(tx[j]) <= ORDINARY) | !(fabs(ty[j]) <= ORDINARY) | !(fabs(tz[j]) <= ORDINARY) | !(th[j] <= ORDINARY);
+            const bool wide = ptg_ballot(odd) != 0;
             Acc<double> acc[TPL];
 #pragma unroll
             for (int j = 0; j < TPL; j++) acc[j] = Acc<double>{0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
             Sky sky{&L.bins[FIELDS == BINS ? lane : 0], 0.0};
             if (FIELDS == BINS)
                 for (int q = 0; q < 6; q++) L.bins[64 * q + lane] = 0.0;
+
+            // entries [0, c) of a list, this lane's slice of them
+            auto nodes_now = [&](int c) {
+                if constexpr (FIELDS == BINS) {
+                    if (wide) {
+#pragma unroll 1
+                        for (int q = sl; q < c; q += slices) sky.template node<true>(L.nodes[q], tx[0], ty[0], tz[0]);
+                    } else {
+                        for (int q = sl; q < c; q += slices) sky.template node<false>(L.nodes[q], tx[0], ty[0], tz[0]);
+                    }
+                } else if (wide) {
+                    sum_nodes<1, TPL, FIELDS, QUAD, true>(L, sl, slices, c, acc, tx, ty, tz);
+                } else {
+                    sum_nodes<UN, TPL, FIELDS, QUAD, false>(L, sl, slices, c, acc, tx, ty, tz);
+                }
+            };
+            auto parts_now = [&](int c) {
+                if constexpr (FIELDS == BINS) {
+                    if (wide) {
+#pragma unroll 1
+                        for (int q = sl; q < c; q += slices)
+                            sky.template part<true>(L.parts[q], L.ph[q], tx[0], ty[0], tz[0]);
+                    } else {
+                        for (int q = sl; q < c; q += slices)
+                            sky.template part<false>(L.parts[q], L.ph[q], tx[0], ty[0], tz[0]);
+                    }
+                } else if (wide) {
+                    sum_parts<1, TPL, FIELDS, true>(L, sl, slices, c, acc, tx, ty, tz, th);
+                } else {
+                    sum_parts<UP, TPL, FIELDS, false>(L, sl, slices, c, acc, tx, ty, tz, th);
+                }
+            };
 
             int sp = 1, gsp = 0, nn = 0, np = 0, visits = 0, n_list = 0, n_part = 0;
             bool overflow = false;
@@ -486,7 +535,7 @@ void k_walk64(const Walk64Args A, const WalkHot H, const WalkPool pool)
                     }
                     // a particle farther from the box than every softening radius needs neither the softening
                     // nor the self test; with quadrupoles it stays a particle (no quadrupole terms)
-                    const bool far_part = !QUAD & ve & ispart & (r2m > hh * hh);
+                    const bool far_part = !QUAD & ve & ispart & (r2m > hh * hh) & !near_all;
                     const bool acc_part = ve & ispart & !far_part;
                     const bool open = ve & !ispart & !acc_node;
                     acc_node |= far_part;
@@ -537,11 +586,7 @@ void k_walk64(const Walk64Args A, const WalkHot H, const WalkPool pool)
 
                     if (nn >= LIST) {
                         const int c = nn & ~(LIST - 1);  // c >= LIST > nn - c
-                        if constexpr (FIELDS == BINS) {
-                            for (int q = sl; q < c; q += slices) sky.node(L.nodes[q], tx[0], ty[0], tz[0]);
-                        } else {
-                            sum_nodes<UN, TPL, FIELDS, QUAD>(L, sl, slices, c, acc, tx, ty, tz);
-                        }
+                        nodes_now(c);
                         __builtin_amdgcn_wave_barrier();
                         if (lane < nn - c) {  // reads [c, nn) and writes [0, nn - c): disjoint
                             L.nodes[lane] = L.nodes[c + lane];
@@ -553,11 +598,7 @@ void k_walk64(const Walk64Args A, const WalkHot H, const WalkPool pool)
                     }
                     if (np >= LIST) {
                         const int c = np & ~(LIST - 1);
-                        if constexpr (FIELDS == BINS) {
-                            for (int q = sl; q < c; q += slices) sky.part(L.parts[q], L.ph[q], tx[0], ty[0], tz[0]);
-                        } else {
-                            sum_parts<UP, TPL, FIELDS>(L, sl, slices, c, acc, tx, ty, tz, th);
-                        }
+                        parts_now(c);
                         __builtin_amdgcn_wave_barrier();
                         if (lane < np - c) {  // disjoint ranges, as above
                             L.parts[lane] = L.parts[c + lane];
@@ -599,16 +640,8 @@ void k_walk64(const Walk64Args A, const WalkHot H, const WalkPool pool)
                 if (lane == 0) atomicOr(&A.ctl->err, 1);
                 nn = np = 0;  // a task's row is still written: the sums read every task's
             }
-            if constexpr (FIELDS == BINS) {
-                for (int q = sl; q < nn; q += slices) sky.node(L.nodes[q], tx[0], ty[0], tz[0]);
-            } else {
-                sum_nodes<UN, TPL, FIELDS, QUAD>(L, sl, slices, nn, acc, tx, ty, tz);
-            }
-            if constexpr (FIELDS == BINS) {
-                for (int q = sl; q < np; q += slices) sky.part(L.parts[q], L.ph[q], tx[0], ty[0], tz[0]);
-            } else {
-                sum_parts<UP, TPL, FIELDS>(L, sl, slices, np, acc, tx, ty, tz, th);
-            }
+            nodes_now(nn);
+            parts_now(np);
             __builtin_amdgcn_wave_barrier();
             [[maybe_unused]] double bin[FIELDS == BINS ? 6 : 1];
             if constexpr (FIELDS == BINS) {
@@ -618,6 +651,11 @@ void k_walk64(const Walk64Args A, const WalkHot H, const WalkPool pool)
 #pragma unroll
                     for (int q = 0; q < 6; q++) bin[q] += __shfl_xor(bin[q], d, 64);
                 }
+            }
+            if (FIELDS != BINS && wide) {  // a target with a nan coordinate meets nothing
+#pragma unroll
+                for (int j = 0; j < TPL; j++)
+                    if (is_nan3(tx[j], ty[j], tz[j])) acc[j] = Acc<double>{0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
             }
             for (int d = P; FIELDS != BINS && d < 64; d <<= 1) {
 #pragma unroll
