@@ -431,8 +431,8 @@ ptg_status ptg_ray_orders(const double *pos, int64_t n, const double *rays, int6
  * box (ColumnDensityBinned_grouped :1197-1276; group_size 1 is ColumnDensityWalk_binned :976-1028).
  * group_size <= 64 walks the FP64 walk pack wt of the same tree (ptg_pack_walk, PTG_F64) with
  * ptg_column_workspace_bytes(group_size) of workspace (traversals past a budget of visits are finished
- * in parts by later passes, as the FP64 walk's); larger groups use the tree's links (wt, ws may be NULL).
- * err: 1 corrupt links, 2 a traversal stack overflow.  counters (nullable, device int64[2],
+ * in shares by a second pass, as the FP64 walk's); larger groups use the tree's links (wt, ws may be NULL).
+ * err: 1 corrupt links, 2 a traversal stack overflow, 4 a share of a cut traversal never finished.  counters (nullable, device int64[2],
  * accumulated): [0] element-target pairs evaluated, [1] elements visited by the group traversals. */
 size_t ptg_column_workspace_bytes(int64_t group_size);
 /* Per-target ray grids for randomize_rays (treewalk.py:1061-1078, misc.random_rotation misc.py:6-54):

@@ -519,7 +519,9 @@ __global__ __launch_bounds__(CD_THREADS) void k_column_binned(const ptg_tree_arr
 
 
 // ---- wavefront-per-group binned walk: k_walk64's traversal (walk64.hip) with six sums per target ----
-#define CB_GCAP 10240  // global spill entries per wave (a step leaves at most 448 a level of the 21 levels)
+// global spill entries per wave: a step leaves at most 448 a level, so 36 levels of a tree all of whose nodes are
+// opened; a tree whose keys collide has up to 84
+#define CB_GCAP 16384
 
 static int cb_cus()
 {
@@ -540,7 +542,8 @@ extern "C" size_t ptg_column_workspace_bytes(int64_t group_size)
 // the walk's flags as ptg_column_binned reports them
 __global__ void k_column_err_out(const WalkCtl *ctl, int32_t *err)
 {
-    if (ctl->err) *err |= 2;  // a traversal stack overflow
+    if (ctl->err & 1) *err |= 2;  // a traversal stack overflow
+    if (ctl->err & 8) *err |= 4;  // the task pass gave up
 }
 __global__ void k_column_err_init(int32_t *err) { *err = 0; }
 static ptg_status column_common(const ptg_tree_arrays *tree, int64_t n, int64_t nnodes, const double *targets,

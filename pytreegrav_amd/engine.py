@@ -755,7 +755,8 @@ def column_binned(tree, targets, group_size=16, theta=0.5, counters=None):
           "ptg_column_binned")
     e = int(err.item())
     if e:
-        raise RuntimeError("ptg_column_binned: " + ("corrupt tree links" if e & 1 else "traversal stack overflow"))
+        what = "corrupt tree links" if e & 1 else "traversal stack overflow" if e & 2 else "cut traversals never finished"
+        raise RuntimeError("ptg_column_binned: " + what)
     return out
 
 
