@@ -418,7 +418,8 @@ ptg_status ptg_column_rays(const ptg_tree_arrays *tree, int64_t n, int64_t nnode
                            const int64_t *order, double *out, int32_t *err, int64_t *counters, void *stream);
 /* The ray-traced columns of shared unit rays by bundles of 64 consecutive targets of `order` (nrays, nt),
  * or of the targets as given (NULL): one wavefront walks the FP64 pack once for its bundle.  The same
- * particles and chord terms as ptg_column_rays, summed in the bundle's order.  err as there. */
+ * particles and chord terms as ptg_column_rays, summed in the bundle's order.  err as there, and 4: a ray is not
+ * of unit length; on 2 or 4 the columns are not complete (ptg_column_rays gives them). */
 ptg_status ptg_column_bundles(const ptg_walk_tree *wt, const double *targets, int64_t nt, const double *rays,
                               int64_t nrays, const int64_t *order, double *out, int32_t *err, void *stream);
 /* order[i][..] = the targets in the 2D Morton order of their positions across unit ray i (no reference

@@ -300,10 +300,13 @@ __global__ __launch_bounds__(64 * CN_WAVES) __attribute__((amdgpu_waves_per_eu(4
     const int64_t j = order ? order[i * nt + jl] : jl;
     const double rx = rays[3 * i], ry = rays[3 * i + 1], rz = rays[3 * i + 2];
     const double px = tp[3 * j], py = tp[3 * j + 1], pz = tp[3 * j + 2];
-    // frame of the bundle: origin at its first finite target, e1 and e2 across the ray, e3 along it.  A ray that
-    // is not of unit length meets every element (its columns are the formulae's, not a geometry's).
-    const double len2 = rx * rx + ry * ry + rz * rz;
-    const double slack0 = fabs(len2 - 1.0) < 1e-9 ? 0.0 : INFINITY;
+    // A ray that is not of unit length has no geometry to bundle by: its columns are what the formulae give along
+    // each target's own walk, which the caller makes.
+    if (!(fabs(rx * rx + ry * ry + rz * rz - 1.0) < 1e-13)) {
+        if (lane == 0) atomicOr(err, 4);
+        return;
+    }
+    // frame of the bundle: origin at its first finite target, e1 and e2 across the ray, e3 along it
     const bool fin = isfinite(px) && isfinite(py) && isfinite(pz);  // others see no column and bound nothing
     const uint64_t mf = ptg_ballot(fin);
     const int ol = mf ? (int)__ffsll((unsigned long long)mf) - 1 : 0;
@@ -348,7 +351,7 @@ __global__ __launch_bounds__(64 * CN_WAVES) __attribute__((amdgpu_waves_per_eu(4
     while (sp > 0) {
         // 64 elements, or as many as the stack has room for the children of
         const int k = std::min(std::min(sp, 64), (CN_SCAP - sp) / 7);
-        if (k < 1) {  // deeper than the stack: the caller reruns the stackless walk
+        if (k < 1) {  // deeper than the stack: the caller makes the targets' own walks
             if (lane == 0) atomicOr(err, 2);
             break;
         }
@@ -367,7 +370,7 @@ __global__ __launch_bounds__(64 * CN_WAVES) __attribute__((amdgpu_waves_per_eu(4
         const double ec = rx * dx + ry * dy + rz * dz;
         // the coordinates above and the targets' carry a few 2^-53 of the distances: 1e-14 covers them
         double reach = ispart ? X2.x : X2.x + X2.y * 0.8660254037844386 + X2.z;
-        reach += 1e-14 * (fabs(dx) + fabs(dy) + fabs(dz) + tmax) + slack0;
+        reach += 1e-14 * (fabs(dx) + fabs(dy) + fabs(dz) + tmax);
         const double rr = reach * reach;
         const double ga = cn_gap(ea, alo, ahi), gb = cn_gap(eb, blo, bhi);
         bool hit = ve & (ga * ga + gb * gb <= rr) & (ec + reach > clo) & (!ispart | (X2.x > 0.0));

@@ -717,9 +717,13 @@ def column_rays(tree, targets, rays, per_target=False, counters=None):
     # shared rays: per ray, the targets in 2D Morton order of their position across the ray, so the
     # 64 targets of a wavefront walk nearly the same path
     order = _ray_orders(tp, r) if not per_target and nt > 64 else None
-    # the wavefront walks over the FP64 pack; a tree deeper than their stacks reruns the stackless walk
-    for wt in (_lib.ctypes.byref(tree.pack(PTG_F64, False)["wt"]), None):
-        if wt is not None and not per_target and counters is None:
+    # the wavefront walks over the FP64 pack: of bundles, then (rays that are not of unit length, a tree deeper than
+    # the bundles' stack) of the targets' own paths; a tree deeper than that one's stack reruns the stackless walk
+    wt = _lib.ctypes.byref(tree.pack(PTG_F64, False)["wt"])
+    for bundles, wt in ((True, wt), (False, wt), (False, None)):
+        if bundles:
+            if per_target or counters is not None:
+                continue
             check(L.ptg_column_bundles(wt, ptr(tp), nt, ptr(r), nr, ptr(order), ptr(out), ptr(err), stream()),
                   "ptg_column_bundles")
         else:
