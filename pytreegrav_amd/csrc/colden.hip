@@ -39,6 +39,15 @@ __device__ __forceinline__ void cd_count(unsigned long long *ctr, int k, int64_t
     if (ptg_lane() == 0 && v) atomicAdd(ctr + k, (unsigned long long)v);
 }
 
+// squared distance across a ray: the product is rounded by itself, so that an element exactly along the ray (r2 = z^2,
+// as on a lattice) is at 0.  As a fused multiply-add its sign was z^2's rounding error, and half of such elements,
+// particles and whole nodes, were skipped.
+__device__ __forceinline__ double across2(double r2, double z)
+{
+#pragma clang fp contract(off)
+    return r2 - z * z;
+}
+
 // column along ray i from target j; visits counts the elements the walk touched
 __device__ __forceinline__ double ray_column(const ptg_tree_arrays &t, int64_t n, int64_t ne, const double *tp,
                                              const double *rays, int64_t nr, int per_target, int64_t i, int64_t j,
@@ -61,7 +70,7 @@ __device__ __forceinline__ double ray_column(const ptg_tree_arrays &t, int64_t n
         const double r2 = dx * dx + dy * dy + dz * dz;
         const double r = sqrt(r2);
         const double z = rx * dx + ry * dy + rz * dz;
-        if (r2 - z * z < 0) {  // rounding below zero: skipped, as ColumnDensityWalk_singleray does
+        if (across2(r2, z) < 0) {  // rounding below zero: skipped, as ColumnDensityWalk_singleray does
             no = t.next_branch[no];
             continue;
         }
@@ -70,7 +79,7 @@ __device__ __forceinline__ double ray_column(const ptg_tree_arrays &t, int64_t n
             if (h_no > 0) {  // a zero radius has no cross-section
                 const double hinv = 1.0 / h_no;
                 const double fac = fac_density * t.masses[no] * hinv * hinv;
-                const double r_proj = sqrt(r2 - z * z);
+                const double r_proj = sqrt(across2(r2, z));
                 const double q = r_proj * hinv;
                 if (r_proj < h_no) {
                     if (r > h_no) {  // target outside the sphere: the whole chord if it lies ahead
@@ -84,7 +93,7 @@ __device__ __forceinline__ double ray_column(const ptg_tree_arrays &t, int64_t n
         } else {
             const double reach = h_no + t.sizes[no] * 0.8660254037844386 + t.deltas[no];
             bool open = r < reach;  // the node holds the ray's origin
-            if (!open && z > 0) open = (r2 - z * z) < reach * reach;
+            if (!open && z > 0) open = (across2(r2, z)) < reach * reach;
             no = open ? t.first_subnode[no] : t.next_branch[no];
         }
     }
@@ -183,13 +192,13 @@ __global__ __launch_bounds__(64 * CR_WAVES) void k_column_rays_wave(const D4 *xy
             const double r2 = dx * dx + dy * dy + dz * dz;
             const double r = sqrt(r2);
             const double z = rx * dx + ry * dy + rz * dz;
-            if (!(r2 - z * z < 0)) {  // rounding below zero: skipped, as ColumnDensityWalk_singleray does
+            if (!(across2(r2, z) < 0)) {  // rounding below zero: skipped, as ColumnDensityWalk_singleray does
                 const double h_no = X2.x;
                 if (K.y == 0) {
                     if (h_no > 0) {  // a zero radius has no cross-section
                         const double hinv = 1.0 / h_no;
                         const double fac = fac_density * X.w * hinv * hinv;
-                        const double r_proj = sqrt(r2 - z * z);
+                        const double r_proj = sqrt(across2(r2, z));
                         const double q = r_proj * hinv;
                         if (r_proj < h_no) {
                             if (r > h_no) {
@@ -202,7 +211,7 @@ __global__ __launch_bounds__(64 * CR_WAVES) void k_column_rays_wave(const D4 *xy
                 } else {
                     const double reach = h_no + X2.y * 0.8660254037844386 + X2.z;
                     open = r < reach;
-                    if (!open && z > 0) open = (r2 - z * z) < reach * reach;
+                    if (!open && z > 0) open = (across2(r2, z)) < reach * reach;
                 }
             }
         }
@@ -270,7 +279,7 @@ __device__ __forceinline__ void cn_flush(const CnLds &S, int c, double px, doubl
         const double dx = P.x - px, dy = P.y - py, dz = P.z - pz;
         const double r2 = dx * dx + dy * dy + dz * dz;
         const double z = rx * dx + ry * dy + rz * dz;
-        const double b2 = r2 - z * z, hh = h * h;
+        const double b2 = across2(r2, z), hh = h * h;
         // b2 < 0 by rounding: skipped, as ColumnDensityWalk_singleray does
         const bool inside = !(r2 > hh);
         if (b2 >= 0 && b2 < hh && (inside || z > 0)) {
