@@ -304,6 +304,14 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint64_t *kin, 
 
 // number of sort tiles of n keys (RS_BINS histogram entries each)
 static int64_t rs_tiles(int64_t n, int items) { return std::max<int64_t>(1, ptg_cdiv(n, RS_THREADS * items)); }
+// the most tiles that n keys or fewer have (shorter tiles below a step of rs_items): a workspace for n serves fewer keys
+static int64_t rs_tiles_upto(int64_t n)
+{
+    int64_t most = rs_tiles(n, rs_items(n));
+    for (int64_t step = 1 << 16; step < n && step <= 1 << 20; step <<= 2)
+        most = std::max(most, rs_tiles(step, rs_items(step)));
+    return most;
+}
 
 struct RsWS {
     int32_t *hist;   // (RS_BINS, ntiles) tile counts, scanned in place per digit
@@ -313,7 +321,7 @@ struct RsWS {
 
 static void carve_rs(PtgArena &A, int64_t n, RsWS &w)
 {
-    w.hist = A.take<int32_t>((int64_t)RS_BINS * rs_tiles(n, rs_items(n)));
+    w.hist = A.take<int32_t>((int64_t)RS_BINS * rs_tiles_upto(n));
     w.dtot = A.take<int32_t>(RS_BINS);
     w.cap = n;
 }
