@@ -112,12 +112,13 @@ template <typename T, int FIELDS> struct DAcc {
     }
 };
 
-// one pair by the reference's branches (bruteforce.py); same: source and target are the same particle
+// one pair by the reference's branches (bruteforce.py), unless skip: source and target are the same particle, or the
+// entry is past the slice (its 0 mass would make a nan of a singular pair)
 template <typename T, int FIELDS, bool SELF>
-__device__ __forceinline__ void pair_branches(DAcc<T, FIELDS> &a, T dx, T dy, T dz, T r2, T m, T h, bool same)
+__device__ __forceinline__ void pair_branches(DAcc<T, FIELDS> &a, T dx, T dy, T dz, T r2, T m, T h, bool skip)
 {
     constexpr bool P = DAcc<T, FIELDS>::P, A = DAcc<T, FIELDS>::A, D = DAcc<T, FIELDS>::D;
-    if (SELF && same) return;
+    if (skip) return;
     const T r = sqrt(r2);
     T phi = 0, K = 0, Q = 0;
     if (P) {
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(64 * DS_WAVES) void k_direct(const double *pt, cons
                     const DV4<T> s = L.s[q];
                     const T ex = s.x - tx, ey = s.y - ty, ez = s.z - tz;
                     pair_branches<T, FIELDS, SELF>(acc, ex, ey, ez, ex * ex + ey * ey + ez * ez, s.w,
-                                                   L.h[q] > th ? L.h[q] : th, jt + q == i);
+                                                   L.h[q] > th ? L.h[q] : th, (SELF && jt + q == i) | (q >= cnt));
                 }
             }
         }
