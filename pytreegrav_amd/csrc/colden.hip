@@ -259,16 +259,7 @@ struct CnLds {
     double a[64], b[64];  // the targets across the ray
 };
 
-// 1/sqrt(x) by the hardware estimate and one cubic step (1-2 ulp), and sqrt(x) of x >= 0
-__device__ __forceinline__ double cn_rsqrt(double x)
-{
-    const double y = __builtin_amdgcn_rsq(x);
-    const double e = fma(-x * y, y, 1.0);
-    return fma(y * e, fma(0.375, e, 0.5), y);
-}
-__device__ __forceinline__ double cn_sqrt(double x) { return x > 0.0 ? x * cn_rsqrt(x) : 0.0; }
-
-__device__ __forceinline__ double cn_gap(double x, double lo, double hi) { return fmax(fmax(lo - x, x - hi), 0.0); }
+__device__ __forceinline__ double cn_sqrt(double x) { return x > 0.0 ? x * ptg_rsqrt64(x) : 0.0; }
 
 __device__ __forceinline__ void cn_flush(const CnLds &S, int c, double px, double py, double pz, double rx, double ry,
                                          double rz, double &column)
@@ -381,14 +372,14 @@ __global__ __launch_bounds__(64 * CN_WAVES) __attribute__((amdgpu_waves_per_eu(4
         double reach = ispart ? X2.x : X2.x + X2.y * 0.8660254037844386 + X2.z;
         reach += 1e-14 * (fabs(dx) + fabs(dy) + fabs(dz) + tmax);
         const double rr = reach * reach;
-        const double ga = cn_gap(ea, alo, ahi), gb = cn_gap(eb, blo, bhi);
+        const double ga = box_gap(ea, alo, ahi), gb = box_gap(eb, blo, bhi);
         bool hit = ve & (ga * ga + gb * gb <= rr) & (ec + reach > clo) & (!ispart | (X2.x > 0.0));
         if (ptg_ballot(hit & (side > CN_WIDE * reach))) {
             bool any = !(side > CN_WIDE * reach);
             for (int q = 0; q < 4; q++) {
                 const double l0 = __shfl(qalo, 16 * q, 64), l1 = __shfl(qahi, 16 * q, 64);
                 const double m0 = __shfl(qblo, 16 * q, 64), m1 = __shfl(qbhi, 16 * q, 64);
-                const double a2 = cn_gap(ea, l0, l1), b2 = cn_gap(eb, m0, m1);
+                const double a2 = box_gap(ea, l0, l1), b2 = box_gap(eb, m0, m1);
                 bool near = hit & !any & (a2 * a2 + b2 * b2 <= rr);
                 if (ptg_ballot(near & (fmax(l1 - l0, m1 - m0) > CN_WIDE * reach))) {
                     bool one = !(fmax(l1 - l0, m1 - m0) > CN_WIDE * reach);
@@ -405,7 +396,7 @@ __global__ __launch_bounds__(64 * CN_WAVES) __attribute__((amdgpu_waves_per_eu(4
         const bool list = hit & ispart;
         const uint64_t bl = ptg_ballot(list);
         if (list) {
-            const int at = np + (int)__popcll(bl & ptg_lanemask_lt());
+            const int at = np + lanes_below(bl);
             const double hinv = 1.0 / X2.x;
             S.part[at] = D4{X.x, X.y, X.z, fac_density * X.w * hinv * hinv};
             S.h[at] = X2.x;
@@ -413,13 +404,8 @@ __global__ __launch_bounds__(64 * CN_WAVES) __attribute__((amdgpu_waves_per_eu(4
         }
         np += (int)__popcll(bl);
         const int cnt = hit & !ispart ? std::min(std::max(K.y, 0), 8) : 0;
-        int below = 0, tot = 0;  // exclusive sum of counts below 16, one ballot per bit
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const uint64_t m = ptg_ballot((cnt >> b) & 1);
-            below += (int)__popcll(m & ptg_lanemask_lt()) << b;
-            tot += (int)__popcll(m) << b;
-        }
+        int tot;
+        const int below = small_excl_scan(cnt, tot);
         {
             int *dst = &S.stack[sp + below];
 #pragma unroll

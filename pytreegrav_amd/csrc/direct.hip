@@ -66,14 +66,9 @@ template <typename T> struct alignas(4 * sizeof(T)) DV4 {
     T x, y, z, w;
 };
 
-// 1/sqrt(x): the hardware's in FP32 (1 ulp); in FP64 its estimate (2^-24) and one cubic step (1-2 ulp)
+// 1/sqrt(x): the hardware's in FP32 (1 ulp)
 __device__ __forceinline__ float d_rsqrt(float x) { return __builtin_amdgcn_rsqf(x); }
-__device__ __forceinline__ double d_rsqrt(double x)
-{
-    const double y = __builtin_amdgcn_rsq(x);
-    const double e = fma(-x * y, y, 1.0);
-    return fma(y * e, fma(0.375, e, 0.5), y);
-}
+__device__ __forceinline__ double d_rsqrt(double x) { return ptg_rsqrt64(x); }
 
 // The plain path takes squared distances from the smallest ordinary number (below, the hardware's
 // reciprocal square root may flush them) and, in FP64, up to 1e300 (its step is nan at infinity, where

@@ -1,5 +1,6 @@
 // Shared device/host helpers for the gfx950 tree-gravity library.
 #pragma once
+#include <float.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -97,6 +98,24 @@ template <typename T> __device__ __forceinline__ T ptg_wave_max(T v)
         v = o > v ? o : v;
     }
     return v;
+}
+
+// -------------------------------------------------------------------------------------------
+// 1/sqrt(x) and 1/x of x > 0 in FP64: the hardware estimate (2^-24) with one cubic step, 1-2 ulp.  WIDE: the
+// step's own terms stay finite for every x, so that infinity gives 0, what is too small for a reciprocal infinity,
+// and a nan nan; without it infinity gives a nan.
+// -------------------------------------------------------------------------------------------
+template <bool WIDE = false> __device__ __forceinline__ double ptg_rsqrt64(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-(WIDE ? fmin(x, DBL_MAX) : x) * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
+}
+template <bool WIDE = false> __device__ __forceinline__ double ptg_rcp64(double x)
+{
+    const double y = __builtin_amdgcn_rcp(x), f = WIDE ? fmin(y, DBL_MAX) : y;
+    const double e = fma(-(WIDE ? fmin(x, DBL_MAX) : x), f, 1.0);
+    return fma(y, fma(e, e, e), y);
 }
 
 // -------------------------------------------------------------------------------------------

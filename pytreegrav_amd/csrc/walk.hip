@@ -418,7 +418,7 @@ __device__ __forceinline__ void flush_parts(const WaveLds<T, QUAD, LF> &L, int c
 // FP32 sums differ at the rounding level.
 #define WALK_NVARIANTS 3
 template <typename T, int TPL, int VAR> struct WalkOcc {
-    static constexpr bool fast = sizeof(T) == 4 && TPL == 1;
+    static constexpr bool fast = TPL == 1;
     static constexpr int waves = !fast ? 1 : VAR == 1 ? 4 : VAR == 2 ? 6 : 5;
     static constexpr int lf = fast && VAR == 2 ? 32 : 64;
     static constexpr int blocks_per_cu = fast && VAR == 2 ? 6 : 5;
@@ -987,7 +987,7 @@ static ptg_status launch_t(const WalkArgs<T> &a, int64_t max_blocks, const WalkW
 template <typename T, int TPL, int FIELDS, bool EXP>
 static ptg_status launch_var(const WalkArgs<T> &a, int variant, int64_t blocks, const WalkWs &ws, hipStream_t s)
 {
-    if constexpr (sizeof(T) == 4 && TPL == 1) {
+    if constexpr (TPL == 1) {
         if (variant == 1) return launch_t<T, TPL, FIELDS, false, EXP, 1>(a, blocks, ws, s);
         if (variant == 2) return launch_t<T, TPL, FIELDS, false, EXP, 2>(a, blocks, ws, s);
     }

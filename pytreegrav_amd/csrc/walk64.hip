@@ -18,8 +18,6 @@
 // ms, tidal tensors with quadrupoles of 6e4 23.3 -> 1.24 ms.  Angle-binned columns of 2e5 particles
 // against their own walk (two waves per SIMD, six selected adds and a division a pair): 4.9 -> 2.15 ms.
 
-#include <cfloat>
-
 #include "walk_shared.hpp"
 
 #define LIST 32           // a list is evaluated in multiples of LIST entries once it holds LIST
@@ -40,21 +38,6 @@ template <int FIELDS, bool QUAD> struct Lds64 {
     double ph[ICAP];
     double bins[FIELDS == BINS ? 6 * 64 : 1];  // [bin][lane]
 };
-
-// 1/sqrt(x) and 1/x of x > 0: the hardware estimate (2^-24) with one cubic step, 1-2 ulp.  WIDE: the step's own
-// terms stay finite for every x, so that infinity gives 0, what is too small for a reciprocal infinity, and a nan nan.
-template <bool WIDE> __device__ __forceinline__ double rsqrt64(double x)
-{
-    const double y = __builtin_amdgcn_rsq(x);
-    const double e = fma(-(WIDE ? fmin(x, DBL_MAX) : x) * y, y, 1.0);
-    return fma(y * e, fma(0.375, e, 0.5), y);
-}
-template <bool WIDE> __device__ __forceinline__ double rcp64(double x)
-{
-    const double y = __builtin_amdgcn_rcp(x), f = WIDE ? fmin(y, DBL_MAX) : y;
-    const double e = fma(-(WIDE ? fmin(x, DBL_MAX) : x), f, 1.0);
-    return fma(y, fma(e, e, e), y);
-}
 
 // A group is walked WIDE where a coordinate of it or of its tree is not at most this large, or a target's softening: no
 // other squared distance can overflow.  Caps in every pair cost 6 to 18 % of the walk (groups of 64 to 256).
@@ -88,7 +71,7 @@ __device__ __forceinline__ void pair_node(Acc<double> &a, const V4<double> &s, c
 {
     const double dx = s.x - tx, dy = s.y - ty, dz = s.z - tz;
     const double r2 = dx * dx + dy * dy + dz * dz;
-    const double rinv = rsqrt64<WIDE>(r2), rinv2 = rinv * rinv;
+    const double rinv = ptg_rsqrt64<WIDE>(r2), rinv2 = rinv * rinv;
     const double mr = s.w * rinv, K = mr * rinv2;
     add_pair<FIELDS>(a, -mr, K, 3.0 * K * rinv2, dx, dy, dz);
     if (QUAD) {
@@ -123,7 +106,7 @@ __device__ __forceinline__ void pair_node(Acc<double> &a, const V4<double> &s, c
 template <int FIELDS, bool WIDE>
 __device__ __forceinline__ void spline64(double r, double rinv, double h, double &phi, double &K, double &Q)
 {
-    const double hinv = rcp64<WIDE>(h), q = r * hinv;
+    const double hinv = ptg_rcp64<WIDE>(h), q = r * hinv;
     const double hinv2 = hinv * hinv, hinv3 = hinv2 * hinv;
     if (q <= 0.5) {
         const double q2 = q * q;
@@ -163,7 +146,7 @@ __device__ __forceinline__ Pair64 part_pair(const V4<double> &s, double hs, doub
 template <int FIELDS, bool SOFT, bool WIDE>
 __device__ __forceinline__ void part_add(Acc<double> &a, const Pair64 &p, double m)
 {
-    const double rinv = p.apart ? rsqrt64<WIDE>(p.r2) : 0.0, rinv2 = rinv * rinv;
+    const double rinv = p.apart ? ptg_rsqrt64<WIDE>(p.r2) : 0.0, rinv2 = rinv * rinv;
     const double mr = m * rinv;
     double phi = -mr, K = mr * rinv2, Q = 3.0 * K * rinv2;
     if (SOFT && p.soft) {
@@ -264,7 +247,7 @@ struct Sky {
     template <bool WIDE> __device__ __forceinline__ void node(const V4<double> &s, double tx, double ty, double tz)
     {
         const double dx = s.x - tx, dy = s.y - ty, dz = s.z - tz;
-        add(dx, dy, dz, s.w * rcp64<WIDE>(dx * dx + dy * dy + dz * dz));
+        add(dx, dy, dz, s.w * ptg_rcp64<WIDE>(dx * dx + dy * dy + dz * dz));
     }
     // a particle: a point mass outside its radius h, a blend of the isotropic and directed limits inside
     template <bool WIDE> __device__ __forceinline__ void part(const V4<double> &s, double h, double tx, double ty, double tz)
@@ -272,13 +255,13 @@ struct Sky {
         const double dx = s.x - tx, dy = s.y - ty, dz = s.z - tz;
         const double r2 = dx * dx + dy * dy + dz * dz, hh = h * h;
         const bool out = r2 > hh;
-        double v = s.w * rcp64<WIDE>(out ? r2 : 1.0);
+        double v = s.w * ptg_rcp64<WIDE>(out ? r2 : 1.0);
         if (ptg_ballot(!out)) {
             if (!out) {
                 v = 0.0;
                 if (h > 0) {
-                    const double hinv = rcp64<WIDE>(h), col0 = s.w * (3.0 / (4.0 * 3.14159265358979323846) * SKY_BIN) * hinv * hinv;
-                    const double fac = r2 == 0 ? 0.0 : r2 * rsqrt64<WIDE>(r2) * hinv;
+                    const double hinv = ptg_rcp64<WIDE>(h), col0 = s.w * (3.0 / (4.0 * 3.14159265358979323846) * SKY_BIN) * hinv * hinv;
+                    const double fac = r2 == 0 ? 0.0 : r2 * ptg_rsqrt64<WIDE>(r2) * hinv;
                     iso += (1.0 - fac) * col0;
                     v = 2.0 * col0 * fac;
                 }
