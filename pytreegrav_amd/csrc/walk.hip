@@ -749,9 +749,7 @@ void k_walk(const WalkArgs<T> A, const WalkHot H, const WalkPool pool)
                     continue;
                 }
                 if (lane == 0) agent_store(&B.tasks[troot].root, 1);
-                walk_add_up<FIELDS, T>(A.ctl, B, parent, grp, A.gs, A.perm, A.G, A.out, lane);
-                closed++;
-                continue;
+                nn = np = 0;  // its row and counts are not used any more
             }
             if (A.counters) {
                 if (EXP) {

@@ -605,9 +605,7 @@ void k_walk64(const Walk64Args A, const WalkHot H, const WalkPool pool)
                     continue;
                 }
                 if (lane == 0) agent_store(&B.tasks[troot].root, 1);
-                walk_add_up<FIELDS, double>(A.ctl, B, parent, grp, A.gs, A.perm, A.G, A.out, lane);
-                closed++;
-                continue;
+                nn = np = 0;  // its row and counts are not used any more
             }
             if (A.counters) {
                 const int64_t n[3] = {(int64_t)n_list * mt, visits, (int64_t)n_part * mt};
