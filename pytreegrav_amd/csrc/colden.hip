@@ -39,14 +39,20 @@ __device__ __forceinline__ void cd_count(unsigned long long *ctr, int k, int64_t
     if (ptg_lane() == 0 && v) atomicAdd(ctr + k, (unsigned long long)v);
 }
 
-// squared distance across a ray: the product is rounded by itself, so that an element exactly along the ray (r2 = z^2,
-// as on a lattice) is at 0.  As a fused multiply-add its sign was z^2's rounding error, and half of such elements,
-// particles and whole nodes, were skipped.
-__device__ __forceinline__ double across2(double r2, double z)
-{
+// An element at d from a target, against a ray u: its squared distance, its distance along the ray and its squared
+// distance across it, each product and sum rounded as in the reference's arithmetic.  An element exactly along the
+// ray (as on a lattice) is at b2 = 0; with fused multiply-adds its sign was a product's rounding error, and half of
+// such elements, particles and whole nodes, were skipped.
+struct Across {
+    double r2, z, b2;
+    __device__ __forceinline__ Across(double dx, double dy, double dz, double ux, double uy, double uz)
+    {
 #pragma clang fp contract(off)
-    return r2 - z * z;
-}
+        r2 = dx * dx + dy * dy + dz * dz;
+        z = ux * dx + uy * dy + uz * dz;
+        b2 = r2 - z * z;
+    }
+};
 
 // column along ray i from target j; visits counts the elements the walk touched
 __device__ __forceinline__ double ray_column(const ptg_tree_arrays &t, int64_t n, int64_t ne, const double *tp,
@@ -67,10 +73,9 @@ __device__ __forceinline__ double ray_column(const ptg_tree_arrays &t, int64_t n
         }
         const double dx = t.coordinates[3 * no] - px, dy = t.coordinates[3 * no + 1] - py;
         const double dz = t.coordinates[3 * no + 2] - pz;
-        const double r2 = dx * dx + dy * dy + dz * dz;
-        const double r = sqrt(r2);
-        const double z = rx * dx + ry * dy + rz * dz;
-        if (across2(r2, z) < 0) {  // rounding below zero: skipped, as ColumnDensityWalk_singleray does
+        const Across e(dx, dy, dz, rx, ry, rz);
+        const double r = sqrt(e.r2), z = e.z, b2 = e.b2;
+        if (b2 < 0) {  // rounding below zero: skipped, as ColumnDensityWalk_singleray does
             no = t.next_branch[no];
             continue;
         }
@@ -79,7 +84,7 @@ __device__ __forceinline__ double ray_column(const ptg_tree_arrays &t, int64_t n
             if (h_no > 0) {  // a zero radius has no cross-section
                 const double hinv = 1.0 / h_no;
                 const double fac = fac_density * t.masses[no] * hinv * hinv;
-                const double r_proj = sqrt(across2(r2, z));
+                const double r_proj = sqrt(b2);
                 const double q = r_proj * hinv;
                 if (r_proj < h_no) {
                     if (r > h_no) {  // target outside the sphere: the whole chord if it lies ahead
@@ -93,7 +98,7 @@ __device__ __forceinline__ double ray_column(const ptg_tree_arrays &t, int64_t n
         } else {
             const double reach = h_no + t.sizes[no] * 0.8660254037844386 + t.deltas[no];
             bool open = r < reach;  // the node holds the ray's origin
-            if (!open && z > 0) open = (across2(r2, z)) < reach * reach;
+            if (!open && z > 0) open = b2 < reach * reach;
             no = open ? t.first_subnode[no] : t.next_branch[no];
         }
     }
@@ -189,16 +194,15 @@ __global__ __launch_bounds__(64 * CR_WAVES) void k_column_rays_wave(const D4 *xy
         if (m & me) {
             visits++;
             const double dx = X.x - px, dy = X.y - py, dz = X.z - pz;
-            const double r2 = dx * dx + dy * dy + dz * dz;
-            const double r = sqrt(r2);
-            const double z = rx * dx + ry * dy + rz * dz;
-            if (!(across2(r2, z) < 0)) {  // rounding below zero: skipped, as ColumnDensityWalk_singleray does
+            const Across a(dx, dy, dz, rx, ry, rz);
+            const double r = sqrt(a.r2), z = a.z, b2 = a.b2;
+            if (!(b2 < 0)) {  // rounding below zero: skipped, as ColumnDensityWalk_singleray does
                 const double h_no = X2.x;
                 if (K.y == 0) {
                     if (h_no > 0) {  // a zero radius has no cross-section
                         const double hinv = 1.0 / h_no;
                         const double fac = fac_density * X.w * hinv * hinv;
-                        const double r_proj = sqrt(across2(r2, z));
+                        const double r_proj = sqrt(b2);
                         const double q = r_proj * hinv;
                         if (r_proj < h_no) {
                             if (r > h_no) {
@@ -211,7 +215,7 @@ __global__ __launch_bounds__(64 * CR_WAVES) void k_column_rays_wave(const D4 *xy
                 } else {
                     const double reach = h_no + X2.y * 0.8660254037844386 + X2.z;
                     open = r < reach;
-                    if (!open && z > 0) open = (across2(r2, z)) < reach * reach;
+                    if (!open && z > 0) open = b2 < reach * reach;
                 }
             }
         }
@@ -268,11 +272,10 @@ __device__ __forceinline__ void cn_flush(const CnLds &S, int c, double px, doubl
         const D4 P = S.part[k];
         const double h = S.h[k];
         const double dx = P.x - px, dy = P.y - py, dz = P.z - pz;
-        const double r2 = dx * dx + dy * dy + dz * dz;
-        const double z = rx * dx + ry * dy + rz * dz;
-        const double b2 = across2(r2, z), hh = h * h;
+        const Across e(dx, dy, dz, rx, ry, rz);
+        const double b2 = e.b2, z = e.z, hh = h * h;
         // b2 < 0 by rounding: skipped, as ColumnDensityWalk_singleray does
-        const bool inside = !(r2 > hh);
+        const bool inside = !(e.r2 > hh);
         if (b2 >= 0 && b2 < hh && (inside || z > 0)) {
             const double hinv = S.hinv[k];
             const double half = cn_sqrt(1.0 - b2 * (hinv * hinv));
