@@ -1,12 +1,14 @@
 // Column density through the octree (treewalk.py:821-1276): particles are uniform spheres of radius
-// equal to their softening.  Both walks follow the tree's own depth-first links (FirstSubnode /
-// NextBranch of the reference layout), so they need no stack and accumulate every sum in the
-// reference's order.
+// equal to their softening.
 //
-// Ray-traced (ptg_column_rays): one thread per (target, ray), ray-major so that a wavefront walks 64
-// Morton-adjacent targets along one direction and its lanes open nearly the same nodes.  The walk is
-// exact: a node is opened whenever its bounding sphere, inflated by the largest particle radius in
-// it, could meet the ray; only particles contribute, by the closed-form chord integral.
+// Ray-traced: exact, a node is opened whenever its bounding sphere, inflated by the largest particle radius in
+// it, could meet the ray; only particles contribute, by the closed-form chord integral.  Three walks:
+//   k_column_bundles (ptg_column_bundles): shared unit rays, one wavefront for 64 targets that neighbour each
+//     other across the ray, 64 elements a step over a stack in LDS; sums in the bundle's order.
+//   k_column_rays_wave (ptg_column_rays with the FP64 pack): rays of each target's own, or of any length, one
+//     wavefront for 64 targets along one ray index, one element a step; sums in the reference's order.
+//   k_column_rays (ptg_column_rays without): one thread per (target, ray) along the tree's depth-first links,
+//     with no stack, for trees deeper than the stacks of the others; sums in the reference's order.
 //
 // Angular-binned (ptg_column_binned), the reference's grouped estimator: a node whose distance to
 // the box of group_size consecutive targets passes the opening test puts its mass in one of six

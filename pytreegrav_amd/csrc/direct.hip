@@ -9,10 +9,10 @@
 // distance is not an ordinary number) are its pairs evaluated by the reference's branches.  Partial sums
 // are added in a fixed order, so results do not depend on scheduling.
 //
-// Bound: VALU (about 18 issue slots a pair in FP32, 38 in FP64).  One Accel call against one lane per
-// target over scalar-loaded sources with IEEE square roots and divisions: FP32 12007 particles 266 ->
-// 76 us, 1e5 11.0 -> 4.4 ms (2.3e12 pairs/s); FP64 4000 particles 124 -> 26 us (host bound), 1e5 17.2 ->
-// 10.0 ms.  Against an extended-precision sum its errors are that kernel's or
+// Bound: VALU (FP32 accelerations: 13 arithmetic instructions a pair of about 18 issue slots; FP64 38 slots).
+// One Accel call against one lane per target over scalar-loaded sources with IEEE square roots and divisions:
+// FP32 12007 particles 312 -> 85 us (the kernel 73), 1e5 11.0 -> 4.4 ms (2.3e12 pairs/s); FP64 4000 particles
+// 124 -> 26 us (host bound), 1e5 17.2 -> 10.0 ms.  Against an extended-precision sum its errors are that kernel's or
 // smaller (FP64 1.5e-16 to 5e-13, FP32 6e-8 to 1e-6; FP32 tidal tensors within the summation noise of it).
 #include <algorithm>
 
@@ -259,9 +259,11 @@ static ptg_status launch_p(int fields, const double *pt, const double *ht, int64
     return PTG_OK;
 }
 
-// Targets per block.  16: many blocks and short sums (12007 targets: 78 us in FP32, 111 with 64).  4 where
-// 16 would leave most CUs idle.  64 where there are blocks enough and 16 targets would read the sources
-// four times as often (equal times at 1e5 targets).
+// Targets per block.  16: many blocks and short sums (12007 targets: 78 us in FP32, 111 with 64).  4 where 16
+// makes less than a block per 4 CUs: the kernel takes, with 4 and with 16, FP64 5.2 and 5.5 us for 256 particles,
+// 6.6 and 9.3 for 1000, 13.7 and 14.1 for 2000, 35 and 25 for 4000 (FP32 4.5 and 4.7, 5.4 and 7.0, 9.6 and 9.6,
+// 20.7 and 16.0); below 4000 the call's 25 us of host and launch hide it.  64 where there are blocks enough and 16
+// targets would read the sources four times as often (equal times at 1e5 targets).
 template <typename T, bool SELF>
 static ptg_status launch_direct(int fields, const double *pt, const double *ht, int64_t nt, const double *ps,
                                 const double *ms, const double *hs, int64_t ns, double G, double *out, hipStream_t s)

@@ -14,9 +14,9 @@
 //
 // Bound: instruction issue, about 60 % of it the traversal (250 instructions per 64-element step).
 // Whole calls, against one wave per group evaluating every entry for 8 of its 64 lanes with IEEE
-// square roots and divisions: 1e6-particle Plummer sphere 333 -> 4.4 ms, uniform cube of 1e5 6.0 -> 0.79
+// square roots and divisions: 1e6-particle Plummer sphere 333 -> 4.3 ms, uniform cube of 1e5 6.0 -> 0.73
 // ms, tidal tensors with quadrupoles of 6e4 23.3 -> 1.24 ms.  Angle-binned columns of 2e5 particles
-// against their own walk (two waves per SIMD, six selected adds and a division a pair): 4.9 -> 2.15 ms.
+// against their own walk (two waves per SIMD, six selected adds and a division a pair): 4.9 -> 2.05 ms.
 
 #include "walk_shared.hpp"
 

@@ -25,9 +25,10 @@ FP32_DEFAULT_GROUP = 64
 
 
 # Accel / Potential with method="adaptive" in float32 walk the tree above this many particles and sum
-# directly below it: on one MI355X a whole float32 Accel call from numpy inputs (tree build + walk vs
-# the direct sum, Plummer spheres, h = 0.01) takes 1.01 vs 0.62 ms at N = 16000 and 1.10 vs 1.48 ms
-# at N = 32000 (0.82 vs 0.42 and 0.84 vs 1.25 ms from device tensors)
+# directly below it.  The line was drawn for a direct sum of three times the time; on one MI355X a whole float32
+# Accel call (tree build + walk vs the direct sum, Plummer spheres, h = 0.01) now takes 0.90 vs 0.29 ms at
+# N = 16000, 0.97 vs 0.71 at 32000 and 1.00 vs 0.99 at 40000 from numpy inputs (0.69 vs 0.15, 0.71 vs 0.49 and
+# 0.71 vs 0.75 from device tensors).  It stays, since it decides which of two answers a call gives.
 FP32_TREE_MIN_N = 24000
 
 
