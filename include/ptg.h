@@ -309,7 +309,7 @@ ptg_status ptg_walk(const ptg_walk_tree *wt, const ptg_forest *forest, const dou
                     int exact, double *out, int64_t *counters, void *ws, size_t ws_bytes, void *stream);
 /* Reads the overflow flag of the last walk on this workspace (synchronises the stream):
  * PTG_ERR_OVERFLOW if a traversal stack exceeded its spill capacity or a share of a cut traversal never
- * finished (its waves gave up waiting after about a minute), PTG_ERR_ARG if a supplied
+ * finished (its waves gave up waiting after some minutes), PTG_ERR_ARG if a supplied
  * group held more than group_size targets or a subtree walk's start slot was out of range. */
 ptg_status ptg_walk_check(void *ws, void *stream);
 

@@ -116,7 +116,7 @@ template <int FIELDS> __device__ __forceinline__ void store_sum(double *o, int c
 // level of sums cost 30.  Its waves end when no task is open; which wave walks which task is in
 // walk_tasks.hpp.  What one wave writes and another reads within it (records, stacks, rows) goes
 // through agent-scope accesses, ordered by the writer's wait before it publishes or counts down.
-#define WALK_LOOKS (1 << 26)  // a wave gives up after a minute without a task and reports it
+#define WALK_LOOKS (1 << 26)  // a wave gives up after some minutes without a task and reports it
 
 // The workspace: the control block, the flags of the task slots and the bits of the groups put back (these
 // cleared before each walk), the spill stacks of the waves, and WALK_POOL bytes for what deferral needs.  The
